@@ -458,6 +458,27 @@ size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K,
                                       int V);
 
 /*
+ * The same for num_seqs independent sequences packed along T (q .. dout
+ * [1, T, ..]): sequence s is the rows cu_seqlens[s] .. cu_seqlens[s + 1] - 1
+ * (cu_seqlens [num_seqs + 1] int32 on the device, non-decreasing; clamped to
+ * [0, T] whatever it holds), with its own h0, dht and dh0 row ([num_seqs, Hv,
+ * K, V]). An empty sequence's dh0 is its dht. Rows of no sequence get zero
+ * gradients. One call's launches for all sequences and no host read of
+ * cu_seqlens. Workspace: pbgdn_chunk_bwd_packed_workspace_size bytes.
+ */
+int pbgdn_chunk_bwd_packed(const void *q, const void *k, const void *v,
+                           int in_dtype, const float *g, const void *beta,
+                           int beta_dtype, const float *h0,
+                           const int32_t *cu_seqlens, int num_seqs,
+                           const void *dout, int do_dtype, const float *dht,
+                           void *dq, void *dk, void *dv, float *dg,
+                           void *dbeta, float *dh0, void *workspace,
+                           size_t workspace_bytes, int T, int Hk, int Hv,
+                           int K, int V, float scale, void *stream);
+size_t pbgdn_chunk_bwd_packed_workspace_size(int T, int num_seqs, int Hk,
+                                             int Hv, int K, int V);
+
+/*
  * Fused decode step of a GatedDeltaNetLayer: one token per sequence, from the
  * input projection to the layer output, in one launch (GatedDeltaNetLayer.forward
  * at T = 1, gated_deltanet.py:415-441: short_convolution :314-338,

@@ -58,10 +58,13 @@ struct BwdParams {
   void *dbeta;
   float *dh0;
   float *ws_T, *ws_c, *ws_beta, *ws_dU0, *ws_J, *ws_S, *ws_dS, *ws_dq, *ws_dk;
+  const int32_t *cu_seqlens;  // [num_seqs + 1] bounds of packed sequences (B = 1), or NULL: B rows of T tokens
+  int num_seqs;               // sequences: B without cu_seqlens
+  int records;                // chunk records (times Hv: records of the workspace)
   int in_dtype, beta_dtype;
-  int B, T, Hk, Hv, K, V, n;
+  int B, T, Hk, Hv, K, V, n;  // n: chunks of a batch row
   float scale;
-  int xcds;  // the device's XCDs (device.hpp)
+  int cus, xcds;  // the device's compute units and XCDs (device.hpp)
 };
 
 // fp32 MFMA: acc (16x16) += A (16x4) B (4x16). Lane l, c = l & 15, g = l >> 4:
@@ -357,9 +360,60 @@ __device__ __forceinline__ void put_pair1(u16 *m, int lo_off, int e, float x) {
   m[lo_off + e] = bf16_bits(x - __uint_as_float(static_cast<uint32_t>(hi) << 16));
 }
 
-// Workspace records of (batch b, value head h, chunk i).
-__device__ __forceinline__ long rec(const BwdParams &p, int b, int h, int i) {
-  return (static_cast<long>(b) * p.Hv + h) * p.n + i;
+// One sequence: its first token row of the [B T] rows, its length, its chunks
+// and its first chunk record. A batch row b holds records b n ..; a packed
+// sequence s (first row bos) records floor(bos / 64) + s .., which is
+// increasing in s and leaves room for every sequence's chunks, so a chunk's
+// record is known without a pass over the lengths. Whatever cu_seqlens holds,
+// the bounds are clamped to 0 <= bos <= bos + len <= T.
+struct BwdSeq {
+  long bos, base;
+  int len, n;
+};
+__device__ __forceinline__ BwdSeq seq_of(const BwdParams &p, int s) {
+  BwdSeq q;
+  if (p.cu_seqlens) {
+    const int lo = __builtin_amdgcn_readfirstlane(min(max(p.cu_seqlens[s], 0), p.T));
+    const int hi = __builtin_amdgcn_readfirstlane(min(max(p.cu_seqlens[s + 1], lo), p.T));
+    q.bos = lo;
+    q.len = hi - lo;
+    q.n = (q.len + BC - 1) / BC;
+    q.base = lo / BC + s;
+  } else {
+    q.bos = static_cast<long>(s) * p.T;
+    q.len = p.T;
+    q.n = p.n;
+    q.base = static_cast<long>(s) * p.n;
+  }
+  return q;
+}
+
+// The sequence and chunk of block (x, z) of a per-chunk grid: chunk x of batch
+// row z, or packed the chunk of record x (false where it holds none): the last sequence whose first record is at most x, counted 64
+// sequences at a time across the wave (every wave gets the same answer).
+__device__ __forceinline__ bool chunk_of(const BwdParams &p, int x, int z, BwdSeq &q, int &i) {
+  int s = z;
+  if (p.cu_seqlens) {
+    const int lane = threadIdx.x & 63;
+    int count = 0;
+    for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
+      const int m = s0 + lane;
+      const int lo = min(max(p.cu_seqlens[min(m, p.num_seqs - 1)], 0), p.T);
+      const int add = __popcll(__ballot(m < p.num_seqs && lo / BC + m <= x));
+      count += add;
+      if (add < 64) break;
+    }
+    s = __builtin_amdgcn_readfirstlane(count) - 1;
+    if (s < 0) return false;
+  }
+  q = seq_of(p, s);
+  i = p.cu_seqlens ? x - static_cast<int>(q.base) : x;
+  return i < q.n;
+}
+
+// Workspace record of chunk i of a sequence, value head h.
+__device__ __forceinline__ long rec(const BwdParams &p, const BwdSeq &q, int h, int i) {
+  return static_cast<long>(h) * p.records + q.base + i;
 }
 
 // A 64 x 64 float32 record (T) into LDS rows of LC floats.
@@ -394,10 +448,10 @@ __device__ __forceinline__ void load_t_pair(u16 *tp, int ld, const float *src) {
 // c (in-chunk cumulative log decay), e^c, e^(c_last - c) and beta of one chunk,
 // from the workspace record (c, and beta as float: 0 past T). Every lane
 // loads; the first wave stores.
-__device__ __forceinline__ void load_decays(const BwdParams &p, int b, int h, int i, float *sc, float *sgam, float *se,
+__device__ __forceinline__ void load_decays(const BwdParams &p, const BwdSeq &q, int h, int i, float *sc, float *sgam, float *se,
                                             float *sbeta) {
   const int tid = threadIdx.x;
-  const long r = rec(p, b, h, i) * BC;
+  const long r = rec(p, q, h, i) * BC;
   const float c = p.ws_c[r + (tid & (BC - 1))], last = p.ws_c[r + BC - 1], bt = p.ws_beta[r + (tid & (BC - 1))];
   if (tid < BC) {
     sc[tid] = c;
@@ -411,33 +465,37 @@ __device__ __forceinline__ void load_decays(const BwdParams &p, int b, int h, in
 // Per (chunk, value head): T, dU0 = M^T dO, J = scale (Gamma Q)^T dO, c and
 // beta as float.
 // ---------------------------------------------------------------------------
-// Rows t0 .. t0+63 of a [B,T,H,W] tensor of TIn (head hd, columns 0 ..
+// Rows t0 .. t0+63 of a sequence of a [B,T,H,W] tensor of TIn (head hd, columns 0 ..
 // COLS-1) as 16-byte pieces in registers, then into LDS as they are (rows of
 // ld elements, ld a multiple of 16 bytes), zero past T. Every lane issues the
 // same loads (rows clamped into the sequence, zeroed after), so a kernel can
 // issue several tensors' rows before its first wait, and that wait is one
 // round trip rather than one per tensor.
-template <typename TIn, int COLS>
+template <typename TIn, int COLS, int NT = BNT>
 struct RawRows {
-  static constexpr int EPP = 16 / sizeof(TIn), PPR = COLS / EPP, TOTAL = BC * PPR, PER = TOTAL / BNT;
-  static_assert(TOTAL % BNT == 0, "whole pieces per thread");
+  static constexpr int EPP = 16 / sizeof(TIn), PPR = COLS / EPP, TOTAL = BC * PPR, PER = TOTAL / NT;
+  static_assert(TOTAL % NT == 0, "whole pieces per thread");
   uint4 raw[PER];
 
-  __device__ __forceinline__ void load(const void *src, const BwdParams &p, int b, int t0, int heads, int hd,
+  __device__ __forceinline__ void load(const void *src, const BwdSeq &q, int t0, int heads, int hd, int width) {
+    load(threadIdx.x, src, q, t0, heads, hd, width);
+  }
+  __device__ __forceinline__ void load(int tid, const void *src, const BwdSeq &q, int t0, int heads, int hd,
                                        int width) {
     const unsigned char *base = static_cast<const unsigned char *>(src);
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-      const int e = threadIdx.x + BNT * m, row = e / PPR, part = e % PPR, t = t0 + row, tc = t < p.T ? t : p.T - 1;
-      const long off = ((static_cast<long>(b) * p.T + tc) * heads + hd) * width * static_cast<long>(sizeof(TIn));
+      const int e = tid + NT * m, row = e / PPR, part = e % PPR, t = t0 + row, tc = t < q.len ? t : q.len - 1;
+      const long off = ((q.bos + tc) * heads + hd) * width * static_cast<long>(sizeof(TIn));
       const uint4 x = *reinterpret_cast<const uint4 *>(base + off + part * 16);
-      raw[m] = t < p.T ? x : uint4{0u, 0u, 0u, 0u};
+      raw[m] = t < q.len ? x : uint4{0u, 0u, 0u, 0u};
     }
   }
-  __device__ __forceinline__ void put(TIn *dst, int ld) const {
+  __device__ __forceinline__ void put(TIn *dst, int ld) const { put(threadIdx.x, dst, ld); }
+  __device__ __forceinline__ void put(int tid, TIn *dst, int ld) const {
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-      const int e = threadIdx.x + BNT * m, row = e / PPR, part = e % PPR;
+      const int e = tid + NT * m, row = e / PPR, part = e % PPR;
       *reinterpret_cast<uint4 *>(&dst[row * ld + part * EPP]) = raw[m];
     }
   }
@@ -450,6 +508,30 @@ template <int K, int V, typename TIn>
 constexpr size_t local_lds() {
   return sizeof(TIn) * BC * (2 * (K + 16 / sizeof(TIn)) + V + 16 / sizeof(TIn)) +
          sizeof(float) * (BC * LC + 3 * BC + 3 * 256);
+}
+
+// Packed calls: the gradients of token rows that belong to no sequence (before
+// the first and after the last) are zeros; the block of chunk record x takes
+// rows 64 x .. 64 x + 63 (there are at least T / 64 + 1 records).
+template <typename TIn>
+__device__ __forceinline__ void zero_uncovered(const BwdParams &p, int x, int h) {
+  const int lo = min(max(p.cu_seqlens[0], 0), p.T), hi = max(min(p.cu_seqlens[p.num_seqs], p.T), lo);
+  const int group = p.Hv / p.Hk, hk = h / group;
+  for (int t = x * BC; t < min((x + 1) * BC, p.T); ++t) {
+    if (t >= lo && t < hi) continue;
+    const long row = static_cast<long>(t) * p.Hv + h;
+    for (int e = threadIdx.x; e < p.V; e += BNT) store_el<TIn>(p.dv, row * p.V + e, 0.f);
+    if (h % group == 0) {
+      for (int e = threadIdx.x; e < p.K; e += BNT) {
+        store_el<TIn>(p.dq, (static_cast<long>(t) * p.Hk + hk) * p.K + e, 0.f);
+        store_el<TIn>(p.dk, (static_cast<long>(t) * p.Hk + hk) * p.K + e, 0.f);
+      }
+    }
+    if (threadIdx.x == 0) {
+      p.dg[row] = 0.f;
+      store_elem(p.dbeta, row, p.beta_dtype, 0.f);
+    }
+  }
 }
 
 template <int K, int V, typename TIn>
@@ -466,23 +548,27 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   constexpr bool BF = std::is_same<TIn, u16>::value;
   constexpr int LM = LC;
   u16 *mh = reinterpret_cast<u16 *>(sa);
-  const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int h = blockIdx.y;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
+  if (p.cu_seqlens) zero_uncovered<TIn>(p, blockIdx.x, h);
+  BwdSeq seq;
+  int i;
+  if (!chunk_of(p, blockIdx.x, blockIdx.z, seq, i)) return;
   const int t0 = i * BC;
   {
     RawRows<TIn, K> rq, rk;
     RawRows<TIn, V> rd;
-    rq.load(p.q, p, b, t0, p.Hk, hk, K);
-    rk.load(p.k, p, b, t0, p.Hk, hk, K);
-    rd.load(p.dout, p, b, t0, p.Hv, h, V);
+    rq.load(p.q, seq, t0, p.Hk, hk, K);
+    rk.load(p.k, seq, t0, p.Hk, hk, K);
+    rd.load(p.dout, seq, t0, p.Hv, h, V);
     rq.put(sq, LK);
     rk.put(sk, LK);
     rd.put(sdo, LV);
   }
   if (wave == 0) {  // inclusive cumulative sum of g over the chunk (zero past T)
     const int t = t0 + lane;
-    float x = t < p.T ? p.g[(static_cast<long>(b) * p.T + t) * p.Hv + h] : 0.f;
+    float x = t < seq.len ? p.g[(seq.bos + t) * p.Hv + h] : 0.f;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const float y = __shfl_up(x, off, 64);
@@ -490,10 +576,10 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
     }
     sc[lane] = x;
     sgam[lane] = expf(x);
-    const float bt = t < p.T ? load_elem(p.beta, (static_cast<long>(b) * p.T + t) * p.Hv + h, p.beta_dtype) : 0.f;
+    const float bt = t < seq.len ? load_elem(p.beta, (seq.bos + t) * p.Hv + h, p.beta_dtype) : 0.f;
     sbeta[lane] = bt;
-    p.ws_c[rec(p, b, h, i) * BC + lane] = x;
-    p.ws_beta[rec(p, b, h, i) * BC + lane] = bt;
+    p.ws_c[rec(p, seq, h, i) * BC + lane] = x;
+    p.ws_beta[rec(p, seq, h, i) * BC + lane] = bt;
   }
   __syncthreads();
   auto krow = [&](int kk, int j, int tc) { return ld4e(sk, (16 * tc + j) * LK + kk); };
@@ -551,7 +637,7 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
     }
     __syncthreads();
   }
-  float *wt = p.ws_T + rec(p, b, h, i) * BC * BC;
+  float *wt = p.ws_T + rec(p, seq, h, i) * BC * BC;
   for (int e = tid; e < BC * BC; e += BNT) wt[e] = sa[(e / BC) * LC + e % BC];
   __syncthreads();  // T is out: M = scale (Q K^T) o D takes its place
   for (int tc = 0; tc < 4; ++tc) {
@@ -577,7 +663,7 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   }
   __syncthreads();
   // dU0 = M^T dO: tiles (row tile, 16-column tile)
-  float *wu = p.ws_dU0 + rec(p, b, h, i) * BC * V;
+  float *wu = p.ws_dU0 + rec(p, seq, h, i) * BC * V;
   if constexpr (BF) {  // M^T fragments and dO's columns by transposing reads
     for (int tile = wave; tile < 4 * (V / 16); tile += 4) {
       const int tr = tile & 3, tv = tile >> 2;
@@ -604,7 +690,7 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
     for (int r = 0; r < 4; ++r) wu[(16 * tr + 4 * g4 + r) * V + 16 * tv + c] = acc[r];
   }
   // J = scale (Gamma Q)^T dO: K x V
-  float *wj = p.ws_J + rec(p, b, h, i) * static_cast<long>(K) * V;
+  float *wj = p.ws_J + rec(p, seq, h, i) * static_cast<long>(K) * V;
   if constexpr (BF) {
     // per column tile of this wave: (Gamma dO)'s columns as bf16 pairs once,
     // then every key tile's Q^T fragments (transposing reads of the q rows)
@@ -673,19 +759,19 @@ struct ScanStage {
   float4_t dur;
   float jr[K / 64][4];
 
-  __device__ __forceinline__ void load(const BwdParams &p, int b, int h, int hk, int i, int v0) {
+  __device__ __forceinline__ void load(const BwdParams &p, const BwdSeq &seq, int h, int hk, int i, int v0) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g4 = lane >> 4;
     const int t0 = i * BC;
-    const long r = rec(p, b, h, i);
+    const long r = rec(p, seq, h, i);
     const unsigned char *kb = static_cast<const unsigned char *>(p.k);
 #pragma unroll
     for (int m = 0; m < KP; ++m) {
       // rows clamped into the sequence and zeroed after: every path issues
       // the same loads, so the waits for them can be partial
-      const int e = tid + BNT * m, row = e / ROW16, part = e % ROW16, t = t0 + row, tc = t < p.T ? t : p.T - 1;
-      const long off = ((static_cast<long>(b) * p.T + tc) * p.Hk + hk) * K * static_cast<long>(sizeof(TIn)) + part * 16;
+      const int e = tid + BNT * m, row = e / ROW16, part = e % ROW16, t = t0 + row, tc = t < seq.len ? t : seq.len - 1;
+      const long off = ((seq.bos + tc) * p.Hk + hk) * K * static_cast<long>(sizeof(TIn)) + part * 16;
       const uint4 kx = *reinterpret_cast<const uint4 *>(kb + off);
-      kr[m] = t < p.T ? kx : uint4{0u, 0u, 0u, 0u};
+      kr[m] = t < seq.len ? kx : uint4{0u, 0u, 0u, 0u};
     }
     const float4_t *wt = reinterpret_cast<const float4_t *>(p.ws_T + r * BC * BC);
 #pragma unroll
@@ -697,9 +783,8 @@ struct ScanStage {
     if constexpr (!ADJ) {
       const int row = tid / TILE16, part = tid % TILE16, t = t0 + row;
       const unsigned char *vb = static_cast<const unsigned char *>(p.v);
-      const long off = (((static_cast<long>(b) * p.T + t) * p.Hv + h) * p.V + v0) * static_cast<long>(sizeof(TIn)) +
-                       part * 16;
-      xr = tid < BC * TILE16 && t < p.T ? *reinterpret_cast<const uint4 *>(vb + off) : uint4{0u, 0u, 0u, 0u};
+      const long off = (((seq.bos + t) * p.Hv + h) * p.V + v0) * static_cast<long>(sizeof(TIn)) + part * 16;
+      xr = tid < BC * TILE16 && t < seq.len ? *reinterpret_cast<const uint4 *>(vb + off) : uint4{0u, 0u, 0u, 0u};
     } else {
       dur = *reinterpret_cast<const float4_t *>(p.ws_dU0 + r * BC * p.V + (tid >> 2) * p.V + v0 + 4 * (tid & 3));
       const float *wj = p.ws_J + r * K * p.V;
@@ -837,8 +922,23 @@ __device__ __forceinline__ float4_t k_cols(const void *sk, int t, int col) {
   }
 }
 
+// Key tile kt of the value columns v0 .. of a state record, from the
+// accumulator layout. bf16 inputs: in that layout as it is, tile (v0 / 16, kt)
+// 64 lanes x 16 bytes (what the gradient kernel's waves hold); else [K][V].
 template <int K, typename TIn>
-__device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int b, int h, int v0) {
+__device__ __forceinline__ void put_state_tile(float *ws, int V, int v0, int kt, float4_t x) {
+  const int lane = threadIdx.x & 63;
+  if constexpr (std::is_same<TIn, u16>::value) {
+    reinterpret_cast<float4_t *>(ws)[((v0 >> 4) * (K / 16) + kt) * 64 + lane] = x;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ws[static_cast<long>(16 * kt + 4 * (lane >> 4) + r) * V + v0 + (lane & 15)] = x[r];
+  }
+}
+
+template <int K, typename TIn>
+__device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
+  const BwdSeq seq = seq_of(p, n);
   using L = ScanLds<K, TIn>;
   constexpr int PER = K / 64, LB = L::LB;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
@@ -849,7 +949,7 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int b
   u16 *xT = reinterpret_cast<u16 *>(base + L::OFF_A), *uT = xT + 2 * 16 * LB;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
-  const long kv = (static_cast<long>(b) * p.Hv + h) * K * p.V;
+  const long kv = (static_cast<long>(n) * p.Hv + h) * K * p.V;
   float4_t s[PER];
 #pragma unroll
   for (int m = 0; m < PER; ++m) {
@@ -860,20 +960,16 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int b
     }
   }
   ScanStage<K, TIn, false> stage;
-  if (p.n > 0) stage.load(p, b, h, hk, 0, v0);
-  for (int i = 0; i < p.n; ++i) {
-    float *ws = p.ws_S + rec(p, b, h, i) * K * p.V;
+  if (seq.n > 0) stage.load(p, seq, h, hk, 0, v0);
+  for (int i = 0; i < seq.n; ++i) {
+    float *ws = p.ws_S + rec(p, seq, h, i) * K * p.V;
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kk = 16 * (wave + 4 * m) + 4 * g4 + r;
-        ws[static_cast<long>(kk) * p.V + v0 + c] = s[m][r];
-      }
+      put_state_tile<K, TIn>(ws, p.V, v0, wave + 4 * m, s[m]);
       put_state_rows<K, TIn>(ss, 16 * (wave + 4 * m) + 4 * g4, c, s[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sx);
-    if (i + 1 < p.n) stage.load(p, b, h, hk, i + 1, v0);
+    if (i + 1 < seq.n) stage.load(p, seq, h, hk, i + 1, v0);
     __syncthreads();
     // X = V - Gamma K S (rows 16w ..)
     const float4_t ks = k_times_state<K, TIn>(sk, 16 * wave, ss);
@@ -934,7 +1030,8 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int b
 // chunk end (the input of that chunk's gradients), then dh0.
 // ---------------------------------------------------------------------------
 template <int K, typename TIn>
-__device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int b, int h, int v0) {
+__device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
+  const BwdSeq seq = seq_of(p, n);
   using L = ScanLds<K, TIn>;
   constexpr int PER = K / 64, LB = L::LB;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
@@ -945,7 +1042,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
   u16 *duT = reinterpret_cast<u16 *>(base + L::OFF_A), *gxT = duT + 2 * 16 * LB;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
-  const long kv = (static_cast<long>(b) * p.Hv + h) * K * p.V;
+  const long kv = (static_cast<long>(n) * p.Hv + h) * K * p.V;
   float4_t ds[PER];
 #pragma unroll
   for (int m = 0; m < PER; ++m) {
@@ -956,16 +1053,12 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     }
   }
   ScanStage<K, TIn, true> stage;
-  if (p.n > 0) stage.load(p, b, h, hk, p.n - 1, v0);
-  for (int i = p.n - 1; i >= 0; --i) {
-    float *wds = p.ws_dS + rec(p, b, h, i) * K * p.V;
+  if (seq.n > 0) stage.load(p, seq, h, hk, seq.n - 1, v0);
+  for (int i = seq.n - 1; i >= 0; --i) {
+    float *wds = p.ws_dS + rec(p, seq, h, i) * K * p.V;
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int kk = 16 * (wave + 4 * m) + 4 * g4 + r;
-        wds[static_cast<long>(kk) * p.V + v0 + c] = ds[m][r];
-      }
+      put_state_tile<K, TIn>(wds, p.V, v0, wave + 4 * m, ds[m]);
       put_state_rows<K, TIn>(sds, 16 * (wave + 4 * m) + 4 * g4, c, ds[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sdu);
@@ -975,7 +1068,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
 #pragma unroll
       for (int r = 0; r < 4; ++r) jv[m][r] = stage.jr[m][r];
     }
-    if (i > 0) stage.load(p, b, h, hk, i - 1, v0);
+    if (i > 0) stage.load(p, seq, h, hk, i - 1, v0);
     __syncthreads();
     // dU = dU0 + E K dS'
     const float4_t kd = k_times_state<K, TIn>(sk, 16 * wave, sds);
@@ -1045,8 +1138,8 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
 }
 
 // The two scans are independent (the reverse one needs the per-chunk records
-// and dht, not the states), so one launch runs both: pair z = (role, batch
-// row, value head), role 0 the forward pass, 1 the reverse pass. Two
+// and dht, not the states), so one launch runs both: pair z = (role,
+// sequence, value head), role 0 the forward pass, 1 the reverse pass. Two
 // workgroups fit a CU, so each CU overlaps a forward and a reverse scan.
 // Workgroups go to the XCDs round-robin by linear index; the V/16 tiles of
 // one pair read the same K rows and T records every step, so when the pairs
@@ -1062,15 +1155,15 @@ __global__ __launch_bounds__(BNT) void bwd_scans_kernel(BwdParams p) {
   extern __shared__ __align__(16) float lds[];
   PBGDN_POISON_LDS(lds, (scan_lds<K, TIn>()));
   PBGDN_POISON_SYNC();
-  const int tiles = p.V / 16, pairs = 2 * p.B * p.Hv;
+  const int tiles = p.V / 16, pairs = 2 * p.num_seqs * p.Hv;
   const int l = blockIdx.x;
   int pair, tile;
   xcd_group(l, pairs, tiles, p.xcds, pair, tile);
-  const int role_b = pair / p.Hv, h = pair % p.Hv;
-  if (role_b < p.B) {
-    state_pass<K, TIn>(p, lds, role_b, h, 16 * tile);
+  const int role_seq = pair / p.Hv, h = pair % p.Hv;
+  if (role_seq < p.num_seqs) {
+    state_pass<K, TIn>(p, lds, role_seq, h, 16 * tile);
   } else {
-    adjoint_pass<K, TIn>(p, lds, role_b - p.B, h, 16 * tile);
+    adjoint_pass<K, TIn>(p, lds, role_seq - p.num_seqs, h, 16 * tile);
   }
 }
 
@@ -1132,7 +1225,10 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
   // bf16 inputs: the tile's S^T and dS'^T as high and low bf16 parts, [16][LS]
   u16 *shT = reinterpret_cast<u16 *>(sred + GNT / 64 + 8), *slT = shT + 16 * LS, *dhT = slT + 16 * LS,
       *dlT = dhT + 16 * LS;
-  const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int h = blockIdx.y;
+  BwdSeq seq;
+  int i;
+  if (!chunk_of(p, blockIdx.x, blockIdx.z, seq, i)) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int half = wave >> 2, tw = 16 * (wave & 3);  // column half; this wave's token rows
   const bool chain = half == 0;
@@ -1140,16 +1236,16 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
   const int t0 = i * BC;
   if (tid < BNT) {  // the loads run on the first four waves
     RawRows<TIn, K> rq, rk;
-    rq.load(p.q, p, b, t0, p.Hk, hk, K);
-    rk.load(p.k, p, b, t0, p.Hk, hk, K);
+    rq.load(p.q, seq, t0, p.Hk, hk, K);
+    rk.load(p.k, seq, t0, p.Hk, hk, K);
     rq.put(sq, LK);
     rk.put(sk, LK);
     if constexpr (BF) {
-      load_t_pair(tp, LB, p.ws_T + rec(p, b, h, i) * BC * BC);
+      load_t_pair(tp, LB, p.ws_T + rec(p, seq, h, i) * BC * BC);
     } else {
-      load_t(st, p.ws_T + rec(p, b, h, i) * BC * BC);
+      load_t(st, p.ws_T + rec(p, seq, h, i) * BC * BC);
     }
-    load_decays(p, b, h, i, sc, sgam, se, sbeta);
+    load_decays(p, seq, h, i, sc, sgam, se, sbeta);
     if (tid < BC) {
       sdgam[tid] = 0.f;
       sde[tid] = 0.f;
@@ -1183,7 +1279,7 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
 #pragma unroll
   for (int m = 0; m < 2; ++m) dtb[m] = dm[m] = zero4();
   float dgam_r[4] = {0.f, 0.f, 0.f, 0.f}, de_r[4] = {0.f, 0.f, 0.f, 0.f}, dgc = 0.f;
-  const long kv = rec(p, b, h, i) * K * V;
+  const long kv = rec(p, seq, h, i) * K * V;
   // Columns v0 .. v0+15 of the start state and end adjoint (K rows of four
   // float4) and of V and dO (16-byte pieces of TIn), fetched into registers a
   // tile ahead by the first four waves and placed in LDS between tiles.
@@ -1200,9 +1296,8 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
       rd[m] = *reinterpret_cast<const float4_t *>(p.ws_dS + o);
     }
     const int row = tid / PPR, part = tid % PPR, t = t0 + row;
-    const long off = (((static_cast<long>(b) * p.T + t) * p.Hv + h) * V + v0) * static_cast<long>(sizeof(TIn)) +
-                     part * 16;
-    const bool ok = tid < BC * PPR && t < p.T;
+    const long off = (((seq.bos + t) * p.Hv + h) * V + v0) * static_cast<long>(sizeof(TIn)) + part * 16;
+    const bool ok = tid < BC * PPR && t < seq.len;
     rv = ok ? *reinterpret_cast<const uint4 *>(static_cast<const unsigned char *>(p.v) + off) : uint4{0u, 0u, 0u, 0u};
     ro = ok ? *reinterpret_cast<const uint4 *>(static_cast<const unsigned char *>(p.dout) + off)
             : uint4{0u, 0u, 0u, 0u};
@@ -1339,8 +1434,8 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
         const int t = tw + 4 * g4 + r;
         if constexpr (!BF) sdx[t * LT + c] = dx[r];
         gx[r] = -sgam[t] * dx[r];
-        if (t0 + t < p.T) {
-          store_el<TIn>(p.dv, ((static_cast<long>(b) * p.T + t0 + t) * p.Hv + h) * V + v0 + c, dx[r]);
+        if (t0 + t < seq.len) {
+          store_el<TIn>(p.dv, ((seq.bos + t0 + t) * p.Hv + h) * V + v0 + c, dx[r]);
         }
         dgam_r[r] -= ks[r] * dx[r];
       }
@@ -1586,13 +1681,13 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = t0 + tw + 4 * g4 + r, kk = 16 * (half * KH + m) + c;
-      if (t >= p.T) continue;
+      if (t >= seq.len) continue;
       if (direct) {
-        const long o = ((static_cast<long>(b) * p.T + t) * p.Hk + hk) * K + kk;
+        const long o = ((seq.bos + t) * p.Hk + hk) * K + kk;
         store_el<TIn>(p.dq, o, dq[m][r]);
         store_el<TIn>(p.dk, o, dk[m][r]);
       } else {
-        const long o = ((static_cast<long>(b) * p.T + t) * p.Hv + h) * K + kk;
+        const long o = ((seq.bos + t) * p.Hv + h) * K + kk;
         p.ws_dq[o] = dq[m][r];
         p.ws_dk[o] = dk[m][r];
       }
@@ -1621,13 +1716,15 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
       const float y = __shfl_down(dcv, off, 64);
       if (lane + off < 64) dcv += y;
     }
-    if (t0 + t < p.T) {
-      const long o = (static_cast<long>(b) * p.T + t0 + t) * p.Hv + h;
+    if (t0 + t < seq.len) {
+      const long o = (seq.bos + t0 + t) * p.Hv + h;
       p.dg[o] = dcv;
       store_elem(p.dbeta, o, p.beta_dtype, dbt);
     }
   }
 }
+
+#include "chunk_bwd_bf16.hpp"
 
 // dq, dk [B,T,Hk,K] = sum over the Hv/Hk value heads of each key head.
 __global__ __launch_bounds__(BNT) void bwd_gqa_reduce_kernel(BwdParams p) {
@@ -1636,6 +1733,7 @@ __global__ __launch_bounds__(BNT) void bwd_gqa_reduce_kernel(BwdParams p) {
   for (long e = static_cast<long>(blockIdx.x) * BNT + threadIdx.x; e < total; e += static_cast<long>(gridDim.x) * BNT) {
     const long kk = e % p.K, rest = e / p.K;
     const long hk = rest % p.Hk, bt = rest / p.Hk;
+    if (p.cu_seqlens && (bt < p.cu_seqlens[0] || bt >= p.cu_seqlens[p.num_seqs])) continue;  // zeroed already
     const long base = (bt * p.Hv + hk * group) * p.K + kk;
     float sq = 0.f, sk = 0.f;
     for (int m = 0; m < group; ++m) {
@@ -1668,12 +1766,37 @@ int launch(Kern kernel, dim3 grid, size_t lds, hipStream_t st, const BwdParams &
   return hipGetLastError() == hipSuccess ? PBGDN_OK : PBGDN_ERR_LAUNCH;
 }
 
+// Value heads of a key head that one workgroup of the bf16 gradient kernel
+// takes in turn: all of them (dq and dk are then summed in registers, with no
+// float32 copies per value head and no reduction pass), unless the call is so
+// small that one head per workgroup (one workgroup a CU) needs fewer rounds of
+// the CUs by more than a quarter: the reduction and the float32 copies cost
+// about an eighth (67 us beside 13 rounds of 30 us at 6,011 tokens of 32 heads).
+int grad_heads(const BwdParams &p) {
+  const long group = p.Hv / p.Hk, items = static_cast<long>(p.records) * p.Hk, cus = p.cus > 0 ? p.cus : 1;
+  const long together = (items + cus - 1) / cus * group, apart = (items * group + cus - 1) / cus;
+  return 4 * together <= 5 * apart ? static_cast<int>(group) : 1;
+}
+
+template <int K, int V>
+int launch_grad_bf16(const BwdParams &p, int heads, hipStream_t st) {
+  using L = GradLds<K, V>;
+  static_assert(L::BYTES <= 160 * 1024, "LDS budget");
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(bwd_grad_bf16_kernel<K, V>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L::BYTES)) != hipSuccess) {
+    return PBGDN_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL((bwd_grad_bf16_kernel<K, V>), dim3(p.cu_seqlens ? p.records : p.n, p.Hv / heads, p.B),
+                     dim3(L::NT), L::BYTES, st, p, heads);
+  return hipGetLastError() == hipSuccess ? PBGDN_OK : PBGDN_ERR_LAUNCH;
+}
+
 template <int K, int V>
 int run_backward(const BwdParams &p, hipStream_t st) {
   static_assert(grad_lds<K, float>() <= 160 * 1024 && grad_lds<K, u16>() <= 160 * 1024 && local_lds<K, V, float>() <= 160 * 1024, "LDS budget");
-  const dim3 per_chunk(p.n, p.Hv, p.B), per_tile2((V / 16) * p.Hv * 2 * p.B);
+  const dim3 per_chunk(p.cu_seqlens ? p.records : p.n, p.Hv, p.B), per_tile2((V / 16) * p.Hv * 2 * p.num_seqs);
   int rc = PBGDN_OK;
-  if (p.n > 0) {
+  if (p.records > 0) {
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_local_kernel<K, V, float>, per_chunk, local_lds<K, V, float>(), st, p); break;
       case PBGDN_BF16: rc = launch(bwd_local_kernel<K, V, u16>, per_chunk, local_lds<K, V, u16>(), st, p); break;
@@ -1687,14 +1810,18 @@ int run_backward(const BwdParams &p, hipStream_t st) {
       default: rc = launch(bwd_scans_kernel<K, half_t>, per_tile2, scan_lds<K, half_t>(), st, p); break;
     }
   }
-  if (rc == PBGDN_OK && p.n > 0) {
+  int heads = 1;  // value heads of a gradient workgroup
+  if (rc == PBGDN_OK && p.records > 0) {
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_grad_kernel<K, V, float>, per_chunk, grad_lds<K, float>(), st, p, GNT); break;
-      case PBGDN_BF16: rc = launch(bwd_grad_kernel<K, V, u16>, per_chunk, grad_lds<K, u16>(), st, p, GNT); break;
+      case PBGDN_BF16:
+        heads = grad_heads(p);
+        rc = launch_grad_bf16<K, V>(p, heads, st);
+        break;
       default: rc = launch(bwd_grad_kernel<K, V, half_t>, per_chunk, grad_lds<K, half_t>(), st, p, GNT); break;
     }
   }
-  if (rc == PBGDN_OK && p.n > 0 && p.Hk != p.Hv) {
+  if (rc == PBGDN_OK && p.records > 0 && heads * p.Hk != p.Hv) {
     const long total = static_cast<long>(p.B) * p.T * p.Hk * K;
     const unsigned blocks = static_cast<unsigned>(std::min<long>((total + BNT - 1) / BNT, 65535L));
     hipLaunchKernelGGL(bwd_gqa_reduce_kernel, dim3(blocks), dim3(BNT), 0, st, p);
@@ -1711,21 +1838,24 @@ long ws_record_floats(int K, int V) {
 }  // namespace
 }  // namespace pbgdn
 
-extern "C" size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K, int V) {
-  using namespace pbgdn;
-  if (B < 0 || T < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0) return 0;
-  const long n = (static_cast<long>(T) + BC - 1) / BC;
-  long floats = static_cast<long>(B) * Hv * n * ws_record_floats(K, V);
-  if (Hk != Hv) floats += 2L * B * T * Hv * K;
+namespace pbgdn {
+namespace {
+
+size_t workspace_bytes_of(long records, long tokens, int Hk, int Hv, int K, int V) {
+  long floats = records * Hv * ws_record_floats(K, V);
+  if (Hk != Hv) floats += 2L * tokens * Hv * K;
   return static_cast<size_t>(floats) * sizeof(float) + 256;
 }
 
-extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int in_dtype, const float *g,
-                               const void *beta, int beta_dtype, const float *h0, const void *dout, int do_dtype,
-                               const float *dht, void *dq, void *dk, void *dv, float *dg, void *dbeta, float *dh0,
-                               void *workspace, size_t workspace_bytes, int B, int T, int Hk, int Hv, int K, int V,
-                               float scale, void *stream) {
-  using namespace pbgdn;
+// Chunk records of a packed call: see BwdSeq.
+long packed_records(long tokens, long num_seqs) { return tokens / BC + num_seqs + 1; }
+
+// Both entry points: B rows of T tokens, or (cu_seqlens) num_seqs sequences
+// packed into B = 1 row.
+int backward(const void *q, const void *k, const void *v, int in_dtype, const float *g, const void *beta,
+             int beta_dtype, const float *h0, const int32_t *cu_seqlens, int num_seqs, const void *dout, int do_dtype,
+             const float *dht, void *dq, void *dk, void *dv, float *dg, void *dbeta, float *dh0, void *workspace,
+             size_t workspace_bytes, int B, int T, int Hk, int Hv, int K, int V, float scale, void *stream) {
   if (B < 0 || T < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0 || Hv % Hk != 0) return PBGDN_ERR_INVALID_ARGUMENT;
   auto dtype_ok = [](int d) { return d == PBGDN_F32 || d == PBGDN_BF16 || d == PBGDN_F16; };
   if (!dtype_ok(in_dtype) || !dtype_ok(beta_dtype) || !dtype_ok(do_dtype)) return PBGDN_ERR_INVALID_ARGUMENT;
@@ -1734,18 +1864,19 @@ extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int 
     if (B > 0 && dh0 == nullptr) return PBGDN_OK;
   }
   const long n = (static_cast<long>(T) + BC - 1) / BC;
+  const long records = n == 0 ? 0 : cu_seqlens ? packed_records(T, num_seqs) : B * n;
   if (n > 0 && (!q || !k || !v || !g || !beta || !dout || !dq || !dk || !dv || !dg || !dbeta)) {
     return PBGDN_ERR_INVALID_ARGUMENT;
   }
   if (B == 0) return PBGDN_OK;
-  if (n > 65535 || Hv > 65535 || B > 32767) return PBGDN_ERR_UNSUPPORTED;
-  if (static_cast<long>(V / 16) * Hv * 2 * B > 0x7fffffffL) return PBGDN_ERR_UNSUPPORTED;  // the scans' 1-D grid
-  if (!workspace || workspace_bytes < pbgdn_chunk_bwd_workspace_size(B, T, Hk, Hv, K, V) ||
+  if ((!cu_seqlens && n > 65535) || records > (1L << 22) || Hv > 65535 || B > 32767) return PBGDN_ERR_UNSUPPORTED;
+  if (static_cast<long>(V / 16) * Hv * 2 * num_seqs > 0x7fffffffL) return PBGDN_ERR_UNSUPPORTED;  // the scans' 1-D grid
+  if (!workspace || workspace_bytes < workspace_bytes_of(records, static_cast<long>(B) * T, Hk, Hv, K, V) ||
       reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
     return PBGDN_ERR_INVALID_ARGUMENT;
   }
   float *ws = static_cast<float *>(workspace);
-  const long recs = static_cast<long>(B) * Hv * n;
+  const long recs = records * Hv;
   {  // debug builds: the gradients and the workspace start as NaN
     hipStream_t s = static_cast<hipStream_t>(stream);
     const long isz = in_dtype == PBGDN_F32 ? 4 : 2, bsz = beta_dtype == PBGDN_F32 ? 4 : 2;
@@ -1755,12 +1886,13 @@ extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int 
     debug_poison(dv, static_cast<size_t>(bt * Hv * V * isz), s);
     debug_poison(dg, static_cast<size_t>(bt * Hv * 4), s);
     debug_poison(dbeta, static_cast<size_t>(bt * Hv * bsz), s);
-    debug_poison(dh0, static_cast<size_t>(static_cast<long>(B) * Hv * K * V * 4), s);
+    debug_poison(dh0, static_cast<size_t>(static_cast<long>(num_seqs) * Hv * K * V * 4), s);
     debug_poison(workspace, workspace_bytes, s);
   }
   BwdParams p{};
   DeviceShape shape;
   if (!device_shape(shape)) return PBGDN_ERR_LAUNCH;
+  p.cus = shape.cus;
   p.xcds = shape.xcds;
   p.q = q;
   p.k = k;
@@ -1786,6 +1918,9 @@ extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int 
   p.ws_dq = p.ws_dS + recs * K * V;
   p.ws_dk = Hk != Hv ? p.ws_dq + static_cast<long>(B) * T * Hv * K : nullptr;
   if (Hk == Hv) p.ws_dq = nullptr;
+  p.cu_seqlens = cu_seqlens;
+  p.num_seqs = num_seqs;
+  p.records = static_cast<int>(records);
   p.in_dtype = in_dtype;
   p.beta_dtype = beta_dtype;
   p.B = B;
@@ -1799,4 +1934,39 @@ extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int 
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (K == 64) return V == 64 ? run_backward<64, 64>(p, st) : run_backward<64, 128>(p, st);
   return V == 64 ? run_backward<128, 64>(p, st) : run_backward<128, 128>(p, st);
+}
+}  // namespace
+}  // namespace pbgdn
+
+extern "C" size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K, int V) {
+  using namespace pbgdn;
+  if (B < 0 || T < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0) return 0;
+  return workspace_bytes_of(static_cast<long>(B) * ((static_cast<long>(T) + BC - 1) / BC), static_cast<long>(B) * T, Hk,
+                            Hv, K, V);
+}
+
+extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int in_dtype, const float *g,
+                               const void *beta, int beta_dtype, const float *h0, const void *dout, int do_dtype,
+                               const float *dht, void *dq, void *dk, void *dv, float *dg, void *dbeta, float *dh0,
+                               void *workspace, size_t workspace_bytes, int B, int T, int Hk, int Hv, int K, int V,
+                               float scale, void *stream) {
+  return pbgdn::backward(q, k, v, in_dtype, g, beta, beta_dtype, h0, nullptr, B, dout, do_dtype, dht, dq, dk, dv, dg,
+                         dbeta, dh0, workspace, workspace_bytes, B, T, Hk, Hv, K, V, scale, stream);
+}
+
+extern "C" size_t pbgdn_chunk_bwd_packed_workspace_size(int T, int num_seqs, int Hk, int Hv, int K, int V) {
+  using namespace pbgdn;
+  if (T < 0 || num_seqs < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0) return 0;
+  return workspace_bytes_of(T == 0 ? 0 : packed_records(T, num_seqs), T, Hk, Hv, K, V);
+}
+
+extern "C" int pbgdn_chunk_bwd_packed(const void *q, const void *k, const void *v, int in_dtype, const float *g,
+                                      const void *beta, int beta_dtype, const float *h0, const int32_t *cu_seqlens,
+                                      int num_seqs, const void *dout, int do_dtype, const float *dht, void *dq,
+                                      void *dk, void *dv, float *dg, void *dbeta, float *dh0, void *workspace,
+                                      size_t workspace_bytes, int T, int Hk, int Hv, int K, int V, float scale,
+                                      void *stream) {
+  if (!cu_seqlens || num_seqs < 0) return PBGDN_ERR_INVALID_ARGUMENT;
+  return pbgdn::backward(q, k, v, in_dtype, g, beta, beta_dtype, h0, cu_seqlens, num_seqs, dout, do_dtype, dht, dq, dk,
+                         dv, dg, dbeta, dh0, workspace, workspace_bytes, 1, T, Hk, Hv, K, V, scale, stream);
 }

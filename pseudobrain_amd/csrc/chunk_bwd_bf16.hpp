@@ -1,0 +1,610 @@
+// The gradient kernel of the chunk backward for bfloat16 inputs (included by
+// chunk_bwd.hip, whose notation and helpers it uses).
+//
+// One workgroup of V / 16 waves per (chunk, key head), the value heads of the
+// key head in turn, so dq and dk are summed over them in registers. For each
+// value head:
+//
+//   chain    wave w holds the 16 value columns 16 w .. of the start state S
+//            and the end adjoint dS' in registers and forms its columns of
+//            X = V - Gamma K S, U = T beta X, dU = M^T dO + E K dS' and
+//            dX = beta T^T dU with no barrier: an accumulator tile is the B
+//            operand of the next product as it stands, once the contraction
+//            slots of the A operand are numbered to match (below).
+//   stages   the contractions over the value columns need every wave's
+//            columns: X, dU, then U, dX and the states pass through LDS as
+//            transposed bf16 high / low halves, one pair at a time, and the
+//            waves share out the output tiles:
+//            dTb = dU X^T, dM = dO U^T (64 x 64), dK1 = U dS'^T,
+//            dK2 = dX S^T, dQ0 = dO S^T (64 x K).
+//   C x C    the gradient through M, T and A, and the sums for dg and dbeta.
+//
+// Row sums that would need K S, K dS' or Q S again come from the K-wide
+// products: sum_v (K dS' o U)_t = sum_k (K o dK1)_t, likewise with dX and dQ0.
+// LDS: 150 KiB at K = V = 128, so one workgroup a CU, eight waves.
+//
+// Contraction slots: the B operand of a 32-row step kb made of two
+// accumulator tiles holds, in lane (c, g), rows 32 kb + 4 g + j (j < 4) and
+// 32 kb + 16 + 4 g + j - 4 of column c; A operands are read in that order (two
+// 8-byte pieces of a row, or two transposing reads).
+
+// The operand reads of one lane (c, g). A struct rather than functions of
+// threadIdx.x, so that a kernel can make its lane opaque to the compiler where
+// addresses and comparisons must not be kept across a loop.
+struct Lane {
+  int c, g;
+
+  // Four rows 4 g .. of column col0 + c of a row-major bf16 array (ds_read_tr16).
+  __device__ __forceinline__ bw_i16x4_t tr(const u16 *m, int ld, int col0) const {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) bw_i16x4_t *)(m + (4 * g + (c >> 2)) * ld + col0 + 4 * (c & 3)));
+  }
+  // Rows row0 + c of a row-major bf16 array as the operand of step kb.
+  __device__ __forceinline__ bh8_t rows(const u16 *m, int ld, int row0, int kb) const {
+    const u16 *a = m + (row0 + c) * ld + 32 * kb + 4 * g;
+    const v2u32_t x = *reinterpret_cast<const v2u32_t *>(a), y = *reinterpret_cast<const v2u32_t *>(a + 16);
+    return __builtin_bit_cast(bh8_t, v4u32_t{x[0], x[1], y[0], y[1]});
+  }
+  // The same with the slots in order (both operands read this way).
+  __device__ __forceinline__ bh8_t rows16(const u16 *m, int ld, int row0, int kb) const {
+    return *reinterpret_cast<const bh8_t *>(m + (row0 + c) * ld + 32 * kb + 8 * g);
+  }
+  // Columns col0 + c, contraction over the array's rows 32 kb ..
+  __device__ __forceinline__ bh8_t cols(const u16 *m, int ld, int kb, int col0) const {
+    const bw_i16x4_t x = tr(m + 32 * kb * ld, ld, col0), y = tr(m + (32 * kb + 16) * ld, ld, col0);
+    return __builtin_bit_cast(bh8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+  // Rows a0 .. of a times rows b0 .. of b, over KD columns.
+  template <int KD>
+  __device__ __forceinline__ float4_t rows_rows(const u16 *a, const u16 *b, int ld, int a0, int b0) const {
+    float4_t acc = zero4();
+#pragma unroll
+    for (int kb = 0; kb < KD / 32; ++kb) acc = mfma_bf16(rows16(a, ld, a0, kb), rows16(b, ld, b0, kb), acc);
+    return acc;
+  }
+};
+
+__device__ __forceinline__ bh8_t frag_pair(v2u32_t x, v2u32_t y) {
+  return __builtin_bit_cast(bh8_t, v4u32_t{x[0], x[1], y[0], y[1]});
+}
+
+// Four bf16 (a transposing read's result) as float.
+__device__ __forceinline__ float4_t bf16x4_float(bw_i16x4_t x) {
+  const v2u32_t w = __builtin_bit_cast(v2u32_t, x);
+  return float4_t{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16),
+                  __uint_as_float(w[1] & 0xffff0000u)};
+}
+
+template <int K, int V>
+struct GradLds {
+  static constexpr int NW = V / 16, NT = 64 * NW, COLS = NW / 2;  // waves; wave pairs
+  static constexpr int LK = K + 8, LV = V + 8, LB = BC + 8;       // row strides (elements)
+  static constexpr int CC = BC * LB;                              // one 64 x 64 half
+  static constexpr int TV = V * LB;                               // one V x 64 half
+  // the shared area: M^T pair and V rows (chain); X^T and dU^T pairs; the U^T
+  // or dX^T pair and one state half; four C x C pairs
+  static constexpr int AREA = 4 * TV > 8 * CC ? 4 * TV : (2 * TV + V * LK > 8 * CC ? 2 * TV + V * LK : 8 * CC);
+  static_assert(2 * CC + BC * LV <= AREA && 2 * TV + V * LK <= AREA, "the area's uses");
+  static constexpr int FLOATS = 4 * BC + 4 * COLS * BC + 4 * BC + 16;
+  static constexpr size_t BYTES = sizeof(u16) * (2 * BC * LK + BC * LV + 2 * CC + AREA) + sizeof(float) * FLOATS;
+};
+
+template <int K, int V>
+__global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int heads) {
+  using L = GradLds<K, V>;
+  constexpr int NW = L::NW, NT = L::NT, COLS = L::COLS, LK = L::LK, LV = L::LV, LB = L::LB, CC = L::CC, TV = L::TV;
+  constexpr int KT = K / 16, KB = K / 32, VB = V / 32;
+  constexpr int KTW = KT / COLS, CTW = 4 / COLS;  // key tiles, C x C column tiles of a wave
+  extern __shared__ __align__(16) float lds[];
+  PBGDN_POISON_LDS(lds, L::BYTES);
+  PBGDN_POISON_SYNC();
+  BwdSeq seq;
+  int i;
+  if (!chunk_of(p, blockIdx.x, blockIdx.z, seq, i)) return;
+  const int t0 = i * BC;
+  const int group = p.Hv / p.Hk;
+  float4_t tq[KTW][2], tk[KTW][2];
+#pragma unroll
+  for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) tq[m][a] = tk[m][a] = zero4();
+  }
+  for (int hh = 0; hh < heads; ++hh) {
+    // The LDS base and the thread index are made opaque in each round: the
+    // compiler otherwise keeps every phase's addresses and comparisons in
+    // registers across the loop (212 spilled registers a lane).
+    int base = 0, tid = threadIdx.x;
+    asm volatile("" : "+s"(base), "+v"(tid));
+    const int lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+    const Lane L4{c, g4};
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), v0 = 16 * wave;
+    const int rp = wave & 1, cp = wave >> 1;  // row tiles 2 rp, 2 rp + 1; column (key) tiles of pair cp
+    u16 *sq = reinterpret_cast<u16 *>(lds + base), *sk = sq + BC * LK, *sdo = sk + BC * LK, *tp = sdo + BC * LV,
+        *area = tp + 2 * CC;
+    float *sc = reinterpret_cast<float *>(area + L::AREA), *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
+    // partial sums: rows by wave pair (dc, dbeta, dgamma, de), columns by wave parity
+    float *prc = sbeta + BC, *prb = prc + COLS * BC, *pdg = prb + COLS * BC, *pde = pdg + COLS * BC;
+    float *pcc = pde + COLS * BC, *pcb = pcc + 2 * BC, *sred = pcb + 2 * BC;
+    const int h = blockIdx.y * heads + hh, hk = h / group;
+    const long r = rec(p, seq, h, i);
+    // ---- this head's inputs
+    float4_t sf[KT], df[KT];
+    {
+      const float4_t *ws = reinterpret_cast<const float4_t *>(p.ws_S + r * K * V) + wave * KT * 64 + lane;
+      const float4_t *wd = reinterpret_cast<const float4_t *>(p.ws_dS + r * K * V) + wave * KT * 64 + lane;
+#pragma unroll
+      for (int m = 0; m < KT; ++m) sf[m] = ws[64 * m];
+#pragma unroll
+      for (int m = 0; m < KT; ++m) df[m] = wd[64 * m];
+    }
+    u16 *mt = area, *sv = area + 2 * CC;
+    {
+      RawRows<u16, V, NT> rv, rd;
+      float4_t rt[BC * BC / 4 / NT];
+      rd.load(tid, p.dout, seq, t0, p.Hv, h, V);
+      rv.load(tid, p.v, seq, t0, p.Hv, h, V);
+      const float4_t *wt = reinterpret_cast<const float4_t *>(p.ws_T + r * BC * BC);
+#pragma unroll
+      for (int m = 0; m < BC * BC / 4 / NT; ++m) rt[m] = wt[tid + NT * m];
+      const float cv = p.ws_c[r * BC + lane], bv = p.ws_beta[r * BC + lane], last = p.ws_c[r * BC + BC - 1];
+      if (hh > 0) __syncthreads();  // the previous head's readers of LDS are done
+      if (hh == 0) {
+        RawRows<u16, K, NT> rq, rk;
+        rq.load(tid, p.q, seq, t0, p.Hk, hk, K);
+        rk.load(tid, p.k, seq, t0, p.Hk, hk, K);
+        rq.put(tid, sq, LK);
+        rk.put(tid, sk, LK);
+      }
+      rd.put(tid, sdo, LV);
+      rv.put(tid, sv, LV);
+#pragma unroll
+      for (int m = 0; m < BC * BC / 4 / NT; ++m) {
+        const int e = tid + NT * m;
+        v2u32_t hi, lo;
+        split_bf16(rt[m], hi, lo);
+        *reinterpret_cast<v2u32_t *>(tp + (e >> 4) * LB + 4 * (e & 15)) = hi;
+        *reinterpret_cast<v2u32_t *>(tp + CC + (e >> 4) * LB + 4 * (e & 15)) = lo;
+      }
+      if (tid < BC) {
+        sc[tid] = cv;
+        sgam[tid] = expf(cv);
+        se[tid] = expf(last - cv);
+        sbeta[tid] = bv;
+      }
+    }
+    __syncthreads();
+    // ---- M^T[s][t] = scale (k_s . q_t) e^(c_t - c_s), t >= s: rows of pair rp
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        const int ts = 2 * rp + a, tt = CTW * cp + m;
+        const float4_t kq = L4.rows_rows<K>(sk, sq, LK, 16 * ts, 16 * tt);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int s2 = 16 * ts + 4 * g4 + e, t = 16 * tt + c;
+          put_pair1(mt, CC, s2 * LB + t, t >= s2 ? p.scale * kq[e] * expf(sc[t] - sc[s2]) : 0.f);
+        }
+      }
+    }
+    // ---- chain: this wave's 16 value columns
+    float dgc = 0.f;
+    v2u32_t sh[KT], sl[KT], dh[KT], dl[KT];
+#pragma unroll
+    for (int m = 0; m < KT; ++m) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dgc += sf[m][e] * df[m][e];
+      split_bf16(sf[m], sh[m], sl[m]);
+      split_bf16(df[m], dh[m], dl[m]);
+    }
+    dgc = wave_sum(dgc);
+    if (lane == 0) sred[wave] = dgc;
+    float4_t du[4];
+    v2u32_t xh[4], xl[4], bxh[4], bxl[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      float4_t ks = zero4(), kd = zero4();
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const bh8_t a = L4.rows(sk, LK, 16 * rt, kb);
+        ks = mfma_bf16(a, frag_pair(sh[2 * kb], sh[2 * kb + 1]), ks);
+        kd = mfma_bf16(a, frag_pair(dh[2 * kb], dh[2 * kb + 1]), kd);
+        ks = mfma_bf16(a, frag_pair(sl[2 * kb], sl[2 * kb + 1]), ks);
+        kd = mfma_bf16(a, frag_pair(dl[2 * kb], dl[2 * kb + 1]), kd);
+      }
+      const int o = 16 * rt + 4 * g4;
+      const float4_t x = bf16x4_float(L4.tr(sv + 16 * rt * LV, LV, v0)) - ld4(&sgam[o]) * ks;
+      split_bf16(x, xh[rt], xl[rt]);
+      split_bf16(x * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
+      du[rt] = ld4(&se[o]) * kd;
+    }
+    __syncthreads();  // M^T is complete
+    v2u32_t duh[4], dul[4];
+    {
+      bh8_t dof[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) dof[kb] = L4.cols(sdo, LV, kb, v0);
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+#pragma unroll
+        for (int kb = rt >> 1; kb < 2; ++kb) {  // t >= s
+          du[rt] = mfma_bf16(L4.rows(mt, LB, 16 * rt, kb), dof[kb], du[rt]);
+          du[rt] = mfma_bf16(L4.rows(mt + CC, LB, 16 * rt, kb), dof[kb], du[rt]);
+        }
+        split_bf16(du[rt], duh[rt], dul[rt]);
+      }
+    }
+    v2u32_t uh[4], ul[4], dxh[4], dxl[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      float4_t u = zero4(), dx = zero4();
+#pragma unroll
+      for (int kb = 0; kb <= rt >> 1; ++kb) {  // U = T (beta X), s <= t
+        const bh8_t th = L4.rows(tp, LB, 16 * rt, kb), tl = L4.rows(tp + CC, LB, 16 * rt, kb);
+        const bh8_t bh = frag_pair(bxh[2 * kb], bxh[2 * kb + 1]), bl = frag_pair(bxl[2 * kb], bxl[2 * kb + 1]);
+        u = mfma_bf16(th, bh, u);
+        u = mfma_bf16(th, bl, u);
+        u = mfma_bf16(tl, bh, u);
+      }
+#pragma unroll
+      for (int kb = rt >> 1; kb < 2; ++kb) {  // dX = beta T^T dU, t >= s
+        const bh8_t th = L4.cols(tp, LB, kb, 16 * rt), tl = L4.cols(tp + CC, LB, kb, 16 * rt);
+        const bh8_t bh = frag_pair(duh[2 * kb], duh[2 * kb + 1]), bl = frag_pair(dul[2 * kb], dul[2 * kb + 1]);
+        dx = mfma_bf16(th, bh, dx);
+        dx = mfma_bf16(th, bl, dx);
+        dx = mfma_bf16(tl, bh, dx);
+      }
+      dx *= ld4(&sbeta[16 * rt + 4 * g4]);
+      split_bf16(u, uh[rt], ul[rt]);
+      split_bf16(dx, dxh[rt], dxl[rt]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // dv = dX, rounded: its high half
+        const int t = t0 + 16 * rt + 4 * g4 + e;
+        if (t < seq.len) {
+          static_cast<u16 *>(p.dv)[((seq.bos + t) * p.Hv + h) * V + v0 + c] =
+              static_cast<u16>(dxh[rt][e >> 1] >> (16 * (e & 1)));
+        }
+      }
+    }
+    // ---- contractions over the value columns
+    u16 *a0 = area, *a1 = area + 2 * TV;
+    auto publish = [&](u16 *m, const v2u32_t (&hi)[4], const v2u32_t (&lo)[4]) {  // [V][64] transposed pair
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        *reinterpret_cast<v2u32_t *>(m + (v0 + c) * LB + 16 * rt + 4 * g4) = hi[rt];
+        *reinterpret_cast<v2u32_t *>(m + TV + (v0 + c) * LB + 16 * rt + 4 * g4) = lo[rt];
+      }
+    };
+    auto publish_state = [&](const v2u32_t (&x)[KT]) {  // [V][K] transposed half
+#pragma unroll
+      for (int m = 0; m < KT; ++m) *reinterpret_cast<v2u32_t *>(a1 + (v0 + c) * LK + 16 * m + 4 * g4) = x[m];
+    };
+    float4_t dtb[CTW][2], dm[CTW][2], dk1[KTW][2], dk2[KTW][2], dq0[KTW][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) dtb[m][a] = dm[m][a] = zero4();
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) dk1[m][a] = dk2[m][a] = dq0[m][a] = zero4();
+    }
+    __syncthreads();
+    publish(a0, xh, xl);
+    publish(a1, duh, dul);
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {  // dTb = dU X^T
+      bh8_t ah[2], al[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        ah[a] = L4.cols(a1, LB, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols(a1 + TV, LB, kb, 32 * rp + 16 * a);
+      }
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        const bh8_t bh = L4.cols(a0, LB, kb, 16 * (CTW * cp + m)), bl = L4.cols(a0 + TV, LB, kb, 16 * (CTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          dtb[m][a] = mfma_bf16(ah[a], bh, dtb[m][a]);
+          dtb[m][a] = mfma_bf16(ah[a], bl, dtb[m][a]);
+          dtb[m][a] = mfma_bf16(al[a], bh, dtb[m][a]);
+        }
+      }
+    }
+    __syncthreads();
+    publish(a0, uh, ul);
+    publish_state(dh);
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {  // dM = dO U^T; dK1 = U dS'^T, the high half of dS'
+      bh8_t od[2], ah[2], al[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols(a0 + TV, LB, kb, 32 * rp + 16 * a);
+      }
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        const bh8_t bh = L4.cols(a0, LB, kb, 16 * (CTW * cp + m)), bl = L4.cols(a0 + TV, LB, kb, 16 * (CTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          dm[m][a] = mfma_bf16(od[a], bh, dm[m][a]);
+          dm[m][a] = mfma_bf16(od[a], bl, dm[m][a]);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          dk1[m][a] = mfma_bf16(ah[a], b, dk1[m][a]);
+          dk1[m][a] = mfma_bf16(al[a], b, dk1[m][a]);
+        }
+      }
+    }
+    __syncthreads();
+    publish_state(dl);
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {  // dK1: the low half of dS'
+      const bh8_t a_0 = L4.cols(a0, LB, kb, 32 * rp), a_1 = L4.cols(a0, LB, kb, 32 * rp + 16);
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+        dk1[m][0] = mfma_bf16(a_0, b, dk1[m][0]);
+        dk1[m][1] = mfma_bf16(a_1, b, dk1[m][1]);
+      }
+    }
+    __syncthreads();
+    publish(a0, dxh, dxl);
+    publish_state(sh);
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {  // dK2 = dX S^T, dQ0 = dO S^T, the high half of S
+      bh8_t od[2], ah[2], al[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols(a0 + TV, LB, kb, 32 * rp + 16 * a);
+      }
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          dk2[m][a] = mfma_bf16(ah[a], b, dk2[m][a]);
+          dq0[m][a] = mfma_bf16(od[a], b, dq0[m][a]);
+          dk2[m][a] = mfma_bf16(al[a], b, dk2[m][a]);
+        }
+      }
+    }
+    __syncthreads();
+    publish_state(sl);
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {  // the low half of S
+      bh8_t od[2], ah[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
+      }
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          dk2[m][a] = mfma_bf16(ah[a], b, dk2[m][a]);
+          dq0[m][a] = mfma_bf16(od[a], b, dq0[m][a]);
+        }
+      }
+    }
+    // ---- the row scales, and the decay sums over the keys
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int o = 32 * rp + 16 * a + 4 * g4;
+      const float4_t gam = ld4(&sgam[o]), e4 = ld4(&se[o]);
+      float4_t dgam = zero4(), de = zero4();
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const int col = 16 * (KTW * cp + m);
+        const float4_t kx = bf16x4_float(L4.tr(sk + (32 * rp + 16 * a) * LK, LK, col));
+        const float4_t qx = bf16x4_float(L4.tr(sq + (32 * rp + 16 * a) * LK, LK, col));
+        dgam += p.scale * (qx * dq0[m][a]) - kx * dk2[m][a];
+        de += kx * dk1[m][a];
+        tq[m][a] += dq0[m][a] * (gam * p.scale);
+        tk[m][a] += e4 * dk1[m][a] - gam * dk2[m][a];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = group_sum(dgam[e], 16), y = group_sum(de[e], 16);
+        if (c == 0) {
+          pdg[cp * BC + o + e] = x;
+          pde[cp * BC + o + e] = y;
+        }
+      }
+    }
+    __syncthreads();  // the stages' readers are done: the area now holds the C x C pairs
+    u16 *b1p = area, *b2p = b1p + 2 * CC, *b3p = b2p + 2 * CC, *b4p = b3p + 2 * CC;
+    // dM o Mt into b1 (and its dc terms); dT = dTb diag(beta) into b2 (and dbeta)
+    float rc[2][4], rb[2][4], cc[CTW], cb[CTW];
+#pragma unroll
+    for (int m = 0; m < CTW; ++m) cc[m] = cb[m] = 0.f;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rc[a][e] = rb[a][e] = 0.f;
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        const int s2 = 16 * (CTW * cp + m) + c;
+        const float4_t qk = L4.rows_rows<K>(sq, sk, LK, 32 * rp + 16 * a, 16 * (CTW * cp + m));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = 32 * rp + 16 * a + 4 * g4 + e;
+          const float d = t >= s2 ? p.scale * expf(sc[t] - sc[s2]) : 0.f;
+          const float dmd = t >= s2 ? dm[m][a][e] * d : 0.f;
+          put_pair1(b1p, CC, t * LB + s2, dmd);
+          rc[a][e] += dmd * qk[e];
+          cc[m] -= dmd * qk[e];
+          put_pair1(b2p, CC, t * LB + s2, dtb[m][a][e] * sbeta[s2]);
+          cb[m] += dtb[m][a][e] * pair_val(tp, CC, t * LB + s2);
+        }
+      }
+    }
+    __syncthreads();
+    // W = T^T dT
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        float4_t w = zero4();
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const bh8_t th = L4.cols(tp, LB, kb, 32 * rp + 16 * a), tl = L4.cols(tp + CC, LB, kb, 32 * rp + 16 * a);
+          const bh8_t bh = L4.cols(b2p, LB, kb, 16 * (CTW * cp + m)),
+                      bl = L4.cols(b2p + CC, LB, kb, 16 * (CTW * cp + m));
+          w = mfma_bf16(th, bh, w);
+          w = mfma_bf16(th, bl, w);
+          w = mfma_bf16(tl, bh, w);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          put_pair1(b4p, CC, (32 * rp + 16 * a + 4 * g4 + e) * LB + 16 * (CTW * cp + m) + c, w[e]);
+        }
+      }
+    }
+    __syncthreads();
+    // dA = -W T^T (strict lower): H = dA beta_t D, as H + H^T in b3; dbeta, dc terms
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int m = 0; m < CTW; ++m) {
+        const int row0 = 32 * rp + 16 * a, col0 = 16 * (CTW * cp + m);
+        float4_t da = zero4();
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const bh8_t wh = L4.rows16(b4p, LB, row0, kb), wl = L4.rows16(b4p + CC, LB, row0, kb);
+          const bh8_t th = L4.rows16(tp, LB, col0, kb), tl = L4.rows16(tp + CC, LB, col0, kb);
+          da = mfma_bf16(wh, th, da);
+          da = mfma_bf16(wh, tl, da);
+          da = mfma_bf16(wl, th, da);
+        }
+        const float4_t gk = L4.rows_rows<K>(sk, sk, LK, row0, col0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = row0 + 4 * g4 + e, s2 = col0 + c;
+          const float d = t > s2 ? expf(sc[t] - sc[s2]) : 0.f;
+          const float dav = t > s2 ? -da[e] : 0.f;
+          const float hv = dav * sbeta[t] * d, b = dav * gk[e] * d;
+          rb[a][e] += b;
+          rc[a][e] += b * sbeta[t];
+          cc[m] -= b * sbeta[t];
+          if (t >= s2) {
+            put_pair1(b3p, CC, t * LB + s2, hv);
+            put_pair1(b3p, CC, s2 * LB + t, hv);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = group_sum(rc[a][e], 16), y = group_sum(rb[a][e], 16);
+        if (c == 0) {
+          prc[cp * BC + 32 * rp + 16 * a + 4 * g4 + e] = x;
+          prb[cp * BC + 32 * rp + 16 * a + 4 * g4 + e] = y;
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < CTW; ++m) {
+      const float x = add_xor32(add_xor16(cc[m])), y = add_xor32(add_xor16(cb[m]));
+      if (g4 == 0) {
+        pcc[rp * BC + 16 * (CTW * cp + m) + c] = x;
+        pcb[rp * BC + 16 * (CTW * cp + m) + c] = y;
+      }
+    }
+    __syncthreads();
+    // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + (H + H^T) K
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      bh8_t a1h[2], a1l[2], a3h[2], a3l[2], t1h[2], t1l[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int row0 = 32 * rp + 16 * a;
+        a1h[a] = L4.rows(b1p, LB, row0, kb);
+        a1l[a] = L4.rows(b1p + CC, LB, row0, kb);
+        a3h[a] = L4.rows(b3p, LB, row0, kb);
+        a3l[a] = L4.rows(b3p + CC, LB, row0, kb);
+        t1h[a] = L4.cols(b1p, LB, kb, row0);
+        t1l[a] = L4.cols(b1p + CC, LB, kb, row0);
+      }
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        const bh8_t kf = L4.cols(sk, LK, kb, 16 * (KTW * cp + m)), qf = L4.cols(sq, LK, kb, 16 * (KTW * cp + m));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          tq[m][a] = mfma_bf16(a1h[a], kf, tq[m][a]);
+          tk[m][a] = mfma_bf16(t1h[a], qf, tk[m][a]);
+          tq[m][a] = mfma_bf16(a1l[a], kf, tq[m][a]);
+          tk[m][a] = mfma_bf16(t1l[a], qf, tk[m][a]);
+          tk[m][a] = mfma_bf16(a3h[a], kf, tk[m][a]);
+          tk[m][a] = mfma_bf16(a3l[a], kf, tk[m][a]);
+        }
+      }
+    }
+    if (wave == 0) {  // dc -> dg = reverse cumulative sum within the chunk
+      const int t = lane;
+      float dct = pcc[t] + pcc[BC + t], dbt = pcb[t] + pcb[BC + t], dgam = 0.f, de = 0.f, gc = 0.f;
+#pragma unroll
+      for (int m = 0; m < COLS; ++m) {
+        dct += prc[m * BC + t];
+        dbt += prb[m * BC + t];
+        dgam += pdg[m * BC + t];
+        de += pde[m * BC + t];
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) gc += sred[w];
+      float dcv = dct + dgam * sgam[t] - de * se[t];
+      const float tail = wave_sum(de * se[t]);
+      if (t == BC - 1) dcv += tail + gc * sgam[BC - 1];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float y = __shfl_down(dcv, off, 64);
+        if (lane + off < 64) dcv += y;
+      }
+      if (t0 + t < seq.len) {
+        const long o = (seq.bos + t0 + t) * p.Hv + h;
+        p.dg[o] = dcv;
+        store_elem(p.dbeta, o, p.beta_dtype, dbt);
+      }
+    }
+  }
+  // dq, dk: summed over the key head's value heads, or (one head a workgroup
+  // of several) per value head in float32 for the reduction kernel
+  const bool direct = heads == group;
+  const int h0 = blockIdx.y * heads, c = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rp = wave & 1, cp = wave >> 1;
+#pragma unroll
+  for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = t0 + 32 * rp + 16 * a + 4 * g4 + e, kk = 16 * (KTW * cp + m) + c;
+        if (t >= seq.len) continue;
+        if (direct) {
+          const long o = ((seq.bos + t) * p.Hk + h0 / group) * K + kk;
+          store_el<u16>(p.dq, o, tq[m][a][e]);
+          store_el<u16>(p.dk, o, tk[m][a][e]);
+        } else {
+          const long o = ((seq.bos + t) * p.Hv + h0) * K + kk;
+          p.ws_dq[o] = tq[m][a][e];
+          p.ws_dk[o] = tk[m][a][e];
+        }
+      }
+    }
+  }
+}

@@ -375,38 +375,58 @@ def chunk_bwd(q, k, v, g, beta, scale: float, h0, do, dht=None):
     (gated_deltanet.py:230-277). Returns (dq, dk [B,T,Hk,K], dv [B,T,Hv,V] in
     q's dtype, dg [B,T,Hv] float32, dbeta in beta's operand dtype, dh0
     [B,Hv,K,V] float32)."""
+    return _chunk_bwd(q, k, v, g, beta, scale, h0, None, do, dht)
+
+
+def _chunk_bwd(q, k, v, g, beta, scale: float, h0, cu_seqlens, do, dht):
+    """chunk_bwd, or with cu_seqlens [N+1] the same for N packed sequences
+    (pbgdn_chunk_bwd_packed; h0, dht and dh0 [N,Hv,K,V])."""
     batch, length, hk, hv, dk, dv = _shapes(q, k, v, g, beta)
-    dev = _require_device(q, k, v, g, beta, h0, do, dht)
+    dev = _require_device(q, k, v, g, beta, h0, cu_seqlens, do, dht)
     if dk not in BACKWARD_HEAD_DIMS or dv not in BACKWARD_HEAD_DIMS:
         raise ValueError(f"chunk backward supports K and V in {BACKWARD_HEAD_DIMS}")
     q, k, v, g, beta = _operands(q, k, v, g, beta)
     if do.shape != (batch, length, hv, dv):
         raise ValueError(f"grad of o must be [B,T,Hv,V] = {(batch, length, hv, dv)}")
     do = _aligned(do.to(q.dtype).contiguous(), 16)  # the reference passes grad_o.to(q.dtype) (:272)
-    state_shape = (batch, hv, dk, dv)
+    nseq = batch
+    if cu_seqlens is not None:
+        if batch != 1:
+            raise ValueError("cu_seqlens needs B == 1 (sequences packed along T)")
+        cu_seqlens = cu_seqlens.to(torch.int32).contiguous()
+        nseq = cu_seqlens.numel() - 1
+    state_shape = (nseq, hv, dk, dv)
     if h0 is not None:
         if h0.shape != state_shape:
-            raise ValueError(f"initial state must be [B,Hv,K,V] = {state_shape}")
-        h0 = h0.to(torch.float32).contiguous()
+            raise ValueError(f"initial state must be [N,Hv,K,V] = {state_shape}")
+        h0 = _aligned(h0.to(torch.float32).contiguous(), 16)
     if dht is not None:
         if dht.shape != state_shape:
-            raise ValueError(f"grad of the final state must be [B,Hv,K,V] = {state_shape}")
-        dht = dht.to(torch.float32).contiguous()
+            raise ValueError(f"grad of the final state must be [N,Hv,K,V] = {state_shape}")
+        dht = _aligned(dht.to(torch.float32).contiguous(), 16)
     dq, dk_ = torch.empty_like(q), torch.empty_like(k)
     dv_ = torch.empty_like(v)
     dg = torch.empty(batch, length, hv, dtype=torch.float32, device=dev)
     dbeta = torch.empty_like(beta)
     dh0 = torch.empty(state_shape, dtype=torch.float32, device=dev)
     lib = _lib.lib()
-    ws_bytes = lib.pbgdn_chunk_bwd_workspace_size(batch, length, hk, hv, dk, dv)
-    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     codes = _lib.DTYPE_CODES
-    status = lib.pbgdn_chunk_bwd(
-        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), codes[q.dtype], _lib.ptr(g), _lib.ptr(beta), codes[beta.dtype],
-        _lib.ptr(h0), _lib.ptr(do), codes[do.dtype], _lib.ptr(dht), _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_),
-        _lib.ptr(dg), _lib.ptr(dbeta), _lib.ptr(dh0), _lib.ptr(workspace), ws_bytes, batch, length, hk, hv, dk, dv,
-        float(scale), _lib.stream_handle(dev))
-    _lib.check(status, "pbgdn_chunk_bwd")
+    tensors = (_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), codes[q.dtype], _lib.ptr(g), _lib.ptr(beta), codes[beta.dtype],
+               _lib.ptr(h0))
+    grads = (_lib.ptr(do), codes[do.dtype], _lib.ptr(dht), _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_), _lib.ptr(dg),
+             _lib.ptr(dbeta), _lib.ptr(dh0))
+    sizes = (length, hk, hv, dk, dv, float(scale), _lib.stream_handle(dev))
+    if cu_seqlens is None:
+        ws_bytes = lib.pbgdn_chunk_bwd_workspace_size(batch, length, hk, hv, dk, dv)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        status = lib.pbgdn_chunk_bwd(*tensors, *grads, _lib.ptr(workspace), ws_bytes, batch, *sizes)
+        _lib.check(status, "pbgdn_chunk_bwd")
+    else:
+        ws_bytes = lib.pbgdn_chunk_bwd_packed_workspace_size(length, nseq, hk, hv, dk, dv)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        status = lib.pbgdn_chunk_bwd_packed(*tensors, _lib.ptr(cu_seqlens), nseq, *grads, _lib.ptr(workspace), ws_bytes,
+                                            *sizes)
+        _lib.check(status, "pbgdn_chunk_bwd_packed")
     return dq, dk_, dv_, dg, dbeta, dh0
 
 
@@ -450,43 +470,66 @@ def _(q, k, v, g, beta, h0, grad_o, grad_final, scale):
             q.new_empty(batch, hv, dk, dv, dtype=torch.float32))
 
 
+@torch.library.custom_op("pbgdn::gated_delta_chunk_packed_backward", mutates_args=(),
+                         schema="(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor? h0, "
+                                "Tensor cu_seqlens, Tensor grad_o, Tensor? grad_final, float scale) "
+                                "-> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)")
+def gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
+    """gated_delta_chunk_backward of packed sequences (cu_seqlens [N+1]; h0,
+    grad_final and dh0 [N,Hv,K,V]): one call for all of them, and cu_seqlens
+    is read on the device only."""
+    return _chunk_bwd(q, k, v, g, beta, scale, h0, cu_seqlens, grad_o, grad_final)
+
+
+@gated_delta_chunk_packed_backward.register_fake
+def _(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
+    beta_dtype = beta.dtype if beta.dtype in (torch.float32, q.dtype) else torch.float32
+    return (torch.empty_like(q), q.new_empty(k.shape), q.new_empty(v.shape),
+            g.new_empty(g.shape, dtype=torch.float32), beta.new_empty(beta.shape, dtype=beta_dtype),
+            q.new_empty(cu_seqlens.shape[0] - 1, v.shape[2], q.shape[3], v.shape[3], dtype=torch.float32))
+
+
+# Workspace up to which a packed backward runs as one call (about 118,000
+# tokens of 32 heads of 128 x 128; all sequences' records live at once there).
+PACKED_BWD_WORKSPACE = 16 << 30
+
+
+def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
+    """The backward of a packed call: one launch set for all sequences; where
+    their workspace would pass PACKED_BWD_WORKSPACE, groups of consecutive
+    sequences that stay within it (a longer sequence alone), so that the
+    memory a call needs does not grow with the number of sequences."""
+    total, nseq = q.shape[1], cu_seqlens.shape[0] - 1
+    size = lambda tokens, n: _lib.lib().pbgdn_chunk_bwd_packed_workspace_size(  # noqa: E731
+        tokens, n, q.shape[2], v.shape[2], q.shape[3], v.shape[3])
+    if nseq <= 1 or size(total, nseq) <= PACKED_BWD_WORKSPACE:
+        return gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale)
+    bounds = [min(max(int(x), 0), total) for x in cu_seqlens.tolist()]
+    groups, first = [], 0
+    for n in range(1, nseq + 1):
+        if n == nseq or size(max(bounds[n + 1] - bounds[first], 0), n + 1 - first) > PACKED_BWD_WORKSPACE:
+            groups.append((first, n))
+            first = n
+    parts = []
+    for a, b in groups:
+        lo, hi = (0 if a == 0 else bounds[a]), (total if b == nseq else max(bounds[a], bounds[b]))
+        sl = slice(lo, hi)
+        parts.append(gated_delta_chunk_packed_backward(
+            q[:, sl], k[:, sl], v[:, sl], g[:, sl], beta[:, sl], None if h0 is None else h0[a:b],
+            cu_seqlens[a:b + 1] - lo, grad_o[:, sl], None if grad_final is None else grad_final[a:b], scale))
+    return tuple(torch.cat([p[j] for p in parts], 1 if j < 5 else 0) for j in range(6))
+
+
 def _chunk_setup(ctx, inputs, output):
     q, k, v, g, beta, h0, cu_seqlens, scale = inputs
     ctx.save_for_backward(q, k, v, g, beta, h0, cu_seqlens)
     ctx.scale = scale
 
 
-def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
-    """The backward of a packed call ([1, sum T] with cu_seqlens): each
-    sequence's slice through the batched backward (its own h0 and final-state
-    gradient), the gradients written back into the packed layout. An empty
-    sequence's final state is its h0, so its dh0 is its final-state gradient."""
-    bounds = [min(max(int(x), 0), q.shape[1]) for x in cu_seqlens.tolist()]
-    nseq = len(bounds) - 1
-    dq, dk, dv = torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
-    dg = torch.zeros(g.shape, dtype=torch.float32, device=g.device)
-    dbeta = torch.zeros(beta.shape, dtype=beta.dtype if beta.dtype in (torch.float32, q.dtype) else torch.float32,
-                        device=beta.device)
-    dh0 = torch.zeros(nseq, v.shape[2], q.shape[3], v.shape[3], dtype=torch.float32, device=q.device)
-    for n in range(nseq):
-        lo, hi = bounds[n], max(bounds[n], bounds[n + 1])
-        if hi == lo:
-            if grad_final is not None:
-                dh0[n] = grad_final[n]
-            continue
-        sl = slice(lo, hi)
-        r = gated_delta_chunk_backward(q[:, sl], k[:, sl], v[:, sl], g[:, sl], beta[:, sl],
-                                       None if h0 is None else h0[n:n + 1], grad_o[:, sl],
-                                       None if grad_final is None else grad_final[n:n + 1], scale)
-        dq[:, sl], dk[:, sl], dv[:, sl], dg[:, sl], dbeta[:, sl] = r[0], r[1], r[2], r[3], r[4]
-        dh0[n] = r[5][0]
-    return dq, dk, dv, dg, dbeta, dh0
-
-
 def _chunk_grad(ctx, grad_o, grad_final):
     """The reference's _fla_grad (gated_deltanet.py:266-275): zeros for a
     missing output gradient, each gradient in its input's dtype. A packed call
-    (cu_seqlens) takes the batched backward sequence by sequence."""
+    (cu_seqlens) takes the packed backward."""
     q, k, v, g, beta, h0, cu_seqlens = ctx.saved_tensors
     if grad_o is None:
         grad_o = torch.zeros(*q.shape[:2], v.shape[2], v.shape[3], dtype=q.dtype, device=q.device)

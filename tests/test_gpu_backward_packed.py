@@ -1,0 +1,62 @@
+"""The packed backward (pbgdn_chunk_bwd_packed) against the batched backward of
+each sequence alone: the same kernels on the same rows, so bit for bit, in
+every head width and dtype; rows that belong to no sequence get zeros, an empty
+sequence's dh0 is its final gradient, and a call split into groups of sequences
+(its workspace bounded) returns what one call returns."""
+import pytest
+import torch
+
+from pseudobrain_amd import gated_deltanet as gd
+from pseudobrain_amd.workloads import generate
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def make(bounds, total, hk, hv, dk, dv, dtype, seed):
+    nseq = len(bounds) - 1
+    q, k, v, g, beta, h0 = (x.to(DEV) for x in generate(1, total, hk, hv, dk, dv, dtype, 0.05, seed=seed, nstates=nseq))
+    gen = torch.Generator().manual_seed(seed)
+    do = (torch.randn(1, total, hv, dv, generator=gen) * 0.1).to(dtype).to(DEV)
+    dht = (torch.randn(nseq, hv, dk, dv, generator=gen) * 0.1).to(DEV)
+    return q, k, v, g, beta, h0, do, dht, torch.tensor(bounds, dtype=torch.int32, device=DEV)
+
+
+def packed(q, k, v, g, beta, h0, do, dht, cu, scale=0.1):
+    return torch.ops.pbgdn.gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu, do, dht, scale)
+
+
+@pytest.mark.parametrize("bounds,total,hk,hv,dk,dv,dtype", [
+    ([0, 1, 1, 64, 129, 300], 300, 1, 2, 128, 128, torch.bfloat16),     # 1-token, empty, 63-, 65- and 171-token
+    ([3, 70, 198], 211, 2, 2, 64, 128, torch.bfloat16),                 # rows before and after every sequence
+    ([0, 64, 128, 192], 192, 1, 3, 128, 64, torch.bfloat16),            # whole chunks
+    (list(range(0, 71 * 9, 9)), 70 * 9, 1, 1, 64, 64, torch.bfloat16),  # 70 sequences: past one wave's count
+    ([0, 100, 100, 250], 260, 2, 4, 64, 64, torch.float16),
+    ([5, 40, 170], 171, 1, 2, 128, 128, torch.float32),
+])
+def test_packed_equals_each_sequence_alone(bounds, total, hk, hv, dk, dv, dtype):
+    print(f"[{bounds[:6]} {hk}->{hv} K={dk} V={dv} {dtype}]", flush=True)
+    q, k, v, g, beta, h0, do, dht, cu = make(bounds, total, hk, hv, dk, dv, dtype, seed=len(bounds))
+    got = packed(q, k, v, g, beta, h0, do, dht, cu)
+    for n, (lo, hi) in enumerate(zip(bounds, bounds[1:])):
+        sl = slice(lo, hi)
+        if hi == lo:
+            assert torch.equal(got[5][n], dht[n])
+            continue
+        ref = gd.chunk_bwd(*(x[:, sl] for x in (q, k, v, g, beta)), 0.1, h0[n:n + 1], do[:, sl], dht[n:n + 1])
+        for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta"), got, ref):
+            assert torch.equal(a[:, sl], b), f"{name} of sequence {n}"
+        assert torch.equal(got[5][n], ref[5][0]), f"dh0 of sequence {n}"
+    for a in got[:5]:
+        assert not a[:, :bounds[0]].any() and not a[:, bounds[-1]:].any()
+
+
+def test_groups_of_sequences_equal_one_call(monkeypatch):
+    bounds = [2, 90, 90, 300, 301, 420]
+    args = make(bounds, 450, 1, 2, 64, 64, torch.bfloat16, seed=4)
+    q, k, v, g, beta, h0, do, dht, cu = args
+    want = packed(*args)
+    monkeypatch.setattr(gd, "PACKED_BWD_WORKSPACE", 1 << 20)
+    got = gd._packed_backward(q, k, v, g, beta, h0, cu, do, dht, 0.1)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and torch.equal(a, b)
