@@ -24,7 +24,7 @@ namespace {
 
 // The scan kernel of a call. The wide scan (chunk_wide.hip: all 128 columns
 // of a (sequence, value head) per workgroup, one wave per 16-column tile)
-// takes 16-bit inputs and outputs at K = 128 with V a multiple of 128. It
+// takes 16-bit inputs at K = 128 with V a multiple of 128. It
 // stages each chunk once for eight tiles, so it wins whenever its workgroups
 // number at least half the CUs (measured at the Qwen3-Next head shape, 32,768
 // tokens: 4 x 8,192 0.53 vs 0.72 ms, 8 x 4,096 0.39 vs 0.73 ms, 1024 x 32
@@ -56,7 +56,9 @@ int run_chunk(const ChunkParams &p, long records, int out_dtype, hipStream_t s) 
   const int st = launch_prep<K, TIn>(p, records, s);
   if (st != PBGDN_OK) return st;
   if constexpr (K == 128 && sizeof(TIn) == 2) {
-    if (out_dtype != PBGDN_F32 && wide_eligible<K, TIn>(p)) return launch_wide<K, TIn, TIn, false>(p, s);
+    if (wide_eligible<K, TIn>(p)) {
+      return out_dtype == PBGDN_F32 ? launch_wide<K, TIn, float, false>(p, s) : launch_wide<K, TIn, TIn, false>(p, s);
+    }
   }
   if (out_dtype == PBGDN_F32) return launch_scan<K, TIn, float>(p, s);
   return launch_scan<K, TIn, TIn>(p, s);  // out_dtype == in_dtype, checked by the caller

@@ -30,7 +30,9 @@
 // update's K^T reads and the state's loads and stores follow the same map.
 // O is formed transposed (O^T = (Q S)^T diag(scale gamma) + U^T QKD^T: the
 // same registers with the MFMA operands swapped), so a lane holds 4
-// contiguous columns of a token row and stores them as one 8-byte piece.
+// contiguous columns of a token row and stores them as one piece of 8 bytes
+// (16 for float32, whose o costs no more than a 16-bit one: the step is not
+// bound by its stores).
 //
 // Staging. A chunk's K and Q rows (16-bit, 256 bytes at K = 128), its record
 // and its V rows (128 columns) are copied HBM -> LDS by direct-to-LDS buffer
@@ -140,7 +142,7 @@ struct WideBlock {
   static_assert(K == 128, "the wide scan is built for K = 128");
   static_assert(REC_BYTES % 1024 == 0 && DMA_KQ % WT == 0 && DMA_V % WT == 0, "whole DMA instructions per wave");
   static_assert(sizeof(TIn) == 2, "16-bit inputs (staged as they are)");
-  static_assert(sizeof(TOut) == 2 || (EPI && sizeof(TOut) == 4), "16-bit o; hs also in float32");
+  static_assert(sizeof(TOut) == 2 || sizeof(TOut) == 4, "o or hs in the input type or in float32");
   static constexpr int GATE_LOADS = EPI ? 4 : 0;  // gate loads a wave issues per chunk, at its start
   static_assert(L::BYTES <= 160 * 1024, "LDS");
 
@@ -662,6 +664,8 @@ int launch_wide(const ChunkParams &p, hipStream_t stream) {
 
 template int launch_wide<128, u16, u16, false>(const ChunkParams &, hipStream_t);
 template int launch_wide<128, half_t, half_t, false>(const ChunkParams &, hipStream_t);
+template int launch_wide<128, u16, float, false>(const ChunkParams &, hipStream_t);
+template int launch_wide<128, half_t, float, false>(const ChunkParams &, hipStream_t);
 template int launch_wide<128, u16, u16, true>(const ChunkParams &, hipStream_t);
 template int launch_wide<128, u16, float, true>(const ChunkParams &, hipStream_t);
 template int launch_wide<128, half_t, half_t, true>(const ChunkParams &, hipStream_t);

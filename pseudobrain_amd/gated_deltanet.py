@@ -451,6 +451,25 @@ def _(q, k, v, g, beta, h0, cu_seqlens, scale):
             q.new_empty(nseq, hv, dk, dv, dtype=torch.float32))
 
 
+@torch.library.custom_op("pbgdn::gated_delta_chunk_f32", mutates_args=(),
+                         schema="(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor? h0, "
+                                "Tensor? cu_seqlens, float scale) -> (Tensor, Tensor)")
+def gated_delta_chunk_f32(q, k, v, g, beta, h0, cu_seqlens, scale):
+    """gated_delta_chunk with o in float32, written by the scan kernel itself:
+    widening a 16-bit o afterwards took 120 us of 860 at 32,768 tokens of 32
+    heads of 128, and the scan's own time does not change."""
+    return _chunk_fwd(q, k, v, g, beta, scale, h0, cu_seqlens, out_dtype=torch.float32)
+
+
+@gated_delta_chunk_f32.register_fake
+def _(q, k, v, g, beta, h0, cu_seqlens, scale):
+    batch, length, _, dk = q.shape
+    hv, dv = v.shape[2], v.shape[3]
+    nseq = batch if cu_seqlens is None else cu_seqlens.shape[0] - 1
+    return (q.new_empty(batch, length, hv, dv, dtype=torch.float32),
+            q.new_empty(nseq, hv, dk, dv, dtype=torch.float32))
+
+
 @torch.library.custom_op("pbgdn::gated_delta_chunk_backward", mutates_args=(),
                          schema="(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor? h0, "
                                 "Tensor grad_o, Tensor? grad_final, float scale) "
@@ -544,6 +563,7 @@ def _chunk_grad(ctx, grad_o, grad_final):
 
 
 gated_delta_chunk.register_autograd(_chunk_grad, setup_context=_chunk_setup)
+gated_delta_chunk_f32.register_autograd(_chunk_grad, setup_context=_chunk_setup)
 
 
 def chunk_residuals(k, g, beta, *, a_dtype: torch.dtype | None = None):
@@ -713,7 +733,7 @@ def delta_rule_hip(q, k, v, g, beta, scale, h0, cu_seqlens=None):
     """The device prefill with the fla path's conventions (gated_deltanet.py:280-285):
     q/k/v at their own precision, fp32 state and decay; returns (o.float(), final).
 
-    The chunk kernels through pbgdn::gated_delta_chunk, the head widths
+    The chunk kernels through pbgdn::gated_delta_chunk_f32, the head widths
     zero-padded to theirs: K <= 128 for every input dtype (differentiable for
     [B,T] batches with K, V <= 128), and 128 < K <= 256 for bfloat16 and
     float16 inputs (K padded to 256, no backward). float32 inputs with
@@ -729,11 +749,13 @@ def delta_rule_hip(q, k, v, g, beta, scale, h0, cu_seqlens=None):
     if dk > CHUNK_HEAD_DIMS[-2] and q.dtype not in (torch.bfloat16, torch.float16):
         return _recurrent_prefill(q, k, v, g, beta, scale, h0, cu_seqlens)
     kp, vp = _chunk_widths(dk, dv, grad)
-    o, final = gated_delta_chunk(_pad_last(q, kp), _pad_last(k, kp), _pad_last(v, vp), g, beta,
-                                 _pad_state(h0, kp, vp), cu_seqlens, float(scale))
+    o, final = gated_delta_chunk_f32(_pad_last(q, kp), _pad_last(k, kp), _pad_last(v, vp), g, beta,
+                                     _pad_state(h0, kp, vp), cu_seqlens, float(scale))
     if (kp, vp) != (dk, dv):
         o, final = o[..., :dv], final[..., :dk, :dv].contiguous()
-    return o.float(), final
+        if q.dtype != torch.float32:
+            o = o.contiguous()
+    return o, final
 
 
 def _recurrent_prefill(q, k, v, g, beta, scale, h0, cu_seqlens):
