@@ -24,6 +24,9 @@
 //   bwd_grad_kernel      per (chunk, value head): dq, dk, dv, dbeta, dg
 //   bwd_gqa_reduce_kernel  dq, dk summed over the value heads of a key head
 //
+// bf16 inputs have kernels of their own for the first three
+// (chunk_bwd_scan.hpp, chunk_bwd_bf16.hpp).
+//
 // Accumulation is float32. With bf16 inputs the products of inputs and states
 // run on bf16 MFMA, a float32 operand entering as a high/low pair of bf16
 // parts (A B_hi + A B_lo, or three products when both are paired: about
@@ -57,7 +60,10 @@ struct BwdParams {
   float *dg;
   void *dbeta;
   float *dh0;
-  float *ws_T, *ws_c, *ws_beta, *ws_dU0, *ws_J, *ws_S, *ws_dS, *ws_dq, *ws_dk;
+  // ws_T: T, 64 x 64 a record in float32 (bf16 inputs: as a bf16 pair, the
+  // high halves' rows, then the low ones); ws_M (bf16 inputs, in ws_dU0's
+  // bytes): M^T, a pair like it
+  float *ws_T, *ws_c, *ws_beta, *ws_dU0, *ws_M, *ws_J, *ws_S, *ws_dS, *ws_dq, *ws_dk;
   const int32_t *cu_seqlens;  // [num_seqs + 1] bounds of packed sequences (B = 1), or NULL: B rows of T tokens
   int num_seqs;               // sequences: B without cu_seqlens
   int records;                // chunk records (times Hv: records of the workspace)
@@ -534,6 +540,50 @@ __device__ __forceinline__ void zero_uncovered(const BwdParams &p, int x, int h)
   }
 }
 
+// T = (I + A)^-1 (unit lower triangular) in place over A (rows of LC floats),
+// by 16 x 16 blocks; sr: 3 x 256 floats. Four waves; ends with a barrier.
+__device__ __forceinline__ void invert_unit_lower(float *sa, float *sr) {
+  const int lane = threadIdx.x & 63, c = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Wave w inverts diagonal block w by forward substitution: lane
+  // (column j, part) sums the terms s = part mod 4 of
+  // T[t][j] = -sum_{s<t} A[t][s] T[s][j] (T is zero above the diagonal, A
+  // too), and two shuffles add the parts; every lane reads row t before it is
+  // written (one wave, one instruction stream).
+  {
+    const int j = lane & 15, part = lane >> 4, base = 16 * wave;
+    for (int t = 0; t < 16; ++t) {
+      float acc = 0.f;
+      for (int s2 = part; s2 < t; s2 += 4) acc += sa[(base + t) * LC + base + s2] * sa[(base + s2) * LC + base + j];
+      acc += __shfl_xor(acc, 16, 64);
+      acc += __shfl_xor(acc, 32, 64);
+      if (part == 0) sa[(base + t) * LC + base + j] = t == j ? 1.f : (t < j ? 0.f : -acc);
+    }
+  }
+  __syncthreads();
+  // Off-diagonal blocks, one block row at a time:
+  // T_ij = -T_ii sum_{k=j}^{i-1} A_ik T_kj, wave j forming block (i, j).
+  for (int bi = 1; bi < 4; ++bi) {
+    if (wave < bi) {
+      float4_t racc = zero4();
+      for (int bk = wave; bk < bi; ++bk) {
+        racc = tile_mm<16>(racc, [&](int r, int kk) { return sa[(16 * bi + r) * LC + 16 * bk + kk]; },
+                           [&](int kk, int col) { return sa[(16 * bk + kk) * LC + 16 * wave + col]; });
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sr[wave * 256 + (4 * g4 + r) * 16 + c] = racc[r];
+    }
+    __syncthreads();  // block row bi of A is read by every wave before any T of it is written
+    if (wave < bi) {
+      const float4_t tacc = tile_mm<16>(zero4(), [&](int r, int kk) { return sa[(16 * bi + r) * LC + 16 * bi + kk]; },
+                                        [&](int kk, int col) { return sr[wave * 256 + kk * 16 + col]; });
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sa[(16 * bi + 4 * g4 + r) * LC + 16 * wave + c] = -tacc[r];
+    }
+    __syncthreads();
+  }
+}
+
 template <int K, int V, typename TIn>
 __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   constexpr int PADE = 16 / sizeof(TIn), LK = K + PADE, LV = V + PADE;
@@ -543,11 +593,6 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   TIn *sq = reinterpret_cast<TIn *>(lds), *sk = sq + BC * LK, *sdo = sk + BC * LK;
   float *sa = reinterpret_cast<float *>(sdo + BC * LV);
   float *sc = sa + BC * LC, *sgam = sc + BC, *sbeta = sgam + BC, *sr = sbeta + BC;
-  // bf16 inputs: M as a bf16 high/low pair (rows of LM) in sa's bytes, and
-  // dU0, J on bf16 MFMA
-  constexpr bool BF = std::is_same<TIn, u16>::value;
-  constexpr int LM = LC;
-  u16 *mh = reinterpret_cast<u16 *>(sa);
   const int h = blockIdx.y;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
@@ -585,13 +630,8 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   auto krow = [&](int kk, int j, int tc) { return ld4e(sk, (16 * tc + j) * LK + kk); };
   // A = strict_lower(beta_t (K K^T) o D), rows 16w .. of this wave
   for (int tc = 0; tc < 4; ++tc) {
-    float4_t kk_acc;
-    if constexpr (std::is_same<TIn, u16>::value) {
-      kk_acc = rows_times_rows<K>(sk, sk, LK, 16 * wave, 16 * tc);
-    } else {
-      kk_acc = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sk, (16 * wave + r) * LK + kk); },
-                           [&](int kk, int j) { return krow(kk, j, tc); });
-    }
+    const float4_t kk_acc = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sk, (16 * wave + r) * LK + kk); },
+                                        [&](int kk, int j) { return krow(kk, j, tc); });
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * wave + 4 * g4 + r, s2 = 16 * tc + c;
@@ -599,86 +639,23 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
     }
   }
   __syncthreads();
-  // T = (I + A)^-1 (unit lower triangular) in place over A, by 16 x 16
-  // blocks. Wave w inverts diagonal block w by forward substitution: lane
-  // (column j, part) sums the terms s = part mod 4 of
-  // T[t][j] = -sum_{s<t} A[t][s] T[s][j] (T is zero above the diagonal, A
-  // too), and two shuffles add the parts; every lane reads row t before it is
-  // written (one wave, one instruction stream).
-  {
-    const int j = lane & 15, part = lane >> 4, base = 16 * wave;
-    for (int t = 0; t < 16; ++t) {
-      float acc = 0.f;
-      for (int s2 = part; s2 < t; s2 += 4) acc += sa[(base + t) * LC + base + s2] * sa[(base + s2) * LC + base + j];
-      acc += __shfl_xor(acc, 16, 64);
-      acc += __shfl_xor(acc, 32, 64);
-      if (part == 0) sa[(base + t) * LC + base + j] = t == j ? 1.f : (t < j ? 0.f : -acc);
-    }
-  }
-  __syncthreads();
-  // Off-diagonal blocks, one block row at a time:
-  // T_ij = -T_ii sum_{k=j}^{i-1} A_ik T_kj, wave j forming block (i, j).
-  for (int bi = 1; bi < 4; ++bi) {
-    if (wave < bi) {
-      float4_t racc = zero4();
-      for (int bk = wave; bk < bi; ++bk) {
-        racc = tile_mm<16>(racc, [&](int r, int kk) { return sa[(16 * bi + r) * LC + 16 * bk + kk]; },
-                           [&](int kk, int col) { return sa[(16 * bk + kk) * LC + 16 * wave + col]; });
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sr[wave * 256 + (4 * g4 + r) * 16 + c] = racc[r];
-    }
-    __syncthreads();  // block row bi of A is read by every wave before any T of it is written
-    if (wave < bi) {
-      const float4_t tacc = tile_mm<16>(zero4(), [&](int r, int kk) { return sa[(16 * bi + r) * LC + 16 * bi + kk]; },
-                                        [&](int kk, int col) { return sr[wave * 256 + kk * 16 + col]; });
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sa[(16 * bi + 4 * g4 + r) * LC + 16 * wave + c] = -tacc[r];
-    }
-    __syncthreads();
-  }
+  invert_unit_lower(sa, sr);
   float *wt = p.ws_T + rec(p, seq, h, i) * BC * BC;
   for (int e = tid; e < BC * BC; e += BNT) wt[e] = sa[(e / BC) * LC + e % BC];
   __syncthreads();  // T is out: M = scale (Q K^T) o D takes its place
   for (int tc = 0; tc < 4; ++tc) {
-    float4_t qk_acc;
-    if constexpr (std::is_same<TIn, u16>::value) {
-      qk_acc = rows_times_rows<K>(sq, sk, LK, 16 * wave, 16 * tc);
-    } else {
-      qk_acc = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sq, (16 * wave + r) * LK + kk); },
-                           [&](int kk, int j) { return krow(kk, j, tc); });
-    }
+    const float4_t qk_acc = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sq, (16 * wave + r) * LK + kk); },
+                                        [&](int kk, int j) { return krow(kk, j, tc); });
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * wave + 4 * g4 + r, s2 = 16 * tc + c;
-      const float mv = t >= s2 ? p.scale * qk_acc[r] * expf(sc[t] - sc[s2]) : 0.f;
-      if constexpr (BF) {  // M as a bf16 high/low pair, rows of LM, in sa's bytes
-        const u16 hi = bf16_bits(mv);
-        mh[t * LM + s2] = hi;
-        mh[BC * LM + t * LM + s2] = bf16_bits(mv - __uint_as_float(static_cast<uint32_t>(hi) << 16));
-      } else {
-        sa[t * LC + s2] = mv;
-      }
+      sa[t * LC + s2] = t >= s2 ? p.scale * qk_acc[r] * expf(sc[t] - sc[s2]) : 0.f;
     }
   }
   __syncthreads();
   // dU0 = M^T dO: tiles (row tile, 16-column tile)
   float *wu = p.ws_dU0 + rec(p, seq, h, i) * BC * V;
-  if constexpr (BF) {  // M^T fragments and dO's columns by transposing reads
-    for (int tile = wave; tile < 4 * (V / 16); tile += 4) {
-      const int tr = tile & 3, tv = tile >> 2;
-      float4_t acc = zero4();
-#pragma unroll
-      for (int ts = 0; ts < BC; ts += 32) {
-        const bh8_t d = tr_frag(sdo, LV, ts, 16 * tv);
-        acc = mfma_bf16(tr_frag(mh, LM, ts, 16 * tr), d, acc);
-        acc = mfma_bf16(tr_frag(mh + BC * LM, LM, ts, 16 * tr), d, acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) wu[(16 * tr + 4 * g4 + r) * V + 16 * tv + c] = acc[r];
-    }
-  }
-  for (int tile = wave; tile < (BF ? 0 : 4 * (V / 16)); tile += 4) {
+  for (int tile = wave; tile < 4 * (V / 16); tile += 4) {
     const int tr = tile & 3, tv = tile >> 2;
     const float4_t acc = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4s(&sa[s2 * LC + 16 * tr + r], LC); },
                                       [&](int s2, int col) {
@@ -691,39 +668,7 @@ __global__ __launch_bounds__(BNT) void bwd_local_kernel(BwdParams p) {
   }
   // J = scale (Gamma Q)^T dO: K x V
   float *wj = p.ws_J + rec(p, seq, h, i) * static_cast<long>(K) * V;
-  if constexpr (BF) {
-    // per column tile of this wave: (Gamma dO)'s columns as bf16 pairs once,
-    // then every key tile's Q^T fragments (transposing reads of the q rows)
-    for (int tv = wave; tv < V / 16; tv += 4) {
-      bh8_t bh[2], bl[2];
-#pragma unroll
-      for (int s8 = 0; s8 < 2; ++s8) {
-        const v4u32_t w = __builtin_bit_cast(v4u32_t, tr_frag(sdo, LV, 32 * s8, 16 * tv));
-        const float4_t g0 = ld4(&sgam[32 * s8 + 8 * g4]), g1 = ld4(&sgam[32 * s8 + 8 * g4 + 4]);
-        const float4_t x0 = float4_t{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u),
-                                     __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u)} * g0;
-        const float4_t x1 = float4_t{__uint_as_float(w[2] << 16), __uint_as_float(w[2] & 0xffff0000u),
-                                     __uint_as_float(w[3] << 16), __uint_as_float(w[3] & 0xffff0000u)} * g1;
-        v2u32_t h0, l0, h1, l1;
-        split_bf16(x0, h0, l0);
-        split_bf16(x1, h1, l1);
-        bh[s8] = __builtin_bit_cast(bh8_t, v4u32_t{h0[0], h0[1], h1[0], h1[1]});
-        bl[s8] = __builtin_bit_cast(bh8_t, v4u32_t{l0[0], l0[1], l1[0], l1[1]});
-      }
-      for (int tk = 0; tk < K / 16; ++tk) {
-        float4_t acc = zero4();
-#pragma unroll
-        for (int s8 = 0; s8 < 2; ++s8) {
-          const bh8_t a = tr_frag(sq, LK, 32 * s8, 16 * tk);
-          acc = mfma_bf16(a, bh[s8], acc);
-          acc = mfma_bf16(a, bl[s8], acc);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wj[(16 * tk + 4 * g4 + r) * V + 16 * tv + c] = p.scale * acc[r];
-      }
-    }
-  }
-  for (int tile = wave; tile < (BF ? 0 : (K / 16) * (V / 16)); tile += 4) {
+  for (int tile = wave; tile < (K / 16) * (V / 16); tile += 4) {
     const int tk = tile % (K / 16), tv = tile / (K / 16);
     const float4_t acc = tile_mm4<BC>(
         zero4(),
@@ -1725,6 +1670,7 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
 }
 
 #include "chunk_bwd_bf16.hpp"
+#include "chunk_bwd_scan.hpp"
 
 // dq, dk [B,T,Hk,K] = sum over the Hv/Hk value heads of each key head.
 __global__ __launch_bounds__(BNT) void bwd_gqa_reduce_kernel(BwdParams p) {
@@ -1791,6 +1737,21 @@ int launch_grad_bf16(const BwdParams &p, int heads, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? PBGDN_OK : PBGDN_ERR_LAUNCH;
 }
 
+template <int K, int NW>
+int launch_scans_bf16(const BwdParams &p, hipStream_t st) {
+  static_assert(Scan16<K, NW>::BYTES <= 160 * 1024, "LDS budget");
+  return launch(bwd_scans_bf16_kernel<K, NW>, dim3(p.V / (16 * NW) * p.Hv * 2 * p.num_seqs), Scan16<K, NW>::BYTES, st,
+                p, 128 * NW);
+}
+
+// The scans of bf16 inputs: 64 value columns a workgroup (four computing
+// waves) where that gives every CU a workgroup, else 32.
+template <int K>
+int run_scans_bf16(const BwdParams &p, hipStream_t st) {
+  const long wide = 2L * p.num_seqs * p.Hv * (p.V / 64);
+  return wide >= p.cus ? launch_scans_bf16<K, 4>(p, st) : launch_scans_bf16<K, 2>(p, st);
+}
+
 template <int K, int V>
 int run_backward(const BwdParams &p, hipStream_t st) {
   static_assert(grad_lds<K, float>() <= 160 * 1024 && grad_lds<K, u16>() <= 160 * 1024 && local_lds<K, V, float>() <= 160 * 1024, "LDS budget");
@@ -1799,14 +1760,14 @@ int run_backward(const BwdParams &p, hipStream_t st) {
   if (p.records > 0) {
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_local_kernel<K, V, float>, per_chunk, local_lds<K, V, float>(), st, p); break;
-      case PBGDN_BF16: rc = launch(bwd_local_kernel<K, V, u16>, per_chunk, local_lds<K, V, u16>(), st, p); break;
+      case PBGDN_BF16: rc = launch(bwd_local_bf16_kernel<K>, per_chunk, local_bf16_lds<K>(), st, p); break;
       default: rc = launch(bwd_local_kernel<K, V, half_t>, per_chunk, local_lds<K, V, half_t>(), st, p); break;
     }
   }
   if (rc == PBGDN_OK) {  // both scans in one launch (with T = 0 only the reverse one writes: dh0 = dht)
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_scans_kernel<K, float>, per_tile2, scan_lds<K, float>(), st, p); break;
-      case PBGDN_BF16: rc = launch(bwd_scans_kernel<K, u16>, per_tile2, scan_lds<K, u16>(), st, p); break;
+      case PBGDN_BF16: rc = run_scans_bf16<K>(p, st); break;
       default: rc = launch(bwd_scans_kernel<K, half_t>, per_tile2, scan_lds<K, half_t>(), st, p); break;
     }
   }
@@ -1912,6 +1873,7 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
   p.ws_c = p.ws_T + recs * BC * BC;
   p.ws_beta = p.ws_c + recs * BC;
   p.ws_dU0 = p.ws_beta + recs * BC;
+  p.ws_M = p.ws_dU0;
   p.ws_J = p.ws_dU0 + recs * BC * V;
   p.ws_S = p.ws_J + recs * K * V;
   p.ws_dS = p.ws_S + recs * K * V;

@@ -140,10 +140,10 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     u16 *mt = area, *sv = area + 2 * CC;
     {
       RawRows<u16, V, NT> rv, rd;
-      float4_t rt[BC * BC / 4 / NT];
+      uint4 rt[BC * BC / 4 / NT];  // T's pair: 1,024 pieces of 16 bytes
       rd.load(tid, p.dout, seq, t0, p.Hv, h, V);
       rv.load(tid, p.v, seq, t0, p.Hv, h, V);
-      const float4_t *wt = reinterpret_cast<const float4_t *>(p.ws_T + r * BC * BC);
+      const uint4 *wt = reinterpret_cast<const uint4 *>(p.ws_T + r * BC * BC);
 #pragma unroll
       for (int m = 0; m < BC * BC / 4 / NT; ++m) rt[m] = wt[tid + NT * m];
       const float cv = p.ws_c[r * BC + lane], bv = p.ws_beta[r * BC + lane], last = p.ws_c[r * BC + BC - 1];
@@ -160,10 +160,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
       for (int m = 0; m < BC * BC / 4 / NT; ++m) {
         const int e = tid + NT * m;
-        v2u32_t hi, lo;
-        split_bf16(rt[m], hi, lo);
-        *reinterpret_cast<v2u32_t *>(tp + (e >> 4) * LB + 4 * (e & 15)) = hi;
-        *reinterpret_cast<v2u32_t *>(tp + CC + (e >> 4) * LB + 4 * (e & 15)) = lo;
+        *reinterpret_cast<uint4 *>(tp + (e >> 3) * LB + 8 * (e & 7)) = rt[m];  // half e / 512, row (e / 8) & 63
       }
       if (tid < BC) {
         sc[tid] = cv;

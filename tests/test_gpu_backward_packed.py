@@ -60,3 +60,25 @@ def test_groups_of_sequences_equal_one_call(monkeypatch):
     got = gd._packed_backward(q, k, v, g, beta, h0, cu, do, dht, 0.1)
     for a, b in zip(got, want):
         assert a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dk,dv", [(128, 128), (64, 64), (128, 64)])
+def test_many_heads_equal_few(dk, dv):
+    """Scans of 64 value columns a workgroup (enough sequences and heads for
+    the device) against those of 32 (one sequence alone): the same sums, so bit
+    for bit, with chunks of one token and of 63."""
+    batch, heads = 8, 32
+    for length in (63, 129):
+        q, k, v, g, beta, h0 = (x.to(DEV) for x in generate(batch, length, heads, heads, dk, dv, torch.bfloat16, 0.05,
+                                                            seed=length))
+        gen = torch.Generator().manual_seed(length)
+        do = (torch.randn(batch, length, heads, dv, generator=gen) * 0.1).to(torch.bfloat16).to(DEV)
+        dht = (torch.randn(batch, heads, dk, dv, generator=gen) * 0.1).to(DEV)
+        got = gd.chunk_bwd(q, k, v, g, beta, 0.1, h0, do, dht)
+        for n in (0, batch - 1):
+            one = slice(n, n + 1)
+            ref = gd.chunk_bwd(*(x[one, :, :2] for x in (q, k, v, g, beta)), 0.1, h0[one, :2], do[one, :, :2],
+                               dht[one, :2])
+            for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta"), got, ref):
+                assert torch.equal(a[one, :, :2], b), f"{name} of row {n}, length {length}"
+            assert torch.equal(got[5][one, :2], ref[5])
