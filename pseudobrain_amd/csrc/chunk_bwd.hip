@@ -1741,7 +1741,7 @@ template <int K, int NW>
 int launch_scans_bf16(const BwdParams &p, hipStream_t st) {
   static_assert(Scan16<K, NW>::BYTES <= 160 * 1024, "LDS budget");
   return launch(bwd_scans_bf16_kernel<K, NW>, dim3(p.V / (16 * NW) * p.Hv * 2 * p.num_seqs), Scan16<K, NW>::BYTES, st,
-                p, 128 * NW);
+                p, Scan16<K, NW>::NT);
 }
 
 // The scans of bf16 inputs: 64 value columns a workgroup (four computing

@@ -7,9 +7,8 @@
 // NW waves compute, each 16 columns with the whole chain of a chunk in its
 // registers (an accumulator tile is the next product's B operand as it
 // stands, see chunk_bwd_bf16.hpp), so a step has no exchange between waves and
-// one barrier. NW more waves load: they hold the next chunk's rows in
-// registers, write them to the LDS buffer that the step before has left, and
-// start on the chunk after.
+// one barrier. Four more waves load: they hold the next two chunks' rows in
+// registers and write each to the LDS buffer that the step before has left.
 //
 //   state    X = V - Gamma K S,  U = T beta X,  S <- gamma_C S + K^T E U
 //   adjoint  dU = M^T dO + E K dS',  dX = beta T^T dU,
@@ -139,11 +138,12 @@ __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------
 template <int K, int NW>
 struct Scan16 {
-  static constexpr int NT = 128 * NW, LOADERS = 64 * NW;
+  static constexpr int LOADERS = 256, NT = 64 * NW + LOADERS;
   static constexpr int LK = K + 8, LB = BC + 8, LC16 = 16 * NW + 8;  // row strides (elements)
   static constexpr int PAIR = 2 * BC * LB;
-  // one buffer: K rows, the T pair, the V or dO columns, the vectors e^c,
-  // e^(c_last - c), beta; the adjoint's also Q rows and the M^T pair
+  // one buffer: K rows, the T pair, the V or dO columns, four vectors (e^c,
+  // e^(c_last - c), beta; the adjoint's scale e^c, e^(c_last - c), -beta e^c;
+  // e^c_last last); the adjoint's also Q rows and the M^T pair
   static constexpr int OFF_T = BC * LK, OFF_X = OFF_T + PAIR, OFF_VEC = OFF_X + BC * LC16;
   static constexpr int OFF_Q = OFF_VEC + 2 * 4 * BC, OFF_M = OFF_Q + BC * LK, BUF = OFF_M + PAIR;
   static constexpr size_t BYTES = 2 * sizeof(u16) * BUF;
@@ -151,13 +151,15 @@ struct Scan16 {
 };
 
 // One chunk's inputs in the registers of the loading waves (thread tid of
-// 64 NW). Rows past the sequence's end are clamped into it and zeroed.
+// LOADERS). Rows past the sequence's end are clamped into it by the loads and
+// zeroed by the stores.
 template <int K, int NW, bool ADJ>
 struct ScanLoad {
   using L = Scan16<K, NW>;
   static constexpr int N = L::LOADERS, KP = BC * K / 8 / N, TP = 768 / N, XP = BC * 2 * NW / N;
   uint4 k[KP], t[TP], x[XP], q[ADJ ? KP : 1], m[ADJ ? TP : 1];
   float cv, bv, last;
+  int left;  // tokens from the chunk's first to the sequence's end
 
   // Piece e of a triangular pair: [half][row][8 pieces], without the quadrant
   // that holds zeros only (T: rows < 32 of columns >= 32; M^T: the other one).
@@ -173,47 +175,61 @@ struct ScanLoad {
     }
   }
 
+  // Uniform bases and 32-bit lane offsets (a chunk's rows of all heads are
+  // under 2^31 bytes: 64 rows, at most 65,535 heads of 128 elements).
   __device__ __forceinline__ void load(const BwdParams &p, const BwdSeq &seq, int h, int hk, int i, int v0, int tid) {
     const int t0 = i * BC;
-    const long r = rec(p, seq, h, i);
+    left = seq.len - t0;
+    const int top = min(left, BC) - 1;
+    const long r = rec(p, seq, h, i), row0 = seq.bos + t0;
+    const u16 *kb = static_cast<const u16 *>(p.k) + (row0 * p.Hk + hk) * K;
+    const u16 *qb = static_cast<const u16 *>(p.q) + (row0 * p.Hk + hk) * K;
+    const u16 *xb = static_cast<const u16 *>(ADJ ? p.dout : p.v) + (row0 * p.Hv + h) * p.V + v0;
     const uint4 *wt = reinterpret_cast<const uint4 *>(p.ws_T + r * BC * BC);
     const uint4 *wm = reinterpret_cast<const uint4 *>(p.ws_M + r * BC * BC);
-    const u16 *src = static_cast<const u16 *>(ADJ ? p.dout : p.v);
-    auto row_of = [&](int row) { return seq.bos + min(t0 + row, seq.len - 1); };
+    const uint32_t kstride = p.Hk * K, xstride = p.Hv * p.V;
 #pragma unroll
     for (int a = 0; a < KP; ++a) {
-      const int e = tid + N * a, row = e / (K / 8), part = e % (K / 8);
-      const long off = (row_of(row) * p.Hk + hk) * K + part * 8;
-      const bool in = t0 + row < seq.len;
-      const uint4 y = *reinterpret_cast<const uint4 *>(static_cast<const u16 *>(p.k) + off);
-      k[a] = in ? y : uint4{0u, 0u, 0u, 0u};
-      if constexpr (ADJ) {
-        const uint4 z = *reinterpret_cast<const uint4 *>(static_cast<const u16 *>(p.q) + off);
-        q[a] = in ? z : uint4{0u, 0u, 0u, 0u};
-      }
+      const int e = tid + N * a;
+      const uint32_t off = min(e / (K / 8), top) * kstride + (e % (K / 8)) * 8;
+      k[a] = *reinterpret_cast<const uint4 *>(kb + off);
+      if constexpr (ADJ) q[a] = *reinterpret_cast<const uint4 *>(qb + off);
     }
 #pragma unroll
     for (int a = 0; a < TP; ++a) {
       int half, row, part;
       tri(tid + N * a, false, half, row, part);
-      t[a] = wt[half * 512 + row * 8 + part];
+      t[a] = wt[static_cast<uint32_t>(half * 512 + row * 8 + part)];
       if constexpr (ADJ) {
         tri(tid + N * a, true, half, row, part);
-        m[a] = wm[half * 512 + row * 8 + part];
+        m[a] = wm[static_cast<uint32_t>(half * 512 + row * 8 + part)];
       }
     }
 #pragma unroll
     for (int a = 0; a < XP; ++a) {
-      const int e = tid + N * a, row = e / (2 * NW), part = e % (2 * NW);
-      const uint4 y = *reinterpret_cast<const uint4 *>(src + (row_of(row) * p.Hv + h) * p.V + v0 + part * 8);
-      x[a] = t0 + row < seq.len ? y : uint4{0u, 0u, 0u, 0u};
+      const int e = tid + N * a;
+      const uint32_t off = min(e / (2 * NW), top) * xstride + (e % (2 * NW)) * 8;
+      x[a] = *reinterpret_cast<const uint4 *>(xb + off);
     }
     cv = p.ws_c[r * BC + (tid & 63)];
     bv = p.ws_beta[r * BC + (tid & 63)];
     last = p.ws_c[r * BC + BC - 1];
   }
 
-  __device__ __forceinline__ void store(u16 *buf, int tid) const {
+  __device__ __forceinline__ void store(u16 *buf, int tid, float scale) {
+    if (left < BC) {
+      const uint4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int a = 0; a < KP; ++a) {
+        if ((tid + N * a) / (K / 8) < left) continue;
+        k[a] = zero;
+        if constexpr (ADJ) q[a] = zero;
+      }
+#pragma unroll
+      for (int a = 0; a < XP; ++a) {
+        if ((tid + N * a) / (2 * NW) >= left) x[a] = zero;
+      }
+    }
 #pragma unroll
     for (int a = 0; a < KP; ++a) {
       const int e = tid + N * a, row = e / (K / 8), part = e % (K / 8);
@@ -237,70 +253,158 @@ struct ScanLoad {
     }
     if (tid < BC) {
       float *vec = reinterpret_cast<float *>(buf + L::OFF_VEC);
-      vec[tid] = expf(cv);
+      const float gam = expf(cv);
+      vec[tid] = ADJ ? scale * gam : gam;
       vec[BC + tid] = expf(last - cv);
-      vec[2 * BC + tid] = bv;
+      vec[2 * BC + tid] = ADJ ? -gam * bv : bv;
+      if (tid == BC - 1) vec[4 * BC - 1] = gam;
     }
   }
 };
 
+// A step's order is written out: the LDS reads of a product are issued before
+// the products (and the splits) that precede it, which hide their latency. The
+// compiler left to itself reads each fragment just before its use (some sixty
+// exposed waits a step: 1,681 us of scans at 1 x 32,768 tokens of 32 heads).
+__device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0); }
+
+// Key tiles' operands of the contraction over tokens 32 kb ..
+template <int KT>
+__device__ __forceinline__ void read_cols(const Lane &ln, const u16 *m, int ld, int kb, bh8_t (&a)[KT]) {
+#pragma unroll
+  for (int t = 0; t < KT; ++t) a[t] = ln.cols(m, ld, kb, 16 * t);
+}
+
+// s += the operands times a pair.
+template <int KT>
+__device__ __forceinline__ void add_products(float4_t (&s)[KT], const bh8_t (&a)[KT], bh8_t bh, bh8_t bl) {
+#pragma unroll
+  for (int t = 0; t < KT; ++t) s[t] = mfma_bf16(a[t], bh, s[t]);
+#pragma unroll
+  for (int t = 0; t < KT; ++t) s[t] = mfma_bf16(a[t], bl, s[t]);
+}
+
 // Chunk i's step on a wave's 16 columns: s is the state (or adjoint) before it
 // and after it.
 template <int K, int NW, bool ADJ>
-__device__ __forceinline__ void scan16_step(const BwdParams &p, const u16 *buf, const Lane &ln, int col,
-                                            float4_t (&s)[K / 16]) {
+__device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int col, float4_t (&s)[K / 16]) {
   using L = Scan16<K, NW>;
   constexpr int KT = K / 16, KB = K / 32, LK = L::LK, LB = L::LB, CC = BC * LB;
   const u16 *sk = buf, *tp = buf + L::OFF_T, *sx = buf + L::OFF_X;
-  const float *sgam = reinterpret_cast<const float *>(buf + L::OFF_VEC), *se = sgam + BC, *sbeta = se + BC;
+  const float *vec = reinterpret_cast<const float *>(buf + L::OFF_VEC) + 4 * ln.g;
+  // ---- K S
+  bh8_t ka[KB][4];
+#pragma unroll
+  for (int kb = 0; kb < KB / 2; ++kb) {
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows(sk, LK, 16 * rt, kb);
+  }
+  keep_order();
   v2u32_t sh[KT], sl[KT];
 #pragma unroll
   for (int m = 0; m < KT; ++m) split_bf16(s[m], sh[m], sl[m]);
-  float4_t y[4];  // K S
+  keep_order();
+#pragma unroll
+  for (int kb = KB / 2; kb < KB; ++kb) {
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows(sk, LK, 16 * rt, kb);
+  }
+  keep_order();
+  float4_t y[4];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) y[rt] = zero4();
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
+  auto ks = [&](int kb) {
     const bh8_t bh = frag_pair(sh[2 * kb], sh[2 * kb + 1]), bl = frag_pair(sl[2 * kb], sl[2 * kb + 1]);
-    bh8_t a[4];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) a[rt] = ln.rows(sk, LK, 16 * rt, kb);
+    for (int rt = 0; rt < 4; ++rt) y[rt] = mfma_bf16(ka[kb][rt], bh, y[rt]);
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) y[rt] = mfma_bf16(a[rt], bh, y[rt]);
+    for (int rt = 0; rt < 4; ++rt) y[rt] = mfma_bf16(ka[kb][rt], bl, y[rt]);
+  };
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) y[rt] = mfma_bf16(a[rt], bl, y[rt]);
-  }
+  for (int kb = 0; kb < KB / 2; ++kb) ks(kb);
+  keep_order();
+  // T's operands (the triangle): fragment (rt, kb) of U's rows or dX's columns
+  bh8_t th[4][2], tl[4][2];
+  auto used = [](int rt, int kb) { return ADJ ? kb >= (rt >> 1) : kb <= (rt >> 1); };
+  auto read_t = [&] {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        if (!used(rt, kb)) continue;
+        th[rt][kb] = ADJ ? ln.cols(tp, LB, kb, 16 * rt) : ln.rows(tp, LB, 16 * rt, kb);
+        tl[rt][kb] = ADJ ? ln.cols(tp + CC, LB, kb, 16 * rt) : ln.rows(tp + CC, LB, 16 * rt, kb);
+      }
+    }
+  };
   v2u32_t xh[4], xl[4];  // beta X, or dU
   v2u32_t oh[4], ol[4];  // scale Gamma dO
+  bw_i16x4_t xr[4];      // V's or dO's rows
+  float4_t w0[4], w1[4];
   if constexpr (!ADJ) {
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      const int o = 16 * rt + 4 * ln.g;
-      const float4_t x = bf16x4_float(ln.tr(sx + 16 * rt * L::LC16, L::LC16, col)) - ld4(&sgam[o]) * y[rt];
-      split_bf16(x * ld4(&sbeta[o]), xh[rt], xl[rt]);
+      xr[rt] = ln.tr(sx + 16 * rt * L::LC16, L::LC16, col);
+      w0[rt] = ld4(vec + 16 * rt);           // e^c
+      w1[rt] = ld4(vec + 2 * BC + 16 * rt);  // beta
+    }
+    read_t();
+    keep_order();
+#pragma unroll
+    for (int kb = KB / 2; kb < KB; ++kb) ks(kb);
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      split_bf16((bf16x4_float(xr[rt]) - w0[rt] * y[rt]) * w1[rt], xh[rt], xl[rt]);
     }
   } else {
     const u16 *mt = buf + L::OFF_M;
-    bh8_t dof[2];
+    bh8_t mh[4][2], ml[4][2], dof[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) dof[kb] = ln.cols(sx, L::LC16, kb, col);
+    for (int rt = 0; rt < 4; ++rt) w0[rt] = ld4(vec + BC + 16 * rt);  // e^(c_last - c)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) y[rt] *= ld4(&se[16 * rt + 4 * ln.g]);
+    for (int rt = 0; rt < 4; ++rt) xr[rt] = ln.tr(sx + 16 * rt * L::LC16, L::LC16, col);
 #pragma unroll
-    for (int kb = 1; kb >= 0; --kb) {  // t >= s
+    for (int kb = 1; kb >= 0; --kb) {
 #pragma unroll
-      for (int rt = 0; rt < 2 * kb + 2; ++rt) y[rt] = mfma_bf16(ln.rows(mt, LB, 16 * rt, kb), dof[kb], y[rt]);
+      for (int rt = 0; rt < 2 * kb + 2; ++rt) {  // t >= s
+        mh[rt][kb] = ln.rows(mt, LB, 16 * rt, kb);
+        ml[rt][kb] = ln.rows(mt + CC, LB, 16 * rt, kb);
+      }
+    }
+    keep_order();
 #pragma unroll
-      for (int rt = 0; rt < 2 * kb + 2; ++rt) y[rt] = mfma_bf16(ln.rows(mt + CC, LB, 16 * rt, kb), dof[kb], y[rt]);
+    for (int kb = KB / 2; kb < KB; ++kb) ks(kb);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      dof[kb] = frag_pair(__builtin_bit_cast(v2u32_t, xr[2 * kb]), __builtin_bit_cast(v2u32_t, xr[2 * kb + 1]));
     }
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      split_bf16(y[rt], xh[rt], xl[rt]);
-      const float4_t d = bf16x4_float(ln.tr(sx + 16 * rt * L::LC16, L::LC16, col));
-      split_bf16(d * (ld4(&sgam[16 * rt + 4 * ln.g]) * p.scale), oh[rt], ol[rt]);
+    for (int rt = 0; rt < 4; ++rt) y[rt] *= w0[rt];
+    keep_order();
+    read_t();
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) w1[rt] = ld4(vec + 16 * rt);  // scale e^c
+    keep_order();
+#pragma unroll
+    for (int kb = 1; kb >= 0; --kb) {
+#pragma unroll
+      for (int rt = 0; rt < 2 * kb + 2; ++rt) y[rt] = mfma_bf16(mh[rt][kb], dof[kb], y[rt]);
+#pragma unroll
+      for (int rt = 0; rt < 2 * kb + 2; ++rt) y[rt] = mfma_bf16(ml[rt][kb], dof[kb], y[rt]);
     }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) split_bf16(bf16x4_float(xr[rt]) * w1[rt], oh[rt], ol[rt]);
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) split_bf16(y[rt], xh[rt], xl[rt]);
   }
-  // U = T (beta X), s <= t; or dX / beta = T^T dU, t >= s
+  keep_order();
+  // ---- U = T (beta X), s <= t; or dX / beta = T^T dU, t >= s
+  bh8_t a0[KT], a1[KT];
+  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, LK, 0, a0);
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt) w0[rt] = ld4(vec + (ADJ ? 2 : 1) * BC + 16 * rt);  // -beta e^c, or e^(c_last - c)
+  const float gam_c = vec[4 * BC - 1 - 4 * ln.g];
+  keep_order();
   float4_t z[4];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) z[rt] = zero4();
@@ -309,51 +413,40 @@ __device__ __forceinline__ void scan16_step(const BwdParams &p, const u16 *buf, 
     const bh8_t bh = frag_pair(xh[2 * kb], xh[2 * kb + 1]), bl = frag_pair(xl[2 * kb], xl[2 * kb + 1]);
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      if (ADJ ? kb < (rt >> 1) : kb > (rt >> 1)) continue;
-      const bh8_t th = ADJ ? ln.cols(tp, LB, kb, 16 * rt) : ln.rows(tp, LB, 16 * rt, kb);
-      const bh8_t tl = ADJ ? ln.cols(tp + CC, LB, kb, 16 * rt) : ln.rows(tp + CC, LB, 16 * rt, kb);
-      z[rt] = mfma_bf16(th, bh, z[rt]);
-      z[rt] = mfma_bf16(th, bl, z[rt]);
-      z[rt] = mfma_bf16(tl, bh, z[rt]);
+      if (used(rt, kb)) z[rt] = mfma_bf16(th[rt][kb], bh, z[rt]);
     }
-  }
-  const float gam_c = sgam[BC - 1];
-  v2u32_t zh[4], zl[4];  // E U, or -Gamma dX
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
-    const int o = 16 * rt + 4 * ln.g;
-    split_bf16(ADJ ? z[rt] * (-(ld4(&sgam[o]) * ld4(&sbeta[o]))) : z[rt] * ld4(&se[o]), zh[rt], zl[rt]);
+    for (int rt = 0; rt < 4; ++rt) {
+      if (used(rt, kb)) z[rt] = mfma_bf16(th[rt][kb], bl, z[rt]);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      if (used(rt, kb)) z[rt] = mfma_bf16(tl[rt][kb], bh, z[rt]);
+    }
   }
 #pragma unroll
   for (int m = 0; m < KT; ++m) s[m] *= gam_c;
+  keep_order();
+  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, LK, 1, a1);
+  keep_order();
+  v2u32_t zh[4], zl[4];  // E U, or -Gamma dX
+  if constexpr (ADJ) {  // Q's products fill the splits' place in the chain
+    add_products(s, a0, frag_pair(oh[0], oh[1]), frag_pair(ol[0], ol[1]));
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const bh8_t bh = frag_pair(zh[2 * kb], zh[2 * kb + 1]), bl = frag_pair(zl[2 * kb], zl[2 * kb + 1]);
+    for (int rt = 0; rt < 4; ++rt) split_bf16(z[rt] * w0[rt], zh[rt], zl[rt]);
+    keep_order();
+    read_cols(ln, sk, LK, 0, a0);
+    keep_order();
+    add_products(s, a1, frag_pair(oh[2], oh[3]), frag_pair(ol[2], ol[3]));
+    keep_order();
+    read_cols(ln, sk, LK, 1, a1);
+    keep_order();
+  } else {
 #pragma unroll
-    for (int m0 = 0; m0 < KT; m0 += 4) {
-      bh8_t a[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) a[m] = ln.cols(sk, LK, kb, 16 * (m0 + m));
-#pragma unroll
-      for (int m = 0; m < 4; ++m) s[m0 + m] = mfma_bf16(a[m], bh, s[m0 + m]);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) s[m0 + m] = mfma_bf16(a[m], bl, s[m0 + m]);
-    }
-    if constexpr (ADJ) {
-      const u16 *sq = buf + L::OFF_Q;
-      const bh8_t ch = frag_pair(oh[2 * kb], oh[2 * kb + 1]), cl = frag_pair(ol[2 * kb], ol[2 * kb + 1]);
-#pragma unroll
-      for (int m0 = 0; m0 < KT; m0 += 4) {
-        bh8_t a[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) a[m] = ln.cols(sq, LK, kb, 16 * (m0 + m));
-#pragma unroll
-        for (int m = 0; m < 4; ++m) s[m0 + m] = mfma_bf16(a[m], ch, s[m0 + m]);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) s[m0 + m] = mfma_bf16(a[m], cl, s[m0 + m]);
-      }
-    }
+    for (int rt = 0; rt < 4; ++rt) split_bf16(z[rt] * w0[rt], zh[rt], zl[rt]);
   }
+  add_products(s, a0, frag_pair(zh[0], zh[1]), frag_pair(zl[0], zl[1]));
+  add_products(s, a1, frag_pair(zh[2], zh[3]), frag_pair(zl[2], zl[3]));
 }
 
 template <int K, int NW, bool ADJ>
@@ -366,16 +459,26 @@ __device__ __forceinline__ void scan16_pass(const BwdParams &p, u16 *lds, int n,
   auto chunk = [&](int j) { return ADJ ? seq.n - 1 - j : j; };  // the chunk of step j
   if (wave >= NW) {
     const int tid = threadIdx.x - 64 * NW;
-    ScanLoad<K, NW, ADJ> in;
+    // Two chunks in flight: a step's loads have two steps to arrive (one step
+    // was too short: the fill of 68 KiB came after the loads' latency, 3.3 us
+    // a step).
+    ScanLoad<K, NW, ADJ> even, odd;
+    auto load = [&](ScanLoad<K, NW, ADJ> &in, int j) { in.load(p, seq, h, hk, chunk(min(j, seq.n - 1)), v0, tid); };
+    u16 *buf1 = lds + L::BUF;
     if (seq.n > 0) {
-      in.load(p, seq, h, hk, chunk(0), v0, tid);
-      in.store(lds, tid);
-      if (seq.n > 1) in.load(p, seq, h, hk, chunk(1), v0, tid);
+      load(even, 0);
+      load(odd, 1);
+      even.store(lds, tid, p.scale);
+      load(even, 2);
     }
-    for (int j = 0; j < seq.n; ++j) {
+    for (int j = 0; j < seq.n; j += 2) {
       __syncthreads();  // step j's buffer is written, step j - 1's is free
-      if (j + 1 < seq.n) in.store(lds + ((j + 1) & 1) * L::BUF, tid);
-      if (j + 2 < seq.n) in.load(p, seq, h, hk, chunk(j + 2), v0, tid);
+      odd.store(buf1, tid, p.scale);
+      load(odd, j + 3);
+      if (j + 1 == seq.n) break;
+      __syncthreads();
+      even.store(lds, tid, p.scale);
+      load(even, j + 4);
     }
     return;
   }
@@ -396,7 +499,7 @@ __device__ __forceinline__ void scan16_pass(const BwdParams &p, u16 *lds, int n,
 #pragma unroll
     for (int m = 0; m < KT; ++m) ws[64 * m] = s[m];
     __syncthreads();
-    scan16_step<K, NW, ADJ>(p, lds + (j & 1) * L::BUF, ln, 16 * wave, s);
+    scan16_step<K, NW, ADJ>(lds + (j & 1) * L::BUF, ln, 16 * wave, s);
   }
   if (ADJ && p.dh0) {
 #pragma unroll
@@ -410,7 +513,7 @@ __device__ __forceinline__ void scan16_pass(const BwdParams &p, u16 *lds, int n,
 // Both roles in one launch, the adjoint (the longer step) first. The column
 // groups and value heads of a key head read the same K and Q rows: one XCD.
 template <int K, int NW>
-__global__ __launch_bounds__(128 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2, NW / 2)))
+__global__ __launch_bounds__(64 * NW + 256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_scans_bf16_kernel(BwdParams p) {
   extern __shared__ __align__(16) float lds[];
   PBGDN_POISON_LDS(lds, (Scan16<K, NW>::BYTES));
