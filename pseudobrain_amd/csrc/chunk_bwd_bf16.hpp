@@ -101,7 +101,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
   BwdSeq seq;
   int i;
   if (!chunk_of(p, blockIdx.x, blockIdx.z, seq, i)) return;
-  const int t0 = i * BC;
+  const int t0 = i * BC, left = seq.len - t0;  // the chunk's tokens: left, if under BC
   const int group = p.Hv / p.Hk;
   float4_t tq[KTW][2], tk[KTW][2];
 #pragma unroll
@@ -140,12 +140,15 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     u16 *mt = area, *sv = area + 2 * CC;
     {
       RawRows<u16, V, NT> rv, rd;
-      uint4 rt[BC * BC / 4 / NT];  // T's pair: 1,024 pieces of 16 bytes
+      uint4 rt[BC * BC / 4 / NT], rm[BC * BC / 4 / NT];  // the T and M^T pairs: 1,024 pieces of 16 bytes each
       rd.load(tid, p.dout, seq, t0, p.Hv, h, V);
       rv.load(tid, p.v, seq, t0, p.Hv, h, V);
       const uint4 *wt = reinterpret_cast<const uint4 *>(p.ws_T + r * BC * BC);
+      const uint4 *wm = reinterpret_cast<const uint4 *>(p.ws_M + r * BC * BC);
 #pragma unroll
       for (int m = 0; m < BC * BC / 4 / NT; ++m) rt[m] = wt[tid + NT * m];
+#pragma unroll
+      for (int m = 0; m < BC * BC / 4 / NT; ++m) rm[m] = wm[tid + NT * m];
       const float cv = p.ws_c[r * BC + lane], bv = p.ws_beta[r * BC + lane], last = p.ws_c[r * BC + BC - 1];
       if (hh > 0) __syncthreads();  // the previous head's readers of LDS are done
       if (hh == 0) {
@@ -161,6 +164,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       for (int m = 0; m < BC * BC / 4 / NT; ++m) {
         const int e = tid + NT * m;
         *reinterpret_cast<uint4 *>(tp + (e >> 3) * LB + 8 * (e & 7)) = rt[m];  // half e / 512, row (e / 8) & 63
+        *reinterpret_cast<uint4 *>(mt + (e >> 3) * LB + 8 * (e & 7)) = rm[m];
       }
       if (tid < BC) {
         sc[tid] = cv;
@@ -170,20 +174,6 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
-    // ---- M^T[s][t] = scale (k_s . q_t) e^(c_t - c_s), t >= s: rows of pair rp
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-#pragma unroll
-      for (int m = 0; m < CTW; ++m) {
-        const int ts = 2 * rp + a, tt = CTW * cp + m;
-        const float4_t kq = L4.rows_rows<K>(sk, sq, LK, 16 * ts, 16 * tt);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int s2 = 16 * ts + 4 * g4 + e, t = 16 * tt + c;
-          put_pair1(mt, CC, s2 * LB + t, t >= s2 ? p.scale * kq[e] * expf(sc[t] - sc[s2]) : 0.f);
-        }
-      }
-    }
     // ---- chain: this wave's 16 value columns
     float dgc = 0.f;
     v2u32_t sh[KT], sl[KT], dh[KT], dl[KT];
@@ -215,7 +205,6 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       split_bf16(x * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
       du[rt] = ld4(&se[o]) * kd;
     }
-    __syncthreads();  // M^T is complete
     v2u32_t duh[4], dul[4];
     {
       bh8_t dof[2];
@@ -254,14 +243,6 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       dx *= ld4(&sbeta[16 * rt + 4 * g4]);
       split_bf16(u, uh[rt], ul[rt]);
       split_bf16(dx, dxh[rt], dxl[rt]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {  // dv = dX, rounded: its high half
-        const int t = t0 + 16 * rt + 4 * g4 + e;
-        if (t < seq.len) {
-          static_cast<u16 *>(p.dv)[((seq.bos + t) * p.Hv + h) * V + v0 + c] =
-              static_cast<u16>(dxh[rt][e >> 1] >> (16 * (e & 1)));
-        }
-      }
     }
     // ---- contractions over the value columns
     u16 *a0 = area, *a1 = area + 2 * TV;
@@ -355,6 +336,15 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     __syncthreads();
     publish(a0, dxh, dxl);
     publish_state(sh);
+    {  // dv = dX, rounded (its high half): this wave's columns, four a lane and token
+      u16 *dv = static_cast<u16 *>(p.dv) + ((seq.bos + t0) * p.Hv + h) * V + v0;
+      const uint32_t stride = p.Hv * V;
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        const v2u32_t x = __builtin_bit_cast(v2u32_t, L4.tr(a0 + v0 * LB, LB, 16 * rt));
+        if (16 * rt + c < left) *reinterpret_cast<v2u32_t *>(dv + (16 * rt + c) * stride + 4 * g4) = x;
+      }
+    }
     __syncthreads();
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {  // dK2 = dX S^T, dQ0 = dO S^T, the high half of S
@@ -423,30 +413,44 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();  // the stages' readers are done: the area now holds the C x C pairs
-    u16 *b1p = area, *b2p = b1p + 2 * CC, *b3p = b2p + 2 * CC, *b4p = b3p + 2 * CC;
+    // The C x C matrices as transposed pairs [column][row]: a lane's four rows
+    // of a column are one 8-byte write a half.
+    u16 *b1t = area, *b2t = b1t + 2 * CC, *b3t = b2t + 2 * CC, *b4t = b3t + 2 * CC;
+    auto put_t = [&](u16 *m, int row0, int col0, float4_t x) {
+      v2u32_t hi, lo;
+      split_bf16(x, hi, lo);
+      u16 *at = m + (col0 + c) * LB + row0 + 4 * g4;
+      *reinterpret_cast<v2u32_t *>(at) = hi;
+      *reinterpret_cast<v2u32_t *>(at + CC) = lo;
+    };
     // dM o Mt into b1 (and its dc terms); dT = dTb diag(beta) into b2 (and dbeta)
-    float rc[2][4], rb[2][4], cc[CTW], cb[CTW];
+    float4_t rc[2], rb[2], dec[CTW][2];  // row sums; D = e^(c_t - c_s)
+    float cc[CTW], cb[CTW];
 #pragma unroll
     for (int m = 0; m < CTW; ++m) cc[m] = cb[m] = 0.f;
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) rc[a][e] = rb[a][e] = 0.f;
+      const int row0 = 32 * rp + 16 * a;
+      const float4_t ct = ld4(&sc[row0 + 4 * g4]);
+      rc[a] = rb[a] = zero4();
 #pragma unroll
       for (int m = 0; m < CTW; ++m) {
-        const int s2 = 16 * (CTW * cp + m) + c;
-        const float4_t qk = L4.rows_rows<K>(sq, sk, LK, 32 * rp + 16 * a, 16 * (CTW * cp + m));
+        const int col0 = 16 * (CTW * cp + m), s2 = col0 + c, above = s2 - row0 - 4 * g4;  // e >= above: t >= s
+        const float cs = sc[s2], bs = sbeta[s2];
+        const float4_t qk = L4.rows_rows<K>(sq, sk, LK, row0, col0);
+        const bw_i16x4_t thi = L4.tr(tp + row0 * LB, LB, col0), tlo = L4.tr(tp + CC + row0 * LB, LB, col0);
+        const float4_t tv = bf16x4_float(thi) + bf16x4_float(tlo);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t = 32 * rp + 16 * a + 4 * g4 + e;
-          const float d = t >= s2 ? p.scale * expf(sc[t] - sc[s2]) : 0.f;
-          const float dmd = t >= s2 ? dm[m][a][e] * d : 0.f;
-          put_pair1(b1p, CC, t * LB + s2, dmd);
-          rc[a][e] += dmd * qk[e];
-          cc[m] -= dmd * qk[e];
-          put_pair1(b2p, CC, t * LB + s2, dtb[m][a][e] * sbeta[s2]);
-          cb[m] += dtb[m][a][e] * pair_val(tp, CC, t * LB + s2);
-        }
+        for (int e = 0; e < 4; ++e) dec[m][a][e] = expf(ct[e] - cs);
+        float4_t dmd = dm[m][a] * (dec[m][a] * p.scale);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dmd[e] = e >= above ? dmd[e] : 0.f;
+        const float4_t dcr = dmd * qk, dbr = dtb[m][a] * tv;
+        put_t(b1t, row0, col0, dmd);
+        put_t(b2t, row0, col0, dtb[m][a] * bs);
+        rc[a] += dcr;
+        cc[m] -= (dcr[0] + dcr[1]) + (dcr[2] + dcr[3]);
+        cb[m] += (dbr[0] + dbr[1]) + (dbr[2] + dbr[3]);
       }
     }
     __syncthreads();
@@ -455,53 +459,45 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     for (int a = 0; a < 2; ++a) {
 #pragma unroll
       for (int m = 0; m < CTW; ++m) {
+        const int row0 = 32 * rp + 16 * a, col0 = 16 * (CTW * cp + m);
         float4_t w = zero4();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const bh8_t th = L4.cols(tp, LB, kb, 32 * rp + 16 * a), tl = L4.cols(tp + CC, LB, kb, 32 * rp + 16 * a);
-          const bh8_t bh = L4.cols(b2p, LB, kb, 16 * (CTW * cp + m)),
-                      bl = L4.cols(b2p + CC, LB, kb, 16 * (CTW * cp + m));
+          const bh8_t th = L4.cols(tp, LB, kb, row0), tl = L4.cols(tp + CC, LB, kb, row0);
+          const bh8_t bh = L4.rows(b2t, LB, col0, kb), bl = L4.rows(b2t + CC, LB, col0, kb);
           w = mfma_bf16(th, bh, w);
           w = mfma_bf16(th, bl, w);
           w = mfma_bf16(tl, bh, w);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          put_pair1(b4p, CC, (32 * rp + 16 * a + 4 * g4 + e) * LB + 16 * (CTW * cp + m) + c, w[e]);
-        }
+        put_t(b4t, row0, col0, w);
       }
     }
     __syncthreads();
-    // dA = -W T^T (strict lower): H = dA beta_t D, as H + H^T in b3; dbeta, dc terms
+    // dA = -W T^T (strict lower): H = dA beta_t D into b3; dbeta, dc terms
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
+      const float4_t bt = ld4(&sbeta[32 * rp + 16 * a + 4 * g4]);
 #pragma unroll
       for (int m = 0; m < CTW; ++m) {
-        const int row0 = 32 * rp + 16 * a, col0 = 16 * (CTW * cp + m);
+        const int row0 = 32 * rp + 16 * a, col0 = 16 * (CTW * cp + m), above = col0 + c - row0 - 4 * g4;
         float4_t da = zero4();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const bh8_t wh = L4.rows16(b4p, LB, row0, kb), wl = L4.rows16(b4p + CC, LB, row0, kb);
-          const bh8_t th = L4.rows16(tp, LB, col0, kb), tl = L4.rows16(tp + CC, LB, col0, kb);
+          const bh8_t wh = L4.cols(b4t, LB, kb, row0), wl = L4.cols(b4t + CC, LB, kb, row0);
+          const bh8_t th = L4.rows(tp, LB, col0, kb), tl = L4.rows(tp + CC, LB, col0, kb);
           da = mfma_bf16(wh, th, da);
           da = mfma_bf16(wh, tl, da);
           da = mfma_bf16(wl, th, da);
         }
         const float4_t gk = L4.rows_rows<K>(sk, sk, LK, row0, col0);
+        float4_t dad = dec[m][a] * -da;  // dA o D, t > s
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t = row0 + 4 * g4 + e, s2 = col0 + c;
-          const float d = t > s2 ? expf(sc[t] - sc[s2]) : 0.f;
-          const float dav = t > s2 ? -da[e] : 0.f;
-          const float hv = dav * sbeta[t] * d, b = dav * gk[e] * d;
-          rb[a][e] += b;
-          rc[a][e] += b * sbeta[t];
-          cc[m] -= b * sbeta[t];
-          if (t >= s2) {
-            put_pair1(b3p, CC, t * LB + s2, hv);
-            put_pair1(b3p, CC, s2 * LB + t, hv);
-          }
-        }
+        for (int e = 0; e < 4; ++e) dad[e] = e > above ? dad[e] : 0.f;
+        const float4_t b = dad * gk, bb = b * bt;
+        put_t(b3t, row0, col0, dad * bt);
+        rb[a] += b;
+        rc[a] += bb;
+        cc[m] -= (bb[0] + bb[1]) + (bb[2] + bb[3]);
       }
     }
 #pragma unroll
@@ -524,19 +520,21 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
-    // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + (H + H^T) K
+    // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + H K + H^T K
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      bh8_t a1h[2], a1l[2], a3h[2], a3l[2], t1h[2], t1l[2];
+      bh8_t a1h[2], a1l[2], a3h[2], a3l[2], t1h[2], t1l[2], t3h[2], t3l[2];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
         const int row0 = 32 * rp + 16 * a;
-        a1h[a] = L4.rows(b1p, LB, row0, kb);
-        a1l[a] = L4.rows(b1p + CC, LB, row0, kb);
-        a3h[a] = L4.rows(b3p, LB, row0, kb);
-        a3l[a] = L4.rows(b3p + CC, LB, row0, kb);
-        t1h[a] = L4.cols(b1p, LB, kb, row0);
-        t1l[a] = L4.cols(b1p + CC, LB, kb, row0);
+        a1h[a] = L4.cols(b1t, LB, kb, row0);
+        a1l[a] = L4.cols(b1t + CC, LB, kb, row0);
+        a3h[a] = L4.cols(b3t, LB, kb, row0);
+        a3l[a] = L4.cols(b3t + CC, LB, kb, row0);
+        t1h[a] = L4.rows(b1t, LB, row0, kb);
+        t1l[a] = L4.rows(b1t + CC, LB, row0, kb);
+        t3h[a] = L4.rows(b3t, LB, row0, kb);
+        t3l[a] = L4.rows(b3t + CC, LB, row0, kb);
       }
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
@@ -549,6 +547,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
           tk[m][a] = mfma_bf16(t1l[a], qf, tk[m][a]);
           tk[m][a] = mfma_bf16(a3h[a], kf, tk[m][a]);
           tk[m][a] = mfma_bf16(a3l[a], kf, tk[m][a]);
+          tk[m][a] = mfma_bf16(t3h[a], kf, tk[m][a]);
+          tk[m][a] = mfma_bf16(t3l[a], kf, tk[m][a]);
         }
       }
     }
@@ -584,23 +584,47 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
   const bool direct = heads == group;
   const int h0 = blockIdx.y * heads, c = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rp = wave & 1, cp = wave >> 1;
+  if (direct) {
+    // each tile through LDS, transposed (this wave writes and reads it), for
+    // pieces of four keys a lane and token
+    __syncthreads();  // the last head's readers of LDS are done
+    const Lane L4{c, g4};
+    const long base = ((seq.bos + t0) * p.Hk + h0 / group) * K;
+    const uint32_t stride = p.Hk * K;
+    u16 *buf = reinterpret_cast<u16 *>(lds) + wave * 16 * LB;
+    auto out = [&](void *dst, const float4_t (&x)[KTW][2]) {
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          *reinterpret_cast<v2u32_t *>(buf + c * LB + 16 * a + 4 * g4) =
+              __builtin_bit_cast(v2u32_t, __builtin_convertvector(x[m][a], bf16x4_t));
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const v2u32_t y = __builtin_bit_cast(v2u32_t, L4.tr(buf, LB, 16 * a));
+          const int t = 32 * rp + 16 * a + c;
+          u16 *row = static_cast<u16 *>(dst) + base + 16 * (KTW * cp + m);
+          if (t < left) *reinterpret_cast<v2u32_t *>(row + t * stride + 4 * g4) = y;
+        }
+      }
+    };
+    out(p.dq, tq);
+    out(p.dk, tk);
+    return;
+  }
 #pragma unroll
   for (int m = 0; m < KTW; ++m) {
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int t = t0 + 32 * rp + 16 * a + 4 * g4 + e, kk = 16 * (KTW * cp + m) + c;
-        if (t >= seq.len) continue;
-        if (direct) {
-          const long o = ((seq.bos + t) * p.Hk + h0 / group) * K + kk;
-          store_el<u16>(p.dq, o, tq[m][a][e]);
-          store_el<u16>(p.dk, o, tk[m][a][e]);
-        } else {
-          const long o = ((seq.bos + t) * p.Hv + h0) * K + kk;
-          p.ws_dq[o] = tq[m][a][e];
-          p.ws_dk[o] = tk[m][a][e];
-        }
+        const int t = 32 * rp + 16 * a + 4 * g4 + e, kk = 16 * (KTW * cp + m) + c;
+        if (t >= left) continue;
+        const long base = ((seq.bos + t0) * p.Hv + h0) * K;
+        const uint32_t off = t * static_cast<uint32_t>(p.Hv * K) + kk;
+        (p.ws_dq + base)[off] = tq[m][a][e];
+        (p.ws_dk + base)[off] = tk[m][a][e];
       }
     }
   }
