@@ -1732,8 +1732,11 @@ int launch_grad_bf16(const BwdParams &p, int heads, hipStream_t st) {
                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L::BYTES)) != hipSuccess) {
     return PBGDN_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL((bwd_grad_bf16_kernel<K, V>), dim3(p.cu_seqlens ? p.records : p.n, p.Hv / heads, p.B),
-                     dim3(L::NT), L::BYTES, st, p, heads);
+  // one workgroup a CU (its LDS), each taking items until none is left
+  const long items = static_cast<long>(p.cu_seqlens ? p.records : p.n) * (p.Hv / heads) * p.B;
+  if (items > 0x3fffffffL) return PBGDN_ERR_UNSUPPORTED;
+  const unsigned grid = static_cast<unsigned>(std::min<long>(items, p.cus > 0 ? p.cus : 256));
+  hipLaunchKernelGGL((bwd_grad_bf16_kernel<K, V>), dim3(grid), dim3(L::NT), L::BYTES, st, p, heads);
   return hipGetLastError() == hipSuccess ? PBGDN_OK : PBGDN_ERR_LAUNCH;
 }
 

@@ -1,9 +1,9 @@
 // The gradient kernel of the chunk backward for bfloat16 inputs (included by
 // chunk_bwd.hip, whose notation and helpers it uses).
 //
-// One workgroup of V / 16 waves per (chunk, key head), the value heads of the
-// key head in turn, so dq and dk are summed over them in registers. For each
-// value head:
+// A workgroup of V / 16 waves takes items (chunk, key head) in turn, and of
+// each the value heads of the key head, so dq and dk are summed over them in
+// registers. For each value head:
 //
 //   chain    wave w holds the 16 value columns 16 w .. of the start state S
 //            and the end adjoint dS' in registers and forms its columns of
@@ -75,6 +75,9 @@ __device__ __forceinline__ float4_t bf16x4_float(bw_i16x4_t x) {
                   __uint_as_float(w[1] & 0xffff0000u)};
 }
 
+// No instruction crosses this point: bounds how far the compiler moves reads.
+__device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0); }
+
 template <int K, int V>
 struct GradLds {
   static constexpr int NW = V / 16, NT = 64 * NW, COLS = NW / 2;  // waves; wave pairs
@@ -89,6 +92,57 @@ struct GradLds {
   static constexpr size_t BYTES = sizeof(u16) * (2 * BC * LK + BC * LV + 2 * CC + AREA) + sizeof(float) * FLOATS;
 };
 
+// Rows 0 .. 63 from a uniform base (the chunk's first row) in registers, to be
+// put into LDS later: rows past `left` are clamped into the sequence by the
+// loads and zeroed by the put, so nothing waits for the loads before that.
+template <int W, int NT>
+struct RowsAhead {
+  static constexpr int PPR = W / 8, PER = BC * PPR / NT;
+  v4u32_t raw[PER];
+
+  __device__ __forceinline__ void load(int tid, const u16 *base, uint32_t stride, int left) {
+    const int top = min(left, BC) - 1;
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      const int e = tid + NT * m;
+      const uint32_t off = static_cast<uint32_t>(min(e / PPR, top)) * stride + (e % PPR) * 8;
+      raw[m] = *reinterpret_cast<const v4u32_t *>(base + off);
+    }
+  }
+  __device__ __forceinline__ void put(int tid, u16 *dst, int ld, int left) {
+    if (left < BC) {
+#pragma unroll
+      for (int m = 0; m < PER; ++m) {
+        if ((tid + NT * m) / PPR >= left) raw[m] = v4u32_t{0u, 0u, 0u, 0u};
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      const int e = tid + NT * m;
+      *reinterpret_cast<v4u32_t *>(dst + (e / PPR) * ld + (e % PPR) * 8) = raw[m];
+    }
+  }
+};
+
+// A gradient workgroup's place in its items (chunk, group of value heads).
+struct GradItem {
+  BwdSeq seq;
+  int i, block;   // the chunk; the value heads block * heads ..
+  unsigned item;  // the item's index
+};
+// The first item at or after `item` (in steps of `step`) that holds a chunk.
+__device__ __forceinline__ bool grad_item(const BwdParams &p, unsigned item, unsigned step, unsigned items,
+                                          unsigned chunks, unsigned blocks, GradItem &it) {
+  for (; item < items; item += step) {
+    const unsigned rest = item / chunks;
+    if (!chunk_of(p, item % chunks, rest / blocks, it.seq, it.i)) continue;
+    it.block = rest % blocks;
+    it.item = item;
+    return true;
+  }
+  return false;
+}
+
 template <int K, int V>
 __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int heads) {
   using L = GradLds<K, V>;
@@ -98,19 +152,60 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
   extern __shared__ __align__(16) float lds[];
   PBGDN_POISON_LDS(lds, L::BYTES);
   PBGDN_POISON_SYNC();
-  BwdSeq seq;
-  int i;
-  if (!chunk_of(p, blockIdx.x, blockIdx.z, seq, i)) return;
-  const int t0 = i * BC, left = seq.len - t0;  // the chunk's tokens: left, if under BC
   const int group = p.Hv / p.Hk;
+  const unsigned chunks = p.cu_seqlens ? p.records : p.n, blocks = p.Hv / heads, items = chunks * blocks * p.B;
+  GradItem it, next;
+  if (!grad_item(p, blockIdx.x, gridDim.x, items, chunks, blocks, it)) return;
+  // A head's inputs, in registers from the stages of the head before: a CU
+  // holds one workgroup, so loads issued at a head's start were waited for in
+  // full (16,000 to 60,000 cycles of a head's 60,000 to 100,000).
+  float4_t sf[KT], df[KT];
+  v4u32_t rt[BC * BC / 4 / NT], rm[BC * BC / 4 / NT];  // the T and M^T pairs: 1,024 pieces of 16 bytes each
+  RowsAhead<V, NT> rv, rd;
+  RowsAhead<K, NT> rq, rk;
+  float cv, bv, last;
+  auto load_adjoint = [&](const GradItem &at, int h, int tid) {
+    const float4_t *wd = reinterpret_cast<const float4_t *>(p.ws_dS + rec(p, at.seq, h, at.i) * K * V) +
+                         __builtin_amdgcn_readfirstlane(tid >> 6) * KT * 64;
+#pragma unroll
+    for (int m = 0; m < KT; ++m) df[m] = wd[static_cast<uint32_t>(64 * m + (tid & 63))];
+  };
+  auto load_state = [&](const GradItem &at, int h, int tid) {
+    const float4_t *ws = reinterpret_cast<const float4_t *>(p.ws_S + rec(p, at.seq, h, at.i) * K * V) +
+                         __builtin_amdgcn_readfirstlane(tid >> 6) * KT * 64;
+#pragma unroll
+    for (int m = 0; m < KT; ++m) sf[m] = ws[static_cast<uint32_t>(64 * m + (tid & 63))];
+  };
+  auto load_rest = [&](const GradItem &at, int h, int tid) {
+    const long r = rec(p, at.seq, h, at.i), row0 = at.seq.bos + at.i * BC;
+    const int left = at.seq.len - at.i * BC;
+    const v4u32_t *wt = reinterpret_cast<const v4u32_t *>(p.ws_T + r * BC * BC);
+    const v4u32_t *wm = reinterpret_cast<const v4u32_t *>(p.ws_M + r * BC * BC);
+#pragma unroll
+    for (int m = 0; m < BC * BC / 4 / NT; ++m) rt[m] = wt[static_cast<uint32_t>(tid + NT * m)];
+#pragma unroll
+    for (int m = 0; m < BC * BC / 4 / NT; ++m) rm[m] = wm[static_cast<uint32_t>(tid + NT * m)];
+    rv.load(tid, static_cast<const u16 *>(p.v) + (row0 * p.Hv + h) * V, p.Hv * V, left);
+    rd.load(tid, static_cast<const u16 *>(p.dout) + (row0 * p.Hv + h) * V, p.Hv * V, left);
+    rq.load(tid, static_cast<const u16 *>(p.q) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
+    rk.load(tid, static_cast<const u16 *>(p.k) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
+    cv = p.ws_c[r * BC + (tid & 63)];
+    bv = p.ws_beta[r * BC + (tid & 63)];
+    last = p.ws_c[r * BC + BC - 1];
+  };
+  load_adjoint(it, it.block * heads, threadIdx.x);
+  load_state(it, it.block * heads, threadIdx.x);
+  load_rest(it, it.block * heads, threadIdx.x);
   float4_t tq[KTW][2], tk[KTW][2];
 #pragma unroll
   for (int m = 0; m < KTW; ++m) {
 #pragma unroll
     for (int a = 0; a < 2; ++a) tq[m][a] = tk[m][a] = zero4();
   }
-  for (int hh = 0; hh < heads; ++hh) {
-    // The LDS base and the thread index are made opaque in each round: the
+  int hh = 0;  // the value head of the item's group
+  bool more = true;
+  for (bool first = true; more; first = false) {
+    // The LDS base and the thread index are made opaque for each head: the
     // compiler otherwise keeps every phase's addresses and comparisons in
     // registers across the loop (212 spilled registers a lane).
     int base = 0, tid = threadIdx.x;
@@ -125,53 +220,26 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     // partial sums: rows by wave pair (dc, dbeta, dgamma, de), columns by wave parity
     float *prc = sbeta + BC, *prb = prc + COLS * BC, *pdg = prb + COLS * BC, *pde = pdg + COLS * BC;
     float *pcc = pde + COLS * BC, *pcb = pcc + 2 * BC, *sred = pcb + 2 * BC;
-    const int h = blockIdx.y * heads + hh, hk = h / group;
-    const long r = rec(p, seq, h, i);
-    // ---- this head's inputs
-    float4_t sf[KT], df[KT];
-    {
-      const float4_t *ws = reinterpret_cast<const float4_t *>(p.ws_S + r * K * V) + wave * KT * 64 + lane;
-      const float4_t *wd = reinterpret_cast<const float4_t *>(p.ws_dS + r * K * V) + wave * KT * 64 + lane;
-#pragma unroll
-      for (int m = 0; m < KT; ++m) sf[m] = ws[64 * m];
-#pragma unroll
-      for (int m = 0; m < KT; ++m) df[m] = wd[64 * m];
-    }
+    const int h = it.block * heads + hh, t0 = it.i * BC, left = it.seq.len - t0;  // the chunk's tokens: left, if under BC
+    const long row0 = it.seq.bos + t0;
+    // ---- this head's inputs into LDS
     u16 *mt = area, *sv = area + 2 * CC;
-    {
-      RawRows<u16, V, NT> rv, rd;
-      uint4 rt[BC * BC / 4 / NT], rm[BC * BC / 4 / NT];  // the T and M^T pairs: 1,024 pieces of 16 bytes each
-      rd.load(tid, p.dout, seq, t0, p.Hv, h, V);
-      rv.load(tid, p.v, seq, t0, p.Hv, h, V);
-      const uint4 *wt = reinterpret_cast<const uint4 *>(p.ws_T + r * BC * BC);
-      const uint4 *wm = reinterpret_cast<const uint4 *>(p.ws_M + r * BC * BC);
+    if (!first) __syncthreads();  // the previous head's readers of LDS are done
+    rq.put(tid, sq, LK, left);
+    rk.put(tid, sk, LK, left);
+    rd.put(tid, sdo, LV, left);
+    rv.put(tid, sv, LV, left);
 #pragma unroll
-      for (int m = 0; m < BC * BC / 4 / NT; ++m) rt[m] = wt[tid + NT * m];
-#pragma unroll
-      for (int m = 0; m < BC * BC / 4 / NT; ++m) rm[m] = wm[tid + NT * m];
-      const float cv = p.ws_c[r * BC + lane], bv = p.ws_beta[r * BC + lane], last = p.ws_c[r * BC + BC - 1];
-      if (hh > 0) __syncthreads();  // the previous head's readers of LDS are done
-      if (hh == 0) {
-        RawRows<u16, K, NT> rq, rk;
-        rq.load(tid, p.q, seq, t0, p.Hk, hk, K);
-        rk.load(tid, p.k, seq, t0, p.Hk, hk, K);
-        rq.put(tid, sq, LK);
-        rk.put(tid, sk, LK);
-      }
-      rd.put(tid, sdo, LV);
-      rv.put(tid, sv, LV);
-#pragma unroll
-      for (int m = 0; m < BC * BC / 4 / NT; ++m) {
-        const int e = tid + NT * m;
-        *reinterpret_cast<uint4 *>(tp + (e >> 3) * LB + 8 * (e & 7)) = rt[m];  // half e / 512, row (e / 8) & 63
-        *reinterpret_cast<uint4 *>(mt + (e >> 3) * LB + 8 * (e & 7)) = rm[m];
-      }
-      if (tid < BC) {
-        sc[tid] = cv;
-        sgam[tid] = expf(cv);
-        se[tid] = expf(last - cv);
-        sbeta[tid] = bv;
-      }
+    for (int m = 0; m < BC * BC / 4 / NT; ++m) {
+      const int e = tid + NT * m;  // half e / 512, row (e / 8) & 63
+      *reinterpret_cast<v4u32_t *>(tp + (e >> 3) * LB + 8 * (e & 7)) = rt[m];
+      *reinterpret_cast<v4u32_t *>(mt + (e >> 3) * LB + 8 * (e & 7)) = rm[m];
+    }
+    if (tid < BC) {
+      sc[tid] = cv;
+      sgam[tid] = expf(cv);
+      se[tid] = expf(last - cv);
+      sbeta[tid] = bv;
     }
     __syncthreads();
     // ---- chain: this wave's 16 value columns
@@ -184,6 +252,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       split_bf16(sf[m], sh[m], sl[m]);
       split_bf16(df[m], dh[m], dl[m]);
     }
+    keep_order();
     dgc = wave_sum(dgc);
     if (lane == 0) sred[wave] = dgc;
     float4_t du[4];
@@ -204,6 +273,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       split_bf16(x, xh[rt], xl[rt]);
       split_bf16(x * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
       du[rt] = ld4(&se[o]) * kd;
+      keep_order();
     }
     v2u32_t duh[4], dul[4];
     {
@@ -243,6 +313,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       dx *= ld4(&sbeta[16 * rt + 4 * g4]);
       split_bf16(u, uh[rt], ul[rt]);
       split_bf16(dx, dxh[rt], dxl[rt]);
+      keep_order();
     }
     // ---- contractions over the value columns
     u16 *a0 = area, *a1 = area + 2 * TV;
@@ -257,13 +328,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
       for (int m = 0; m < KT; ++m) *reinterpret_cast<v2u32_t *>(a1 + (v0 + c) * LK + 16 * m + 4 * g4) = x[m];
     };
-    float4_t dtb[CTW][2], dm[CTW][2], dk1[KTW][2], dk2[KTW][2], dq0[KTW][2];
+    float4_t dtb[CTW][2], dm[CTW][2], dk1[KTW][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
 #pragma unroll
       for (int m = 0; m < CTW; ++m) dtb[m][a] = dm[m][a] = zero4();
 #pragma unroll
-      for (int m = 0; m < KTW; ++m) dk1[m][a] = dk2[m][a] = dq0[m][a] = zero4();
+      for (int m = 0; m < KTW; ++m) dk1[m][a] = zero4();
     }
     __syncthreads();
     publish(a0, xh, xl);
@@ -333,11 +404,28 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         dk1[m][1] = mfma_bf16(a_1, b, dk1[m][1]);
       }
     }
+    // dK1's row scale, and its part of the decay sums over the keys
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int o = 32 * rp + 16 * a + 4 * g4;
+      const float4_t e4 = ld4(&se[o]);
+      float4_t de = zero4();
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        de += bf16x4_float(L4.tr(sk + (32 * rp + 16 * a) * LK, LK, 16 * (KTW * cp + m))) * dk1[m][a];
+        tk[m][a] += e4 * dk1[m][a];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float y = group_sum(de[e], 16);
+        if (c == 0) pde[cp * BC + o + e] = y;
+      }
+    }
     __syncthreads();
     publish(a0, dxh, dxl);
     publish_state(sh);
     {  // dv = dX, rounded (its high half): this wave's columns, four a lane and token
-      u16 *dv = static_cast<u16 *>(p.dv) + ((seq.bos + t0) * p.Hv + h) * V + v0;
+      u16 *dv = static_cast<u16 *>(p.dv) + (row0 * p.Hv + h) * V + v0;
       const uint32_t stride = p.Hv * V;
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
@@ -346,6 +434,12 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    float4_t dk2[KTW][2], dq0[KTW][2];
+#pragma unroll
+    for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) dk2[m][a] = dq0[m][a] = zero4();
+    }
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {  // dK2 = dX S^T, dQ0 = dO S^T, the high half of S
       bh8_t od[2], ah[2], al[2];
@@ -387,29 +481,25 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         }
       }
     }
-    // ---- the row scales, and the decay sums over the keys
+    // ---- the other row scales and decay sums
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
       const int o = 32 * rp + 16 * a + 4 * g4;
-      const float4_t gam = ld4(&sgam[o]), e4 = ld4(&se[o]);
-      float4_t dgam = zero4(), de = zero4();
+      const float4_t gam = ld4(&sgam[o]);
+      float4_t dgam = zero4();
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
         const int col = 16 * (KTW * cp + m);
         const float4_t kx = bf16x4_float(L4.tr(sk + (32 * rp + 16 * a) * LK, LK, col));
         const float4_t qx = bf16x4_float(L4.tr(sq + (32 * rp + 16 * a) * LK, LK, col));
         dgam += p.scale * (qx * dq0[m][a]) - kx * dk2[m][a];
-        de += kx * dk1[m][a];
         tq[m][a] += dq0[m][a] * (gam * p.scale);
-        tk[m][a] += e4 * dk1[m][a] - gam * dk2[m][a];
+        tk[m][a] -= gam * dk2[m][a];
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = group_sum(dgam[e], 16), y = group_sum(de[e], 16);
-        if (c == 0) {
-          pdg[cp * BC + o + e] = x;
-          pde[cp * BC + o + e] = y;
-        }
+        const float x = group_sum(dgam[e], 16);
+        if (c == 0) pdg[cp * BC + o + e] = x;
       }
     }
     __syncthreads();  // the stages' readers are done: the area now holds the C x C pairs
@@ -520,36 +610,42 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    // The next head's inputs (the same head's again if it is the last: a load
+    // left out on one path would keep the old values alive to the end of the
+    // loop on every path). Earlier they do not fit into the registers: issued
+    // among the stages they were spilled as they arrived.
+    const bool last_head = hh + 1 == heads;
+    next = it;
+    if (last_head) more = grad_item(p, it.item + gridDim.x, gridDim.x, items, chunks, blocks, next);
+    if (!more) next = it;
+    const int nh = next.block * heads + (last_head ? 0 : hh + 1);
+    load_adjoint(next, nh, tid);
+    load_state(next, nh, tid);
+    load_rest(next, nh, tid);
     // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + H K + H^T K
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      bh8_t a1h[2], a1l[2], a3h[2], a3l[2], t1h[2], t1l[2], t3h[2], t3l[2];
+      keep_order();
+      bh8_t kf[KTW], qf[KTW];
+#pragma unroll
+      for (int m = 0; m < KTW; ++m) {
+        kf[m] = L4.cols(sk, LK, kb, 16 * (KTW * cp + m));
+        qf[m] = L4.cols(sq, LK, kb, 16 * (KTW * cp + m));
+      }
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
         const int row0 = 32 * rp + 16 * a;
-        a1h[a] = L4.cols(b1t, LB, kb, row0);
-        a1l[a] = L4.cols(b1t + CC, LB, kb, row0);
-        a3h[a] = L4.cols(b3t, LB, kb, row0);
-        a3l[a] = L4.cols(b3t + CC, LB, kb, row0);
-        t1h[a] = L4.rows(b1t, LB, row0, kb);
-        t1l[a] = L4.rows(b1t + CC, LB, row0, kb);
-        t3h[a] = L4.rows(b3t, LB, row0, kb);
-        t3l[a] = L4.rows(b3t + CC, LB, row0, kb);
-      }
+        auto product = [&](float4_t (&x)[KTW][2], bh8_t hi, bh8_t lo, const bh8_t (&b)[KTW]) {
 #pragma unroll
-      for (int m = 0; m < KTW; ++m) {
-        const bh8_t kf = L4.cols(sk, LK, kb, 16 * (KTW * cp + m)), qf = L4.cols(sq, LK, kb, 16 * (KTW * cp + m));
+          for (int m = 0; m < KTW; ++m) x[m][a] = mfma_bf16(hi, b[m], x[m][a]);
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          tq[m][a] = mfma_bf16(a1h[a], kf, tq[m][a]);
-          tk[m][a] = mfma_bf16(t1h[a], qf, tk[m][a]);
-          tq[m][a] = mfma_bf16(a1l[a], kf, tq[m][a]);
-          tk[m][a] = mfma_bf16(t1l[a], qf, tk[m][a]);
-          tk[m][a] = mfma_bf16(a3h[a], kf, tk[m][a]);
-          tk[m][a] = mfma_bf16(a3l[a], kf, tk[m][a]);
-          tk[m][a] = mfma_bf16(t3h[a], kf, tk[m][a]);
-          tk[m][a] = mfma_bf16(t3l[a], kf, tk[m][a]);
-        }
+          for (int m = 0; m < KTW; ++m) x[m][a] = mfma_bf16(lo, b[m], x[m][a]);
+        };
+        product(tq, L4.cols(b1t, LB, kb, row0), L4.cols(b1t + CC, LB, kb, row0), kf);
+        product(tk, L4.rows(b1t, LB, row0, kb), L4.rows(b1t + CC, LB, row0, kb), qf);
+        product(tk, L4.cols(b3t, LB, kb, row0), L4.cols(b3t + CC, LB, kb, row0), kf);
+        product(tk, L4.rows(b3t, LB, row0, kb), L4.rows(b3t + CC, LB, row0, kb), kf);
+        keep_order();
       }
     }
     if (wave == 0) {  // dc -> dg = reverse cumulative sum within the chunk
@@ -572,60 +668,65 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         const float y = __shfl_down(dcv, off, 64);
         if (lane + off < 64) dcv += y;
       }
-      if (t0 + t < seq.len) {
-        const long o = (seq.bos + t0 + t) * p.Hv + h;
+      if (t < left) {
+        const long o = (row0 + t) * p.Hv + h;
         p.dg[o] = dcv;
         store_elem(p.dbeta, o, p.beta_dtype, dbt);
       }
     }
-  }
-  // dq, dk: summed over the key head's value heads, or (one head a workgroup
-  // of several) per value head in float32 for the reduction kernel
-  const bool direct = heads == group;
-  const int h0 = blockIdx.y * heads, c = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rp = wave & 1, cp = wave >> 1;
-  if (direct) {
-    // each tile through LDS, transposed (this wave writes and reads it), for
-    // pieces of four keys a lane and token
-    __syncthreads();  // the last head's readers of LDS are done
-    const Lane L4{c, g4};
-    const long base = ((seq.bos + t0) * p.Hk + h0 / group) * K;
-    const uint32_t stride = p.Hk * K;
-    u16 *buf = reinterpret_cast<u16 *>(lds) + wave * 16 * LB;
-    auto out = [&](void *dst, const float4_t (&x)[KTW][2]) {
+    if (last_head) {
+      // dq, dk: summed over the key head's value heads, or (one head an item of
+      // several) per value head in float32 for the reduction kernel
+      if (heads == group) {
+        // each tile through LDS, transposed (this wave writes and reads it), for
+        // pieces of four keys a lane and token
+        __syncthreads();  // this head's readers of sq and sk are done
+        const long base = (row0 * p.Hk + h / group) * K;
+        const uint32_t stride = p.Hk * K;
+        u16 *buf = sq + wave * 16 * LB;
+        auto out = [&](void *dst, const float4_t (&x)[KTW][2]) {
+#pragma unroll
+          for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+              *reinterpret_cast<v2u32_t *>(buf + c * LB + 16 * a + 4 * g4) =
+                  __builtin_bit_cast(v2u32_t, __builtin_convertvector(x[m][a], bf16x4_t));
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+              const v2u32_t y = __builtin_bit_cast(v2u32_t, L4.tr(buf, LB, 16 * a));
+              const int t = 32 * rp + 16 * a + c;
+              u16 *row = static_cast<u16 *>(dst) + base + 16 * (KTW * cp + m);
+              if (t < left) *reinterpret_cast<v2u32_t *>(row + t * stride + 4 * g4) = y;
+            }
+          }
+        };
+        out(p.dq, tq);
+        out(p.dk, tk);
+      } else {
+        const long base = (row0 * p.Hv + h) * K;
+#pragma unroll
+        for (int m = 0; m < KTW; ++m) {
+#pragma unroll
+          for (int a = 0; a < 2; ++a) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int t = 32 * rp + 16 * a + 4 * g4 + e, kk = 16 * (KTW * cp + m) + c;
+              if (t >= left) continue;
+              const uint32_t off = t * static_cast<uint32_t>(p.Hv * K) + kk;
+              (p.ws_dq + base)[off] = tq[m][a][e];
+              (p.ws_dk + base)[off] = tk[m][a][e];
+            }
+          }
+        }
+      }
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          *reinterpret_cast<v2u32_t *>(buf + c * LB + 16 * a + 4 * g4) =
-              __builtin_bit_cast(v2u32_t, __builtin_convertvector(x[m][a], bf16x4_t));
-        }
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          const v2u32_t y = __builtin_bit_cast(v2u32_t, L4.tr(buf, LB, 16 * a));
-          const int t = 32 * rp + 16 * a + c;
-          u16 *row = static_cast<u16 *>(dst) + base + 16 * (KTW * cp + m);
-          if (t < left) *reinterpret_cast<v2u32_t *>(row + t * stride + 4 * g4) = y;
-        }
-      }
-    };
-    out(p.dq, tq);
-    out(p.dk, tk);
-    return;
-  }
-#pragma unroll
-  for (int m = 0; m < KTW; ++m) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 32 * rp + 16 * a + 4 * g4 + e, kk = 16 * (KTW * cp + m) + c;
-        if (t >= left) continue;
-        const long base = ((seq.bos + t0) * p.Hv + h0) * K;
-        const uint32_t off = t * static_cast<uint32_t>(p.Hv * K) + kk;
-        (p.ws_dq + base)[off] = tq[m][a][e];
-        (p.ws_dk + base)[off] = tk[m][a][e];
+        for (int a = 0; a < 2; ++a) tq[m][a] = tk[m][a] = zero4();
       }
     }
+    it = next;
+    hh = last_head ? 0 : hh + 1;
   }
 }

@@ -266,8 +266,6 @@ struct ScanLoad {
 // the products (and the splits) that precede it, which hide their latency. The
 // compiler left to itself reads each fragment just before its use (some sixty
 // exposed waits a step: 1,681 us of scans at 1 x 32,768 tokens of 32 heads).
-__device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0); }
-
 // Key tiles' operands of the contraction over tokens 32 kb ..
 template <int KT>
 __device__ __forceinline__ void read_cols(const Lane &ln, const u16 *m, int ld, int kb, bh8_t (&a)[KT]) {
