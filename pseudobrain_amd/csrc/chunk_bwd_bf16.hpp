@@ -21,45 +21,76 @@
 //
 // Row sums that would need K S, K dS' or Q S again come from the K-wide
 // products: sum_v (K dS' o U)_t = sum_k (K o dK1)_t, likewise with dX and dQ0.
-// LDS: 150 KiB at K = V = 128, so one workgroup a CU, eight waves.
+// LDS: 134 KiB at K = V = 128, so one workgroup a CU, eight waves.
 //
 // Contraction slots: the B operand of a 32-row step kb made of two
 // accumulator tiles holds, in lane (c, g), rows 32 kb + 4 g + j (j < 4) and
 // 32 kb + 16 + 4 g + j - 4 of column c; A operands are read in that order (two
 // 8-byte pieces of a row, or two transposing reads).
 
-// The operand reads of one lane (c, g). A struct rather than functions of
-// threadIdx.x, so that a kernel can make its lane opaque to the compiler where
-// addresses and comparisons must not be kept across a loop.
+// LDS arrays are row-major without padding, W elements a row, the 16-byte units
+// of row r swizzled: unit u stands at u ^ unit_swz<W>(r). Both kinds of operand
+// read are then free of bank conflicts: 32 lanes of a transposing read take 32
+// bytes of 8 rows, 32 lanes of a row read 16 bytes of 16 rows, and either way
+// the 16 units differ modulo 256 bytes. (With rows padded by 16 bytes the
+// transposing reads conflicted two ways, with 32 the row reads: 46% of the
+// gradient kernel's LDS cycles.)
+template <int W>
+__device__ __forceinline__ constexpr int unit_swz(int r) {
+  static_assert(W == 128 || W == 64 || W == 32, "row widths");
+  return W == 128 ? 2 * (r & 7) + ((r >> 3) & 1)
+         : W == 64 ? 2 * ((r >> 1) & 3) + ((r >> 3) & 1)
+                   : 2 * ((r >> 2) & 1);  // (transposing reads only)
+}
+// Offset of 16-byte unit u of row r.
+template <int W>
+__device__ __forceinline__ constexpr int unit_at(int r, int u) {
+  return r * W + 8 * (u ^ unit_swz<W>(r));
+}
+
+// The operand reads of one lane (c, g); row0, col0 multiples of 16, kb steps of
+// 32. A struct rather than functions of threadIdx.x, so that a kernel can make
+// its lane opaque to the compiler where addresses and comparisons must not be
+// kept across a loop.
 struct Lane {
   int c, g;
 
-  // Four rows 4 g .. of column col0 + c of a row-major bf16 array (ds_read_tr16).
-  __device__ __forceinline__ bw_i16x4_t tr(const u16 *m, int ld, int col0) const {
-    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) bw_i16x4_t *)(m + (4 * g + (c >> 2)) * ld + col0 + 4 * (c & 3)));
+  // Element (row0 + c, col0 + 4 g): four of a row, 8 bytes.
+  template <int W>
+  __device__ __forceinline__ int four(int row0, int col0) const {
+    return row0 * W + ((unit_at<W>(c, g >> 1) + 4 * (g & 1)) ^ col0);
   }
-  // Rows row0 + c of a row-major bf16 array as the operand of step kb.
-  __device__ __forceinline__ bh8_t rows(const u16 *m, int ld, int row0, int kb) const {
-    const u16 *a = m + (row0 + c) * ld + 32 * kb + 4 * g;
-    const v2u32_t x = *reinterpret_cast<const v2u32_t *>(a), y = *reinterpret_cast<const v2u32_t *>(a + 16);
+  // Four rows row0 + 4 g .. of column col0 + c (ds_read_tr16).
+  template <int W>
+  __device__ __forceinline__ bw_i16x4_t tr(const u16 *m, int row0, int col0) const {
+    const int at = (unit_at<W>(4 * g + (c >> 2), (c >> 1) & 1) + 4 * (c & 1)) ^ col0;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) bw_i16x4_t *)(m + row0 * W + at));
+  }
+  // Rows row0 + c as the operand of step kb.
+  template <int W>
+  __device__ __forceinline__ bh8_t rows(const u16 *m, int row0, int kb) const {
+    const v2u32_t x = *reinterpret_cast<const v2u32_t *>(m + four<W>(row0, 32 * kb));
+    const v2u32_t y = *reinterpret_cast<const v2u32_t *>(m + four<W>(row0, 32 * kb + 16));
     return __builtin_bit_cast(bh8_t, v4u32_t{x[0], x[1], y[0], y[1]});
   }
   // The same with the slots in order (both operands read this way).
-  __device__ __forceinline__ bh8_t rows16(const u16 *m, int ld, int row0, int kb) const {
-    return *reinterpret_cast<const bh8_t *>(m + (row0 + c) * ld + 32 * kb + 8 * g);
+  template <int W>
+  __device__ __forceinline__ bh8_t rows16(const u16 *m, int row0, int kb) const {
+    return *reinterpret_cast<const bh8_t *>(m + row0 * W + (unit_at<W>(c, g) ^ (32 * kb)));
   }
   // Columns col0 + c, contraction over the array's rows 32 kb ..
-  __device__ __forceinline__ bh8_t cols(const u16 *m, int ld, int kb, int col0) const {
-    const bw_i16x4_t x = tr(m + 32 * kb * ld, ld, col0), y = tr(m + (32 * kb + 16) * ld, ld, col0);
+  template <int W>
+  __device__ __forceinline__ bh8_t cols(const u16 *m, int kb, int col0) const {
+    const bw_i16x4_t x = tr<W>(m, 32 * kb, col0), y = tr<W>(m, 32 * kb + 16, col0);
     return __builtin_bit_cast(bh8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
   }
   // Rows a0 .. of a times rows b0 .. of b, over KD columns.
   template <int KD>
-  __device__ __forceinline__ float4_t rows_rows(const u16 *a, const u16 *b, int ld, int a0, int b0) const {
+  __device__ __forceinline__ float4_t rows_rows(const u16 *a, const u16 *b, int a0, int b0) const {
     float4_t acc = zero4();
 #pragma unroll
-    for (int kb = 0; kb < KD / 32; ++kb) acc = mfma_bf16(rows16(a, ld, a0, kb), rows16(b, ld, b0, kb), acc);
+    for (int kb = 0; kb < KD / 32; ++kb) acc = mfma_bf16(rows16<KD>(a, a0, kb), rows16<KD>(b, b0, kb), acc);
     return acc;
   }
 };
@@ -81,15 +112,15 @@ __device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0)
 template <int K, int V>
 struct GradLds {
   static constexpr int NW = V / 16, NT = 64 * NW, COLS = NW / 2;  // waves; wave pairs
-  static constexpr int LK = K + 8, LV = V + 8, LB = BC + 8;       // row strides (elements)
-  static constexpr int CC = BC * LB;                              // one 64 x 64 half
-  static constexpr int TV = V * LB;                               // one V x 64 half
+  static constexpr int CC = BC * BC;                              // one 64 x 64 half
+  static constexpr int TV = V * BC;                               // one V x 64 half
   // the shared area: M^T pair and V rows (chain); X^T and dU^T pairs; the U^T
   // or dX^T pair and one state half; four C x C pairs
-  static constexpr int AREA = 4 * TV > 8 * CC ? 4 * TV : (2 * TV + V * LK > 8 * CC ? 2 * TV + V * LK : 8 * CC);
-  static_assert(2 * CC + BC * LV <= AREA && 2 * TV + V * LK <= AREA, "the area's uses");
+  static constexpr int USED = 4 * TV > 2 * TV + V * K ? 4 * TV : 2 * TV + V * K,
+                       AREA = USED > 8 * CC ? USED : 8 * CC;
+  static_assert(2 * CC + BC * V <= AREA && 2 * TV + V * K <= AREA, "the area's uses");
   static constexpr int FLOATS = 4 * BC + 4 * COLS * BC + 4 * BC + 16;
-  static constexpr size_t BYTES = sizeof(u16) * (2 * BC * LK + BC * LV + 2 * CC + AREA) + sizeof(float) * FLOATS;
+  static constexpr size_t BYTES = sizeof(u16) * (2 * BC * K + BC * V + 2 * CC + AREA) + sizeof(float) * FLOATS;
 };
 
 // Rows 0 .. 63 from a uniform base (the chunk's first row) in registers, to be
@@ -109,7 +140,11 @@ struct RowsAhead {
       raw[m] = *reinterpret_cast<const v4u32_t *>(base + off);
     }
   }
-  __device__ __forceinline__ void put(int tid, u16 *dst, int ld, int left) {
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int m = 0; m < PER; ++m) raw[m] = v4u32_t{0u, 0u, 0u, 0u};
+  }
+  __device__ __forceinline__ void put(int tid, u16 *dst, int left) {
     if (left < BC) {
 #pragma unroll
       for (int m = 0; m < PER; ++m) {
@@ -119,7 +154,7 @@ struct RowsAhead {
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
       const int e = tid + NT * m;
-      *reinterpret_cast<v4u32_t *>(dst + (e / PPR) * ld + (e % PPR) * 8) = raw[m];
+      *reinterpret_cast<v4u32_t *>(dst + unit_at<W>(e / PPR, e % PPR)) = raw[m];
     }
   }
 };
@@ -146,7 +181,7 @@ __device__ __forceinline__ bool grad_item(const BwdParams &p, unsigned item, uns
 template <int K, int V>
 __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int heads) {
   using L = GradLds<K, V>;
-  constexpr int NW = L::NW, NT = L::NT, COLS = L::COLS, LK = L::LK, LV = L::LV, LB = L::LB, CC = L::CC, TV = L::TV;
+  constexpr int NW = L::NW, NT = L::NT, COLS = L::COLS, CC = L::CC, TV = L::TV;
   constexpr int KT = K / 16, KB = K / 32, VB = V / 32;
   constexpr int KTW = KT / COLS, CTW = 4 / COLS;  // key tiles, C x C column tiles of a wave
   extern __shared__ __align__(16) float lds[];
@@ -176,7 +211,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
     for (int m = 0; m < KT; ++m) sf[m] = ws[static_cast<uint32_t>(64 * m + (tid & 63))];
   };
-  auto load_rest = [&](const GradItem &at, int h, int tid) {
+  auto load_rest = [&](const GradItem &at, int h, bool keys, int tid) {
     const long r = rec(p, at.seq, h, at.i), row0 = at.seq.bos + at.i * BC;
     const int left = at.seq.len - at.i * BC;
     const v4u32_t *wt = reinterpret_cast<const v4u32_t *>(p.ws_T + r * BC * BC);
@@ -187,15 +222,20 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     for (int m = 0; m < BC * BC / 4 / NT; ++m) rm[m] = wm[static_cast<uint32_t>(tid + NT * m)];
     rv.load(tid, static_cast<const u16 *>(p.v) + (row0 * p.Hv + h) * V, p.Hv * V, left);
     rd.load(tid, static_cast<const u16 *>(p.dout) + (row0 * p.Hv + h) * V, p.Hv * V, left);
-    rq.load(tid, static_cast<const u16 *>(p.q) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
-    rk.load(tid, static_cast<const u16 *>(p.k) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
+    if (keys) {
+      rq.load(tid, static_cast<const u16 *>(p.q) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
+      rk.load(tid, static_cast<const u16 *>(p.k) + (row0 * p.Hk + h / group) * K, p.Hk * K, left);
+    } else {  // (a value on every path: see the call)
+      rq.clear();
+      rk.clear();
+    }
     cv = p.ws_c[r * BC + (tid & 63)];
     bv = p.ws_beta[r * BC + (tid & 63)];
     last = p.ws_c[r * BC + BC - 1];
   };
   load_adjoint(it, it.block * heads, threadIdx.x);
   load_state(it, it.block * heads, threadIdx.x);
-  load_rest(it, it.block * heads, threadIdx.x);
+  load_rest(it, it.block * heads, true, threadIdx.x);
   float4_t tq[KTW][2], tk[KTW][2];
 #pragma unroll
   for (int m = 0; m < KTW; ++m) {
@@ -211,10 +251,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     int base = 0, tid = threadIdx.x;
     asm volatile("" : "+s"(base), "+v"(tid));
     const int lane = tid & 63, c = lane & 15, g4 = lane >> 4;
-    const Lane L4{c, g4};
+    Lane L4{c, g4};
+    // makes the operand addresses of the phase before unknown to the compiler,
+    // which would keep them in registers for the next
+    auto renew = [&] { asm volatile("" : "+v"(L4.c), "+v"(L4.g)); };
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), v0 = 16 * wave;
     const int rp = wave & 1, cp = wave >> 1;  // row tiles 2 rp, 2 rp + 1; column (key) tiles of pair cp
-    u16 *sq = reinterpret_cast<u16 *>(lds + base), *sk = sq + BC * LK, *sdo = sk + BC * LK, *tp = sdo + BC * LV,
+    u16 *sq = reinterpret_cast<u16 *>(lds + base), *sk = sq + BC * K, *sdo = sk + BC * K, *tp = sdo + BC * V,
         *area = tp + 2 * CC;
     float *sc = reinterpret_cast<float *>(area + L::AREA), *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
     // partial sums: rows by wave pair (dc, dbeta, dgamma, de), columns by wave parity
@@ -225,15 +268,17 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     // ---- this head's inputs into LDS
     u16 *mt = area, *sv = area + 2 * CC;
     if (!first) __syncthreads();  // the previous head's readers of LDS are done
-    rq.put(tid, sq, LK, left);
-    rk.put(tid, sk, LK, left);
-    rd.put(tid, sdo, LV, left);
-    rv.put(tid, sv, LV, left);
+    if (hh == 0) {
+      rq.put(tid, sq, left);
+      rk.put(tid, sk, left);
+    }
+    rd.put(tid, sdo, left);
+    rv.put(tid, sv, left);
 #pragma unroll
     for (int m = 0; m < BC * BC / 4 / NT; ++m) {
       const int e = tid + NT * m;  // half e / 512, row (e / 8) & 63
-      *reinterpret_cast<v4u32_t *>(tp + (e >> 3) * LB + 8 * (e & 7)) = rt[m];
-      *reinterpret_cast<v4u32_t *>(mt + (e >> 3) * LB + 8 * (e & 7)) = rm[m];
+      *reinterpret_cast<v4u32_t *>(tp + unit_at<BC>(e >> 3, e & 7)) = rt[m];
+      *reinterpret_cast<v4u32_t *>(mt + unit_at<BC>(e >> 3, e & 7)) = rm[m];
     }
     if (tid < BC) {
       sc[tid] = cv;
@@ -262,14 +307,14 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       float4_t ks = zero4(), kd = zero4();
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-        const bh8_t a = L4.rows(sk, LK, 16 * rt, kb);
+        const bh8_t a = L4.rows<K>(sk, 16 * rt, kb);
         ks = mfma_bf16(a, frag_pair(sh[2 * kb], sh[2 * kb + 1]), ks);
         kd = mfma_bf16(a, frag_pair(dh[2 * kb], dh[2 * kb + 1]), kd);
         ks = mfma_bf16(a, frag_pair(sl[2 * kb], sl[2 * kb + 1]), ks);
         kd = mfma_bf16(a, frag_pair(dl[2 * kb], dl[2 * kb + 1]), kd);
       }
       const int o = 16 * rt + 4 * g4;
-      const float4_t x = bf16x4_float(L4.tr(sv + 16 * rt * LV, LV, v0)) - ld4(&sgam[o]) * ks;
+      const float4_t x = bf16x4_float(L4.tr<V>(sv, 16 * rt, v0)) - ld4(&sgam[o]) * ks;
       split_bf16(x, xh[rt], xl[rt]);
       split_bf16(x * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
       du[rt] = ld4(&se[o]) * kd;
@@ -279,13 +324,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     {
       bh8_t dof[2];
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) dof[kb] = L4.cols(sdo, LV, kb, v0);
+      for (int kb = 0; kb < 2; ++kb) dof[kb] = L4.cols<V>(sdo, kb, v0);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
 #pragma unroll
         for (int kb = rt >> 1; kb < 2; ++kb) {  // t >= s
-          du[rt] = mfma_bf16(L4.rows(mt, LB, 16 * rt, kb), dof[kb], du[rt]);
-          du[rt] = mfma_bf16(L4.rows(mt + CC, LB, 16 * rt, kb), dof[kb], du[rt]);
+          du[rt] = mfma_bf16(L4.rows<BC>(mt, 16 * rt, kb), dof[kb], du[rt]);
+          du[rt] = mfma_bf16(L4.rows<BC>(mt + CC, 16 * rt, kb), dof[kb], du[rt]);
         }
         split_bf16(du[rt], duh[rt], dul[rt]);
       }
@@ -296,7 +341,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       float4_t u = zero4(), dx = zero4();
 #pragma unroll
       for (int kb = 0; kb <= rt >> 1; ++kb) {  // U = T (beta X), s <= t
-        const bh8_t th = L4.rows(tp, LB, 16 * rt, kb), tl = L4.rows(tp + CC, LB, 16 * rt, kb);
+        const bh8_t th = L4.rows<BC>(tp, 16 * rt, kb), tl = L4.rows<BC>(tp + CC, 16 * rt, kb);
         const bh8_t bh = frag_pair(bxh[2 * kb], bxh[2 * kb + 1]), bl = frag_pair(bxl[2 * kb], bxl[2 * kb + 1]);
         u = mfma_bf16(th, bh, u);
         u = mfma_bf16(th, bl, u);
@@ -304,7 +349,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
 #pragma unroll
       for (int kb = rt >> 1; kb < 2; ++kb) {  // dX = beta T^T dU, t >= s
-        const bh8_t th = L4.cols(tp, LB, kb, 16 * rt), tl = L4.cols(tp + CC, LB, kb, 16 * rt);
+        const bh8_t th = L4.cols<BC>(tp, kb, 16 * rt), tl = L4.cols<BC>(tp + CC, kb, 16 * rt);
         const bh8_t bh = frag_pair(duh[2 * kb], duh[2 * kb + 1]), bl = frag_pair(dul[2 * kb], dul[2 * kb + 1]);
         dx = mfma_bf16(th, bh, dx);
         dx = mfma_bf16(th, bl, dx);
@@ -315,18 +360,19 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       split_bf16(dx, dxh[rt], dxl[rt]);
       keep_order();
     }
+    renew();
     // ---- contractions over the value columns
     u16 *a0 = area, *a1 = area + 2 * TV;
     auto publish = [&](u16 *m, const v2u32_t (&hi)[4], const v2u32_t (&lo)[4]) {  // [V][64] transposed pair
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
-        *reinterpret_cast<v2u32_t *>(m + (v0 + c) * LB + 16 * rt + 4 * g4) = hi[rt];
-        *reinterpret_cast<v2u32_t *>(m + TV + (v0 + c) * LB + 16 * rt + 4 * g4) = lo[rt];
+        *reinterpret_cast<v2u32_t *>(m + L4.four<BC>(v0, 16 * rt)) = hi[rt];
+        *reinterpret_cast<v2u32_t *>(m + TV + L4.four<BC>(v0, 16 * rt)) = lo[rt];
       }
     };
     auto publish_state = [&](const v2u32_t (&x)[KT]) {  // [V][K] transposed half
 #pragma unroll
-      for (int m = 0; m < KT; ++m) *reinterpret_cast<v2u32_t *>(a1 + (v0 + c) * LK + 16 * m + 4 * g4) = x[m];
+      for (int m = 0; m < KT; ++m) *reinterpret_cast<v2u32_t *>(a1 + L4.four<K>(v0, 16 * m)) = x[m];
     };
     float4_t dtb[CTW][2], dm[CTW][2], dk1[KTW][2];
 #pragma unroll
@@ -345,12 +391,12 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       bh8_t ah[2], al[2];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        ah[a] = L4.cols(a1, LB, kb, 32 * rp + 16 * a);
-        al[a] = L4.cols(a1 + TV, LB, kb, 32 * rp + 16 * a);
+        ah[a] = L4.cols<BC>(a1, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols<BC>(a1 + TV, kb, 32 * rp + 16 * a);
       }
 #pragma unroll
       for (int m = 0; m < CTW; ++m) {
-        const bh8_t bh = L4.cols(a0, LB, kb, 16 * (CTW * cp + m)), bl = L4.cols(a0 + TV, LB, kb, 16 * (CTW * cp + m));
+        const bh8_t bh = L4.cols<BC>(a0, kb, 16 * (CTW * cp + m)), bl = L4.cols<BC>(a0 + TV, kb, 16 * (CTW * cp + m));
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           dtb[m][a] = mfma_bf16(ah[a], bh, dtb[m][a]);
@@ -360,6 +406,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     publish(a0, uh, ul);
     publish_state(dh);
     __syncthreads();
@@ -368,13 +415,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       bh8_t od[2], ah[2], al[2];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
-        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
-        al[a] = L4.cols(a0 + TV, LB, kb, 32 * rp + 16 * a);
+        od[a] = L4.rows<V>(sdo, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols<BC>(a0, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols<BC>(a0 + TV, kb, 32 * rp + 16 * a);
       }
 #pragma unroll
       for (int m = 0; m < CTW; ++m) {
-        const bh8_t bh = L4.cols(a0, LB, kb, 16 * (CTW * cp + m)), bl = L4.cols(a0 + TV, LB, kb, 16 * (CTW * cp + m));
+        const bh8_t bh = L4.cols<BC>(a0, kb, 16 * (CTW * cp + m)), bl = L4.cols<BC>(a0 + TV, kb, 16 * (CTW * cp + m));
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           dm[m][a] = mfma_bf16(od[a], bh, dm[m][a]);
@@ -383,7 +430,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+        const bh8_t b = L4.cols<K>(a1, kb, 16 * (KTW * cp + m));
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           dk1[m][a] = mfma_bf16(ah[a], b, dk1[m][a]);
@@ -392,18 +439,20 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     publish_state(dl);
     __syncthreads();
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {  // dK1: the low half of dS'
-      const bh8_t a_0 = L4.cols(a0, LB, kb, 32 * rp), a_1 = L4.cols(a0, LB, kb, 32 * rp + 16);
+      const bh8_t a_0 = L4.cols<BC>(a0, kb, 32 * rp), a_1 = L4.cols<BC>(a0, kb, 32 * rp + 16);
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+        const bh8_t b = L4.cols<K>(a1, kb, 16 * (KTW * cp + m));
         dk1[m][0] = mfma_bf16(a_0, b, dk1[m][0]);
         dk1[m][1] = mfma_bf16(a_1, b, dk1[m][1]);
       }
     }
+    renew();
     // dK1's row scale, and its part of the decay sums over the keys
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -412,7 +461,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       float4_t de = zero4();
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        de += bf16x4_float(L4.tr(sk + (32 * rp + 16 * a) * LK, LK, 16 * (KTW * cp + m))) * dk1[m][a];
+        de += bf16x4_float(L4.tr<K>(sk, 32 * rp + 16 * a, 16 * (KTW * cp + m))) * dk1[m][a];
         tk[m][a] += e4 * dk1[m][a];
       }
 #pragma unroll
@@ -422,6 +471,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     publish(a0, dxh, dxl);
     publish_state(sh);
     {  // dv = dX, rounded (its high half): this wave's columns, four a lane and token
@@ -429,7 +479,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       const uint32_t stride = p.Hv * V;
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
-        const v2u32_t x = __builtin_bit_cast(v2u32_t, L4.tr(a0 + v0 * LB, LB, 16 * rt));
+        const v2u32_t x = __builtin_bit_cast(v2u32_t, L4.tr<BC>(a0, v0, 16 * rt));
         if (16 * rt + c < left) *reinterpret_cast<v2u32_t *>(dv + (16 * rt + c) * stride + 4 * g4) = x;
       }
     }
@@ -445,13 +495,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       bh8_t od[2], ah[2], al[2];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
-        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
-        al[a] = L4.cols(a0 + TV, LB, kb, 32 * rp + 16 * a);
+        od[a] = L4.rows<V>(sdo, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols<BC>(a0, kb, 32 * rp + 16 * a);
+        al[a] = L4.cols<BC>(a0 + TV, kb, 32 * rp + 16 * a);
       }
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+        const bh8_t b = L4.cols<K>(a1, kb, 16 * (KTW * cp + m));
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           dk2[m][a] = mfma_bf16(ah[a], b, dk2[m][a]);
@@ -461,6 +511,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     publish_state(sl);
     __syncthreads();
 #pragma unroll
@@ -468,12 +519,12 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       bh8_t od[2], ah[2];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        od[a] = L4.rows(sdo, LV, 32 * rp + 16 * a, kb);
-        ah[a] = L4.cols(a0, LB, kb, 32 * rp + 16 * a);
+        od[a] = L4.rows<V>(sdo, 32 * rp + 16 * a, kb);
+        ah[a] = L4.cols<BC>(a0, kb, 32 * rp + 16 * a);
       }
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        const bh8_t b = L4.cols(a1, LK, kb, 16 * (KTW * cp + m));
+        const bh8_t b = L4.cols<K>(a1, kb, 16 * (KTW * cp + m));
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           dk2[m][a] = mfma_bf16(ah[a], b, dk2[m][a]);
@@ -481,6 +532,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         }
       }
     }
+    renew();
     // ---- the other row scales and decay sums
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -490,8 +542,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
         const int col = 16 * (KTW * cp + m);
-        const float4_t kx = bf16x4_float(L4.tr(sk + (32 * rp + 16 * a) * LK, LK, col));
-        const float4_t qx = bf16x4_float(L4.tr(sq + (32 * rp + 16 * a) * LK, LK, col));
+        const float4_t kx = bf16x4_float(L4.tr<K>(sk, 32 * rp + 16 * a, col));
+        const float4_t qx = bf16x4_float(L4.tr<K>(sq, 32 * rp + 16 * a, col));
         dgam += p.scale * (qx * dq0[m][a]) - kx * dk2[m][a];
         tq[m][a] += dq0[m][a] * (gam * p.scale);
         tk[m][a] -= gam * dk2[m][a];
@@ -503,13 +555,14 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();  // the stages' readers are done: the area now holds the C x C pairs
+    renew();
     // The C x C matrices as transposed pairs [column][row]: a lane's four rows
     // of a column are one 8-byte write a half.
     u16 *b1t = area, *b2t = b1t + 2 * CC, *b3t = b2t + 2 * CC, *b4t = b3t + 2 * CC;
     auto put_t = [&](u16 *m, int row0, int col0, float4_t x) {
       v2u32_t hi, lo;
       split_bf16(x, hi, lo);
-      u16 *at = m + (col0 + c) * LB + row0 + 4 * g4;
+      u16 *at = m + L4.four<BC>(col0, row0);
       *reinterpret_cast<v2u32_t *>(at) = hi;
       *reinterpret_cast<v2u32_t *>(at + CC) = lo;
     };
@@ -527,8 +580,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       for (int m = 0; m < CTW; ++m) {
         const int col0 = 16 * (CTW * cp + m), s2 = col0 + c, above = s2 - row0 - 4 * g4;  // e >= above: t >= s
         const float cs = sc[s2], bs = sbeta[s2];
-        const float4_t qk = L4.rows_rows<K>(sq, sk, LK, row0, col0);
-        const bw_i16x4_t thi = L4.tr(tp + row0 * LB, LB, col0), tlo = L4.tr(tp + CC + row0 * LB, LB, col0);
+        const float4_t qk = L4.rows_rows<K>(sq, sk, row0, col0);
+        const bw_i16x4_t thi = L4.tr<BC>(tp, row0, col0), tlo = L4.tr<BC>(tp + CC, row0, col0);
         const float4_t tv = bf16x4_float(thi) + bf16x4_float(tlo);
 #pragma unroll
         for (int e = 0; e < 4; ++e) dec[m][a][e] = expf(ct[e] - cs);
@@ -544,6 +597,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     // W = T^T dT
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -553,8 +607,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         float4_t w = zero4();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const bh8_t th = L4.cols(tp, LB, kb, row0), tl = L4.cols(tp + CC, LB, kb, row0);
-          const bh8_t bh = L4.rows(b2t, LB, col0, kb), bl = L4.rows(b2t + CC, LB, col0, kb);
+          const bh8_t th = L4.cols<BC>(tp, kb, row0), tl = L4.cols<BC>(tp + CC, kb, row0);
+          const bh8_t bh = L4.rows<BC>(b2t, col0, kb), bl = L4.rows<BC>(b2t + CC, col0, kb);
           w = mfma_bf16(th, bh, w);
           w = mfma_bf16(th, bl, w);
           w = mfma_bf16(tl, bh, w);
@@ -563,6 +617,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     __syncthreads();
+    renew();
     // dA = -W T^T (strict lower): H = dA beta_t D into b3; dbeta, dc terms
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
@@ -573,13 +628,13 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         float4_t da = zero4();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const bh8_t wh = L4.cols(b4t, LB, kb, row0), wl = L4.cols(b4t + CC, LB, kb, row0);
-          const bh8_t th = L4.rows(tp, LB, col0, kb), tl = L4.rows(tp + CC, LB, col0, kb);
+          const bh8_t wh = L4.cols<BC>(b4t, kb, row0), wl = L4.cols<BC>(b4t + CC, kb, row0);
+          const bh8_t th = L4.rows<BC>(tp, col0, kb), tl = L4.rows<BC>(tp + CC, col0, kb);
           da = mfma_bf16(wh, th, da);
           da = mfma_bf16(wh, tl, da);
           da = mfma_bf16(wl, th, da);
         }
-        const float4_t gk = L4.rows_rows<K>(sk, sk, LK, row0, col0);
+        const float4_t gk = L4.rows_rows<K>(sk, sk, row0, col0);
         float4_t dad = dec[m][a] * -da;  // dA o D, t > s
 #pragma unroll
         for (int e = 0; e < 4; ++e) dad[e] = e > above ? dad[e] : 0.f;
@@ -621,7 +676,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     const int nh = next.block * heads + (last_head ? 0 : hh + 1);
     load_adjoint(next, nh, tid);
     load_state(next, nh, tid);
-    load_rest(next, nh, tid);
+    load_rest(next, nh, last_head, tid);
+    renew();
     // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + H K + H^T K
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -629,8 +685,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       bh8_t kf[KTW], qf[KTW];
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
-        kf[m] = L4.cols(sk, LK, kb, 16 * (KTW * cp + m));
-        qf[m] = L4.cols(sq, LK, kb, 16 * (KTW * cp + m));
+        kf[m] = L4.cols<K>(sk, kb, 16 * (KTW * cp + m));
+        qf[m] = L4.cols<K>(sq, kb, 16 * (KTW * cp + m));
       }
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -641,10 +697,10 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
           for (int m = 0; m < KTW; ++m) x[m][a] = mfma_bf16(lo, b[m], x[m][a]);
         };
-        product(tq, L4.cols(b1t, LB, kb, row0), L4.cols(b1t + CC, LB, kb, row0), kf);
-        product(tk, L4.rows(b1t, LB, row0, kb), L4.rows(b1t + CC, LB, row0, kb), qf);
-        product(tk, L4.cols(b3t, LB, kb, row0), L4.cols(b3t + CC, LB, kb, row0), kf);
-        product(tk, L4.rows(b3t, LB, row0, kb), L4.rows(b3t + CC, LB, row0, kb), kf);
+        product(tq, L4.cols<BC>(b1t, kb, row0), L4.cols<BC>(b1t + CC, kb, row0), kf);
+        product(tk, L4.rows<BC>(b1t, row0, kb), L4.rows<BC>(b1t + CC, row0, kb), qf);
+        product(tk, L4.cols<BC>(b3t, kb, row0), L4.cols<BC>(b3t + CC, kb, row0), kf);
+        product(tk, L4.rows<BC>(b3t, row0, kb), L4.rows<BC>(b3t + CC, row0, kb), kf);
         keep_order();
       }
     }
@@ -683,18 +739,18 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         __syncthreads();  // this head's readers of sq and sk are done
         const long base = (row0 * p.Hk + h / group) * K;
         const uint32_t stride = p.Hk * K;
-        u16 *buf = sq + wave * 16 * LB;
+        u16 *buf = sq + wave * 16 * BC;
         auto out = [&](void *dst, const float4_t (&x)[KTW][2]) {
 #pragma unroll
           for (int m = 0; m < KTW; ++m) {
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
-              *reinterpret_cast<v2u32_t *>(buf + c * LB + 16 * a + 4 * g4) =
+              *reinterpret_cast<v2u32_t *>(buf + L4.four<BC>(0, 16 * a)) =
                   __builtin_bit_cast(v2u32_t, __builtin_convertvector(x[m][a], bf16x4_t));
             }
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
-              const v2u32_t y = __builtin_bit_cast(v2u32_t, L4.tr(buf, LB, 16 * a));
+              const v2u32_t y = __builtin_bit_cast(v2u32_t, L4.tr<BC>(buf, 0, 16 * a));
               const int t = 32 * rp + 16 * a + c;
               u16 *row = static_cast<u16 *>(dst) + base + 16 * (KTW * cp + m);
               if (t < left) *reinterpret_cast<v2u32_t *>(row + t * stride + 4 * g4) = y;

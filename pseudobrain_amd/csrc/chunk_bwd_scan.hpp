@@ -28,17 +28,16 @@
 // ---------------------------------------------------------------------------
 template <int K>
 constexpr size_t local_bf16_lds() {
-  return sizeof(u16) * BC * (K + 8) + sizeof(float) * (BC * LC + 2 * BC + 3 * 256);
+  return sizeof(u16) * BC * K + sizeof(float) * (BC * LC + 2 * BC + 3 * 256);
 }
 
 template <int K>
 __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
-  constexpr int LK = K + 8;
   extern __shared__ __align__(16) float lds[];
   PBGDN_POISON_LDS(lds, local_bf16_lds<K>());
   PBGDN_POISON_SYNC();
   u16 *sk = reinterpret_cast<u16 *>(lds);
-  float *sa = reinterpret_cast<float *>(sk + BC * LK), *sc = sa + BC * LC, *sbeta = sc + BC, *sr = sbeta + BC;
+  float *sa = reinterpret_cast<float *>(sk + BC * K), *sc = sa + BC * LC, *sbeta = sc + BC, *sr = sbeta + BC;
   u16 *mh = reinterpret_cast<u16 *>(sa);  // M^T, a pair of rows of LC, in sa's bytes once T is out
   const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -52,8 +51,8 @@ __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
   const long r = rec(p, seq, h, i);
   bh8_t qf[K / 32];
   {
-    RawRows<u16, K> rk;
-    rk.load(p.k, seq, t0, p.Hk, hk, K);
+    RowsAhead<K, BNT> rk;
+    rk.load(tid, static_cast<const u16 *>(p.k) + ((seq.bos + t0) * p.Hk + hk) * K, p.Hk * K, seq.len - t0);
     const int t = t0 + 16 * wave + ln.c;
     const u16 *row = static_cast<const u16 *>(p.q) + ((seq.bos + min(t, seq.len - 1)) * p.Hk + hk) * K + 8 * ln.g;
 #pragma unroll
@@ -72,7 +71,7 @@ __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
       p.ws_c[r * BC + lane] = x;
       p.ws_beta[r * BC + lane] = bt;
     }
-    rk.put(sk, LK);
+    rk.put(tid, sk, seq.len - t0);
   }
   __syncthreads();
   // A = strict_lower(beta_t (K K^T) o D), rows 16w .. of this wave; M^T's
@@ -87,8 +86,8 @@ __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
       float4_t kk = zero4(), kq = zero4();
 #pragma unroll
       for (int kb = 0; kb < K / 32; ++kb) {
-        const bh8_t kr = ln.rows16(sk, LK, 16 * tc, kb);
-        kk = mfma_bf16(ln.rows16(sk, LK, 16 * wave, kb), kr, kk);
+        const bh8_t kr = ln.rows16<K>(sk, 16 * tc, kb);
+        kk = mfma_bf16(ln.rows16<K>(sk, 16 * wave, kb), kr, kk);
         kq = mfma_bf16(kr, qf[kb], kq);
       }
 #pragma unroll
@@ -139,13 +138,12 @@ __global__ __launch_bounds__(BNT) void bwd_local_bf16_kernel(BwdParams p) {
 template <int K, int NW>
 struct Scan16 {
   static constexpr int LOADERS = 256, NT = 64 * NW + LOADERS;
-  static constexpr int LK = K + 8, LB = BC + 8, LC16 = 16 * NW + 8;  // row strides (elements)
-  static constexpr int PAIR = 2 * BC * LB;
+  static constexpr int COLS = 16 * NW, PAIR = 2 * BC * BC;
   // one buffer: K rows, the T pair, the V or dO columns, four vectors (e^c,
   // e^(c_last - c), beta; the adjoint's scale e^c, e^(c_last - c), -beta e^c;
   // e^c_last last); the adjoint's also Q rows and the M^T pair
-  static constexpr int OFF_T = BC * LK, OFF_X = OFF_T + PAIR, OFF_VEC = OFF_X + BC * LC16;
-  static constexpr int OFF_Q = OFF_VEC + 2 * 4 * BC, OFF_M = OFF_Q + BC * LK, BUF = OFF_M + PAIR;
+  static constexpr int OFF_T = BC * K, OFF_X = OFF_T + PAIR, OFF_VEC = OFF_X + BC * COLS;
+  static constexpr int OFF_Q = OFF_VEC + 2 * 4 * BC, OFF_M = OFF_Q + BC * K, BUF = OFF_M + PAIR;
   static constexpr size_t BYTES = 2 * sizeof(u16) * BUF;
   static_assert(OFF_VEC % 8 == 0 && OFF_Q % 8 == 0 && BUF % 8 == 0, "16-byte pieces");
 };
@@ -233,23 +231,23 @@ struct ScanLoad {
 #pragma unroll
     for (int a = 0; a < KP; ++a) {
       const int e = tid + N * a, row = e / (K / 8), part = e % (K / 8);
-      *reinterpret_cast<uint4 *>(buf + row * L::LK + part * 8) = k[a];
-      if constexpr (ADJ) *reinterpret_cast<uint4 *>(buf + L::OFF_Q + row * L::LK + part * 8) = q[a];
+      *reinterpret_cast<uint4 *>(buf + unit_at<K>(row, part)) = k[a];
+      if constexpr (ADJ) *reinterpret_cast<uint4 *>(buf + L::OFF_Q + unit_at<K>(row, part)) = q[a];
     }
 #pragma unroll
     for (int a = 0; a < TP; ++a) {
       int half, row, part;
       tri(tid + N * a, false, half, row, part);
-      *reinterpret_cast<uint4 *>(buf + L::OFF_T + (half * BC + row) * L::LB + part * 8) = t[a];
+      *reinterpret_cast<uint4 *>(buf + L::OFF_T + unit_at<BC>(half * BC + row, part)) = t[a];
       if constexpr (ADJ) {
         tri(tid + N * a, true, half, row, part);
-        *reinterpret_cast<uint4 *>(buf + L::OFF_M + (half * BC + row) * L::LB + part * 8) = m[a];
+        *reinterpret_cast<uint4 *>(buf + L::OFF_M + unit_at<BC>(half * BC + row, part)) = m[a];
       }
     }
 #pragma unroll
     for (int a = 0; a < XP; ++a) {
       const int e = tid + N * a, row = e / (2 * NW), part = e % (2 * NW);
-      *reinterpret_cast<uint4 *>(buf + L::OFF_X + row * L::LC16 + part * 8) = x[a];
+      *reinterpret_cast<uint4 *>(buf + L::OFF_X + unit_at<L::COLS>(row, part)) = x[a];
     }
     if (tid < BC) {
       float *vec = reinterpret_cast<float *>(buf + L::OFF_VEC);
@@ -268,9 +266,9 @@ struct ScanLoad {
 // exposed waits a step: 1,681 us of scans at 1 x 32,768 tokens of 32 heads).
 // Key tiles' operands of the contraction over tokens 32 kb ..
 template <int KT>
-__device__ __forceinline__ void read_cols(const Lane &ln, const u16 *m, int ld, int kb, bh8_t (&a)[KT]) {
+__device__ __forceinline__ void read_cols(const Lane &ln, const u16 *m, int kb, bh8_t (&a)[KT]) {
 #pragma unroll
-  for (int t = 0; t < KT; ++t) a[t] = ln.cols(m, ld, kb, 16 * t);
+  for (int t = 0; t < KT; ++t) a[t] = ln.cols<16 * KT>(m, kb, 16 * t);
 }
 
 // s += the operands times a pair.
@@ -287,7 +285,7 @@ __device__ __forceinline__ void add_products(float4_t (&s)[KT], const bh8_t (&a)
 template <int K, int NW, bool ADJ>
 __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int col, float4_t (&s)[K / 16]) {
   using L = Scan16<K, NW>;
-  constexpr int KT = K / 16, KB = K / 32, LK = L::LK, LB = L::LB, CC = BC * LB;
+  constexpr int KT = K / 16, KB = K / 32, W = L::COLS, CC = BC * BC;
   const u16 *sk = buf, *tp = buf + L::OFF_T, *sx = buf + L::OFF_X;
   const float *vec = reinterpret_cast<const float *>(buf + L::OFF_VEC) + 4 * ln.g;
   // ---- K S
@@ -295,7 +293,7 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
   for (int kb = 0; kb < KB / 2; ++kb) {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows(sk, LK, 16 * rt, kb);
+    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows<K>(sk, 16 * rt, kb);
   }
   keep_order();
   v2u32_t sh[KT], sl[KT];
@@ -305,7 +303,7 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
   for (int kb = KB / 2; kb < KB; ++kb) {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows(sk, LK, 16 * rt, kb);
+    for (int rt = 0; rt < 4; ++rt) ka[kb][rt] = ln.rows<K>(sk, 16 * rt, kb);
   }
   keep_order();
   float4_t y[4];
@@ -330,8 +328,8 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
         if (!used(rt, kb)) continue;
-        th[rt][kb] = ADJ ? ln.cols(tp, LB, kb, 16 * rt) : ln.rows(tp, LB, 16 * rt, kb);
-        tl[rt][kb] = ADJ ? ln.cols(tp + CC, LB, kb, 16 * rt) : ln.rows(tp + CC, LB, 16 * rt, kb);
+        th[rt][kb] = ADJ ? ln.cols<BC>(tp, kb, 16 * rt) : ln.rows<BC>(tp, 16 * rt, kb);
+        tl[rt][kb] = ADJ ? ln.cols<BC>(tp + CC, kb, 16 * rt) : ln.rows<BC>(tp + CC, 16 * rt, kb);
       }
     }
   };
@@ -342,7 +340,7 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
   if constexpr (!ADJ) {
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      xr[rt] = ln.tr(sx + 16 * rt * L::LC16, L::LC16, col);
+      xr[rt] = ln.tr<W>(sx, 16 * rt, col);
       w0[rt] = ld4(vec + 16 * rt);           // e^c
       w1[rt] = ld4(vec + 2 * BC + 16 * rt);  // beta
     }
@@ -360,13 +358,13 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) w0[rt] = ld4(vec + BC + 16 * rt);  // e^(c_last - c)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) xr[rt] = ln.tr(sx + 16 * rt * L::LC16, L::LC16, col);
+    for (int rt = 0; rt < 4; ++rt) xr[rt] = ln.tr<W>(sx, 16 * rt, col);
 #pragma unroll
     for (int kb = 1; kb >= 0; --kb) {
 #pragma unroll
       for (int rt = 0; rt < 2 * kb + 2; ++rt) {  // t >= s
-        mh[rt][kb] = ln.rows(mt, LB, 16 * rt, kb);
-        ml[rt][kb] = ln.rows(mt + CC, LB, 16 * rt, kb);
+        mh[rt][kb] = ln.rows<BC>(mt, 16 * rt, kb);
+        ml[rt][kb] = ln.rows<BC>(mt + CC, 16 * rt, kb);
       }
     }
     keep_order();
@@ -398,7 +396,7 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
   keep_order();
   // ---- U = T (beta X), s <= t; or dX / beta = T^T dU, t >= s
   bh8_t a0[KT], a1[KT];
-  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, LK, 0, a0);
+  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, 0, a0);
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) w0[rt] = ld4(vec + (ADJ ? 2 : 1) * BC + 16 * rt);  // -beta e^c, or e^(c_last - c)
   const float gam_c = vec[4 * BC - 1 - 4 * ln.g];
@@ -425,7 +423,7 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
   for (int m = 0; m < KT; ++m) s[m] *= gam_c;
   keep_order();
-  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, LK, 1, a1);
+  read_cols(ln, ADJ ? buf + L::OFF_Q : sk, 1, a1);
   keep_order();
   v2u32_t zh[4], zl[4];  // E U, or -Gamma dX
   if constexpr (ADJ) {  // Q's products fill the splits' place in the chain
@@ -433,11 +431,11 @@ __device__ __forceinline__ void scan16_step(const u16 *buf, const Lane &ln, int 
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) split_bf16(z[rt] * w0[rt], zh[rt], zl[rt]);
     keep_order();
-    read_cols(ln, sk, LK, 0, a0);
+    read_cols(ln, sk, 0, a0);
     keep_order();
     add_products(s, a1, frag_pair(oh[2], oh[3]), frag_pair(ol[2], ol[3]));
     keep_order();
-    read_cols(ln, sk, LK, 1, a1);
+    read_cols(ln, sk, 1, a1);
     keep_order();
   } else {
 #pragma unroll
