@@ -667,16 +667,14 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     __syncthreads();
     // The next head's inputs (the same head's again if it is the last: a load
     // left out on one path would keep the old values alive to the end of the
-    // loop on every path). Earlier they do not fit into the registers: issued
-    // among the stages they were spilled as they arrived.
+    // loop on every path), loaded during the last products. Earlier they do not
+    // fit into the registers: issued among the stages they were spilled as they
+    // arrived.
     const bool last_head = hh + 1 == heads;
     next = it;
     if (last_head) more = grad_item(p, it.item + gridDim.x, gridDim.x, items, chunks, blocks, next);
     if (!more) next = it;
     const int nh = next.block * heads + (last_head ? 0 : hh + 1);
-    load_adjoint(next, nh, tid);
-    load_state(next, nh, tid);
-    load_rest(next, nh, last_head, tid);
     renew();
     // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + H K + H^T K
 #pragma unroll
@@ -690,6 +688,11 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
+        // (spread over the products, which go on while the CU takes the loads)
+        if (kb == 0 && a == 0) load_adjoint(next, nh, tid);
+        if (kb == 0 && a == 1) load_state(next, nh, tid);
+        if (kb == 1 && a == 0) load_rest(next, nh, last_head, tid);
+        keep_order();
         const int row0 = 32 * rp + 16 * a;
         auto product = [&](float4_t (&x)[KTW][2], bh8_t hi, bh8_t lo, const bh8_t (&b)[KTW]) {
 #pragma unroll
