@@ -206,132 +206,7 @@ __device__ __forceinline__ float4_t mfma_bf16(bh8_t a, bh8_t b, float4_t acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
 }
 
-// Rows row0 .. row0+15 of a [64][ldr] bf16 array (exact inputs) times a
-// state tile given as its transpose in two bf16 parts, hiT + loT ([16][lds],
-// x = hi + lo to 16 bits): sum over k < KD, on bf16 MFMA with fp32
-// accumulation. Both operands are read k-contiguous, 16 bytes a lane.
-template <int KD>
-__device__ __forceinline__ float4_t rows_times_state(const u16 *rows, int ldr, int row0, const u16 *hiT,
-                                                     const u16 *loT, int ldt) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int kb = 0; kb < KD; kb += 32) {
-    const bh8_t a = *reinterpret_cast<const bh8_t *>(rows + (row0 + c) * ldr + kb + 8 * g);
-    acc = mfma_bf16(a, *reinterpret_cast<const bh8_t *>(hiT + c * ldt + kb + 8 * g), acc);
-    acc = mfma_bf16(a, *reinterpret_cast<const bh8_t *>(loT + c * ldt + kb + 8 * g), acc);
-  }
-  return acc;
-}
-
-// Rows a0 .. a0+15 of one [64][ld] bf16 array times the transpose of rows
-// b0 .. b0+15 of another (exact inputs, sum over k < KD) on bf16 MFMA.
-template <int KD>
-__device__ __forceinline__ float4_t rows_times_rows(const u16 *a, const u16 *b, int ld, int a0, int b0) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int kb = 0; kb < KD; kb += 32) {
-    acc = mfma_bf16(*reinterpret_cast<const bh8_t *>(a + (a0 + c) * ld + kb + 8 * g),
-                    *reinterpret_cast<const bh8_t *>(b + (b0 + c) * ld + kb + 8 * g), acc);
-  }
-  return acc;
-}
-
 typedef short bw_i16x4_t __attribute__((ext_vector_type(4)));
-
-// x (rows k0 .. k0+3 of column c) into a transposed pair of bf16 tiles
-// (high at hiT, low 16 rows of ld after it): 8 bytes each.
-__device__ __forceinline__ void put_t_pair(u16 *hiT, int ld, int k0, int c, float4_t x) {
-  v2u32_t hi, lo;
-  split_bf16(x, hi, lo);
-  *reinterpret_cast<v2u32_t *>(hiT + c * ld + k0) = hi;
-  *reinterpret_cast<v2u32_t *>(hiT + 16 * ld + c * ld + k0) = lo;
-}
-
-// Rows row0 .. row0+15 of an A pair (high ah, low al; rows of lda) times a B
-// pair given transposed (bh, bl: [16][ldb]), over k < KD: A_hi B_hi + A_hi
-// B_lo + A_lo B_hi on bf16 MFMA (fp32 accurate to about 2^-16).
-template <int KD>
-__device__ __forceinline__ float4_t pair_times_pair(const u16 *ah, const u16 *al, int lda, int row0, const u16 *bh,
-                                                    const u16 *bl, int ldb) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int kb = 0; kb < KD; kb += 32) {
-    const bh8_t a_h = *reinterpret_cast<const bh8_t *>(ah + (row0 + c) * lda + kb + 8 * g);
-    const bh8_t a_l = *reinterpret_cast<const bh8_t *>(al + (row0 + c) * lda + kb + 8 * g);
-    const bh8_t b_h = *reinterpret_cast<const bh8_t *>(bh + c * ldb + kb + 8 * g);
-    const bh8_t b_l = *reinterpret_cast<const bh8_t *>(bl + c * ldb + kb + 8 * g);
-    acc = mfma_bf16(a_h, b_h, acc);
-    acc = mfma_bf16(a_h, b_l, acc);
-    acc = mfma_bf16(a_l, b_h, acc);
-  }
-  return acc;
-}
-
-// The A fragment of columns col0 .. col0+15 of a row-major bf16 array (rows
-// of ld) taken as rows, contraction rows k0 + 8g .. k0 + 8g + 7: two
-// transposing reads (lanes 4k .. 4k+3 of group g address row k0 + 8g + k
-// (+ 4), 8 bytes at column col0 + 4 (c & 3); lane c receives column col0 + c).
-__device__ __forceinline__ bh8_t tr_frag(const u16 *m, int ld, int k0, int col0) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const u16 *a = m + (k0 + 8 * g + (c >> 2)) * ld + col0 + 4 * (c & 3);
-  const bw_i16x4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bw_i16x4_t *)(a));
-  const bw_i16x4_t hi4 =
-      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bw_i16x4_t *)(a + 4 * ld));
-  return __builtin_bit_cast(bh8_t, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// bf16 MFMA with four k per lane: acc (16x16) += A (16x16) B (16x16); lane l,
-// c = l & 15, g = l >> 4: A[m=c][k=4g..4g+3], B[k=4g..4g+3][n=c].
-__device__ __forceinline__ float4_t mfma_bf16_k16(bw_i16x4_t a, bw_i16x4_t b, float4_t acc) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-}
-
-// Rows 4g .. 4g+3 of column col0 + c of a row-major 16-bit array (rows of
-// ld) in lane (c, g): one transposing read (lanes 4k .. 4k+3 of group g
-// address row 4g + k, 8 bytes at column col0 + 4 (c & 3)). Taken from a
-// transposed tile M^T it is the A or B operand of M's rows col0 .. col0+15
-// with k the 16 rows of M^T.
-__device__ __forceinline__ bw_i16x4_t tr4(const u16 *m, int ld, int col0) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) bw_i16x4_t *)(m + (4 * g + (c >> 2)) * ld + col0 + 4 * (c & 3)));
-}
-
-// (columns k0 .. k0+15 of the K rows)^T times a B pair given transposed,
-// over the 64 tokens: K is exact in bf16, so two products per step.
-__device__ __forceinline__ float4_t kt_times_pair(const u16 *sk, int ldk, int k0, const u16 *bh, const u16 *bl,
-                                                  int ldb) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ts = 0; ts < BC; ts += 32) {
-    const bh8_t a = tr_frag(sk, ldk, ts, k0);
-    acc = mfma_bf16(a, *reinterpret_cast<const bh8_t *>(bh + c * ldb + ts + 8 * g), acc);
-    acc = mfma_bf16(a, *reinterpret_cast<const bh8_t *>(bl + c * ldb + ts + 8 * g), acc);
-  }
-  return acc;
-}
-
-// (columns col0 .. col0+15 of T)^T, T a high/low pair of rows of ldt, times
-// a B pair given transposed, over the 64 rows of T.
-__device__ __forceinline__ float4_t tt_times_pair(const u16 *th, const u16 *tl, int ldt, int col0, const u16 *bh,
-                                                  const u16 *bl, int ldb) {
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ts = 0; ts < BC; ts += 32) {
-    const bh8_t a_h = tr_frag(th, ldt, ts, col0), a_l = tr_frag(tl, ldt, ts, col0);
-    const bh8_t b_h = *reinterpret_cast<const bh8_t *>(bh + c * ldb + ts + 8 * g);
-    const bh8_t b_l = *reinterpret_cast<const bh8_t *>(bl + c * ldb + ts + 8 * g);
-    acc = mfma_bf16(a_h, b_h, acc);
-    acc = mfma_bf16(a_h, b_l, acc);
-    acc = mfma_bf16(a_l, b_h, acc);
-  }
-  return acc;
-}
 
 // Round to the nearest bf16 (ties to even) of a finite float, as its bits.
 __device__ __forceinline__ u16 bf16_bits(float x) {
@@ -352,11 +227,6 @@ __device__ __forceinline__ void store_el(void *p, long i, float x) {
   } else {
     static_cast<half_t *>(p)[i] = static_cast<half_t>(x);
   }
-}
-
-// The value of a bf16 high/low pair.
-__device__ __forceinline__ float pair_val(const u16 *m, int lo_off, int e) {
-  return __uint_as_float(static_cast<uint32_t>(m[e]) << 16) + __uint_as_float(static_cast<uint32_t>(m[lo_off + e]) << 16);
 }
 
 // x as a bf16 high/low pair: element e of the high array, e + lo_off of the low.
@@ -432,22 +302,6 @@ __device__ __forceinline__ void load_t(float *st, const float *src) {
   for (int m = 0; m < 4; ++m) {
     const int e = threadIdx.x + BNT * m;
     *reinterpret_cast<float4_t *>(&st[(e >> 4) * LC + 4 * (e & 15)]) = raw[m];
-  }
-}
-
-// A 64 x 64 float32 record (T) into LDS as a bf16 high/low pair of rows ld.
-__device__ __forceinline__ void load_t_pair(u16 *tp, int ld, const float *src) {
-  const float4_t *w = reinterpret_cast<const float4_t *>(src);
-  float4_t raw[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) raw[m] = w[threadIdx.x + BNT * m];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int e = threadIdx.x + BNT * m;
-    v2u32_t hi, lo;
-    split_bf16(raw[m], hi, lo);
-    *reinterpret_cast<v2u32_t *>(tp + (e >> 4) * ld + 4 * (e & 15)) = hi;
-    *reinterpret_cast<v2u32_t *>(tp + BC * ld + (e >> 4) * ld + 4 * (e & 15)) = lo;
   }
 }
 
@@ -741,39 +595,26 @@ struct ScanStage {
     }
   }
 
-  // K rows, T, the decays and the tile into LDS (sk, st, vectors, tile). K
-  // rows go in as they are for bf16 inputs (rows of K + 8), else as float
-  // (rows of K + 4).
+  // K rows (as float, rows of K + 4), T, the decays and the tile into LDS (sk,
+  // st, vectors, tile).
   __device__ __forceinline__ void store(void *sk, void *st, float *sc, float *sgam, float *se, float *sbeta,
                                         float *tile) const {
     const int tid = threadIdx.x;
 #pragma unroll
     for (int m = 0; m < KP; ++m) {
       const int e = tid + BNT * m, row = e / ROW16, part = e % ROW16;
-      if constexpr (std::is_same<TIn, u16>::value) {
-        *reinterpret_cast<uint4 *>(static_cast<u16 *>(sk) + row * (K + 8) + part * EPP) = kr[m];
-      } else {
-        float x[EPP];
-        decode16<TIn>(kr[m], x);
+      float x[EPP];
+      decode16<TIn>(kr[m], x);
 #pragma unroll
-        for (int j = 0; j < EPP; j += 4) {
-          *reinterpret_cast<float4_t *>(static_cast<float *>(sk) + row * (K + 4) + part * EPP + j) =
-              float4_t{x[j], x[j + 1], x[j + 2], x[j + 3]};
-        }
+      for (int j = 0; j < EPP; j += 4) {
+        *reinterpret_cast<float4_t *>(static_cast<float *>(sk) + row * (K + 4) + part * EPP + j) =
+            float4_t{x[j], x[j + 1], x[j + 2], x[j + 3]};
       }
     }
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const int e = tid + BNT * m;
-      if constexpr (std::is_same<TIn, u16>::value) {  // T as bf16 high/low rows of BC + 8
-        u16 *th = static_cast<u16 *>(st);
-        v2u32_t hi, lo;
-        split_bf16(tr[m], hi, lo);
-        *reinterpret_cast<v2u32_t *>(th + (e >> 4) * (BC + 8) + 4 * (e & 15)) = hi;
-        *reinterpret_cast<v2u32_t *>(th + BC * (BC + 8) + (e >> 4) * (BC + 8) + 4 * (e & 15)) = lo;
-      } else {
-        *reinterpret_cast<float4_t *>(static_cast<float *>(st) + (e >> 4) * LC + 4 * (e & 15)) = tr[m];
-      }
+      *reinterpret_cast<float4_t *>(static_cast<float *>(st) + (e >> 4) * LC + 4 * (e & 15)) = tr[m];
     }
     if (tid < BC) {
       const float last = __shfl(cv, BC - 1, 64);
@@ -803,95 +644,62 @@ struct ScanStage {
 // start. Wave w holds key-row tiles w, w+4 (K/64 of them) of the state. The
 // next chunk's inputs load during each step.
 // ---------------------------------------------------------------------------
-// LDS of one scan workgroup. bf16 inputs: K rows as they are and the state
-// tile as its transpose in bf16 high/low parts (for K S on bf16 MFMA); other
-// inputs: K rows and the state tile in float.
+// LDS of one scan workgroup: K rows, T, the state tile, the step's V or dU0
+// tile, the tile the next products read and the decay vectors, in float.
 template <int K, typename TIn>
 struct ScanLds {
-  static constexpr bool BF = std::is_same<TIn, u16>::value;
-  static constexpr int LK = BF ? K + 8 : K + 4, LS = K + 8, LB = BC + 8;
-  // K rows; T (bf16: high and low parts, rows of LB); the state tile (bf16:
-  // its transpose, high and low); the step's V or dU0 tile in float; the
-  // tiles the next products read (bf16: two transposed high/low pairs
-  // [16][LB], float: one [64][LT] tile); decay vectors.
-  static constexpr size_t K_BYTES = BF ? sizeof(u16) * BC * LK : sizeof(float) * BC * LK;
-  static constexpr size_t T_BYTES = BF ? sizeof(u16) * 2 * BC * LB : sizeof(float) * BC * LC;
-  static constexpr size_t S_BYTES = BF ? sizeof(u16) * 2 * 16 * LS : sizeof(float) * K * LT;
-  static constexpr size_t A_BYTES = BF ? sizeof(u16) * 2 * 2 * 16 * LB : sizeof(float) * BC * LT;
+  static constexpr int LK = K + 4;
+  static constexpr size_t K_BYTES = sizeof(float) * BC * LK;
+  static constexpr size_t T_BYTES = sizeof(float) * BC * LC;
+  static constexpr size_t S_BYTES = sizeof(float) * K * LT;
+  static constexpr size_t A_BYTES = sizeof(float) * BC * LT;
   static constexpr size_t OFF_T = K_BYTES, OFF_S = OFF_T + T_BYTES, OFF_TILE = OFF_S + S_BYTES,
                           OFF_A = OFF_TILE + sizeof(float) * BC * LT, OFF_VEC = OFF_A + A_BYTES;
   static constexpr size_t BYTES = OFF_VEC + sizeof(float) * 4 * BC;
 };
 
-// K rows (row0 + r) times the state tile kept in LDS: bf16 MFMA on the high
-// and low parts of its transpose, or the fp32 MFMA on the float tile.
+// K rows (row0 + r) times the state tile kept in LDS.
 template <int K, typename TIn>
 __device__ __forceinline__ float4_t k_times_state(const void *sk, int row0, const void *sstate) {
   using L = ScanLds<K, TIn>;
-  if constexpr (L::BF) {
-    const u16 *hiT = static_cast<const u16 *>(sstate);
-    return rows_times_state<K>(static_cast<const u16 *>(sk), L::LK, row0, hiT, hiT + 16 * L::LS, L::LS);
-  } else {
-    const float *kf = static_cast<const float *>(sk), *sf = static_cast<const float *>(sstate);
-    return tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4(&kf[(row0 + r) * L::LK + kk]); },
-                       [&](int kk, int col) { return ld4s(&sf[kk * LT + col], LT); });
-  }
+  const float *kf = static_cast<const float *>(sk), *sf = static_cast<const float *>(sstate);
+  return tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4(&kf[(row0 + r) * L::LK + kk]); },
+                     [&](int kk, int col) { return ld4s(&sf[kk * LT + col], LT); });
 }
 
-// Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the state tile, column c, into LDS: the
-// float tile, or the high/low parts of its transpose (8 bytes each).
+// Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the state tile, column c, into LDS.
 template <int K, typename TIn>
 __device__ __forceinline__ void put_state_rows(void *sstate, int kk0, int c, float4_t x) {
-  using L = ScanLds<K, TIn>;
-  if constexpr (L::BF) {
-    u16 *hiT = static_cast<u16 *>(sstate);
-    v2u32_t hi, lo;
-    split_bf16(x, hi, lo);
-    *reinterpret_cast<v2u32_t *>(hiT + c * L::LS + kk0) = hi;
-    *reinterpret_cast<v2u32_t *>(hiT + 16 * L::LS + c * L::LS + kk0) = lo;
-  } else {
-    float *sf = static_cast<float *>(sstate);
+  float *sf = static_cast<float *>(sstate);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sf[(kk0 + r) * LT + c] = x[r];
-  }
+  for (int r = 0; r < 4; ++r) sf[(kk0 + r) * LT + c] = x[r];
 }
 
 // (diag(w) K)^T rows k0 + r, four tokens t .. t+3 of the K rows in LDS.
 template <int K, typename TIn>
 __device__ __forceinline__ float4_t k_cols(const void *sk, int t, int col) {
   using L = ScanLds<K, TIn>;
-  if constexpr (L::BF) {
-    return ld4es(static_cast<const u16 *>(sk), t * L::LK + col, L::LK);
-  } else {
-    return ld4s(static_cast<const float *>(sk) + t * L::LK + col, L::LK);
-  }
+  return ld4s(static_cast<const float *>(sk) + t * L::LK + col, L::LK);
 }
 
-// Key tile kt of the value columns v0 .. of a state record, from the
-// accumulator layout. bf16 inputs: in that layout as it is, tile (v0 / 16, kt)
-// 64 lanes x 16 bytes (what the gradient kernel's waves hold); else [K][V].
+// Key tile kt of the value columns v0 .. of a state record ([K][V]), from the
+// accumulator layout.
 template <int K, typename TIn>
 __device__ __forceinline__ void put_state_tile(float *ws, int V, int v0, int kt, float4_t x) {
   const int lane = threadIdx.x & 63;
-  if constexpr (std::is_same<TIn, u16>::value) {
-    reinterpret_cast<float4_t *>(ws)[((v0 >> 4) * (K / 16) + kt) * 64 + lane] = x;
-  } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ws[static_cast<long>(16 * kt + 4 * (lane >> 4) + r) * V + v0 + (lane & 15)] = x[r];
-  }
+  for (int r = 0; r < 4; ++r) ws[static_cast<long>(16 * kt + 4 * (lane >> 4) + r) * V + v0 + (lane & 15)] = x[r];
 }
 
 template <int K, typename TIn>
 __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
   const BwdSeq seq = seq_of(p, n);
   using L = ScanLds<K, TIn>;
-  constexpr int PER = K / 64, LB = L::LB;
+  constexpr int PER = K / 64;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
   void *sk = base, *st = base + L::OFF_T, *ss = base + L::OFF_S;
   float *sx = reinterpret_cast<float *>(base + L::OFF_TILE), *su = reinterpret_cast<float *>(base + L::OFF_A);
   float *sc = reinterpret_cast<float *>(base + L::OFF_VEC), *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
-  // bf16 inputs: (beta X)^T and (E U)^T as high/low pairs
-  u16 *xT = reinterpret_cast<u16 *>(base + L::OFF_A), *uT = xT + 2 * 16 * LB;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
   const long kv = (static_cast<long>(n) * p.Hv + h) * K * p.V;
@@ -918,38 +726,19 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
     __syncthreads();
     // X = V - Gamma K S (rows 16w ..)
     const float4_t ks = k_times_state<K, TIn>(sk, 16 * wave, ss);
-    if constexpr (L::BF) {
-      float4_t xb;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * wave + 4 * g4 + r;
-        xb[r] = (sx[t * LT + c] - sgam[t] * ks[r]) * sbeta[t];
-      }
-      put_t_pair(xT, LB, 16 * wave + 4 * g4, c, xb);
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * wave + 4 * g4 + r;
-        sx[t * LT + c] -= sgam[t] * ks[r];
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * wave + 4 * g4 + r;
+      sx[t * LT + c] -= sgam[t] * ks[r];
     }
     __syncthreads();
     // U = T diag(beta) X
-    if constexpr (L::BF) {
-      const u16 *th = static_cast<const u16 *>(st);
-      const float4_t u = pair_times_pair<BC>(th, th + BC * LB, LB, 16 * wave, xT, xT + 16 * LB, LB);
-      float4_t eu;
+    const float *stf = static_cast<const float *>(st);
+    const float4_t u = tile_mm4<BC>(
+        zero4(), [&](int r, int s2) { return ld4(&stf[(16 * wave + r) * LC + s2]) * ld4(&sbeta[s2]); },
+        [&](int s2, int col) { return ld4s(&sx[s2 * LT + col], LT); });
 #pragma unroll
-      for (int r = 0; r < 4; ++r) eu[r] = se[16 * wave + 4 * g4 + r] * u[r];
-      put_t_pair(uT, LB, 16 * wave + 4 * g4, c, eu);
-    } else {
-      const float *stf = static_cast<const float *>(st);
-      const float4_t u = tile_mm4<BC>(
-          zero4(), [&](int r, int s2) { return ld4(&stf[(16 * wave + r) * LC + s2]) * ld4(&sbeta[s2]); },
-          [&](int s2, int col) { return ld4s(&sx[s2 * LT + col], LT); });
-#pragma unroll
-      for (int r = 0; r < 4; ++r) su[(16 * wave + 4 * g4 + r) * LT + c] = u[r];
-    }
+    for (int r = 0; r < 4; ++r) su[(16 * wave + 4 * g4 + r) * LT + c] = u[r];
     __syncthreads();
     // S = gamma_C S + K^T E U
     const float gam_c = sgam[BC - 1];
@@ -957,12 +746,8 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
     for (int m = 0; m < PER; ++m) {
       const int k0 = 16 * (wave + 4 * m);
       float4_t y;
-      if constexpr (L::BF) {
-        y = kt_times_pair(static_cast<const u16 *>(sk), L::LK, k0, uT, uT + 16 * LB, LB);
-      } else {
-        y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&se[t]); },
-                         [&](int t, int col) { return ld4s(&su[t * LT + col], LT); });
-      }
+      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&se[t]); },
+                       [&](int t, int col) { return ld4s(&su[t * LT + col], LT); });
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[m][r] = gam_c * s[m][r] + y[r];
     }
@@ -978,13 +763,11 @@ template <int K, typename TIn>
 __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
   const BwdSeq seq = seq_of(p, n);
   using L = ScanLds<K, TIn>;
-  constexpr int PER = K / 64, LB = L::LB;
+  constexpr int PER = K / 64;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
   void *sk = base, *st = base + L::OFF_T, *sds = base + L::OFF_S;
   float *sdu = reinterpret_cast<float *>(base + L::OFF_TILE), *sdx = reinterpret_cast<float *>(base + L::OFF_A);
   float *sc = reinterpret_cast<float *>(base + L::OFF_VEC), *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
-  // bf16 inputs: dU^T and (Gamma dX)^T as high/low pairs
-  u16 *duT = reinterpret_cast<u16 *>(base + L::OFF_A), *gxT = duT + 2 * 16 * LB;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int hk = h / (p.Hv / p.Hk);
   const long kv = (static_cast<long>(n) * p.Hv + h) * K * p.V;
@@ -1017,41 +800,19 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     __syncthreads();
     // dU = dU0 + E K dS'
     const float4_t kd = k_times_state<K, TIn>(sk, 16 * wave, sds);
-    if constexpr (L::BF) {
-      float4_t du;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * wave + 4 * g4 + r;
-        du[r] = sdu[t * LT + c] + se[t] * kd[r];
-      }
-      put_t_pair(duT, LB, 16 * wave + 4 * g4, c, du);
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * wave + 4 * g4 + r;
-        sdu[t * LT + c] += se[t] * kd[r];
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * wave + 4 * g4 + r;
+      sdu[t * LT + c] += se[t] * kd[r];
     }
     __syncthreads();
     // dX = (T diag(beta))^T dU
-    if constexpr (L::BF) {
-      const u16 *th = static_cast<const u16 *>(st);
-      const float4_t dx = tt_times_pair(th, th + BC * LB, LB, 16 * wave, duT, duT + 16 * LB, LB);
-      float4_t gx;
+    const float *stf = static_cast<const float *>(st);
+    const float4_t dx = tile_mm4<BC>(
+        zero4(), [&](int r, int s2) { return ld4s(&stf[s2 * LC + 16 * wave + r], LC) * sbeta[16 * wave + r]; },
+        [&](int s2, int col) { return ld4s(&sdu[s2 * LT + col], LT); });
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * wave + 4 * g4 + r;
-        gx[r] = sgam[t] * (sbeta[t] * dx[r]);
-      }
-      put_t_pair(gxT, LB, 16 * wave + 4 * g4, c, gx);
-    } else {
-      const float *stf = static_cast<const float *>(st);
-      const float4_t dx = tile_mm4<BC>(
-          zero4(), [&](int r, int s2) { return ld4s(&stf[s2 * LC + 16 * wave + r], LC) * sbeta[16 * wave + r]; },
-          [&](int s2, int col) { return ld4s(&sdu[s2 * LT + col], LT); });
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sdx[(16 * wave + 4 * g4 + r) * LT + c] = dx[r];
-    }
+    for (int r = 0; r < 4; ++r) sdx[(16 * wave + 4 * g4 + r) * LT + c] = dx[r];
     __syncthreads();
     // dS = gamma_C dS' + J - (Gamma K)^T dX
     const float gam_c = sgam[BC - 1];
@@ -1059,12 +820,8 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     for (int m = 0; m < PER; ++m) {
       const int k0 = 16 * (wave + 4 * m);
       float4_t y;
-      if constexpr (L::BF) {
-        y = kt_times_pair(static_cast<const u16 *>(sk), L::LK, k0, gxT, gxT + 16 * LB, LB);
-      } else {
-        y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&sgam[t]); },
-                         [&](int t, int col) { return ld4s(&sdx[t * LT + col], LT); });
-      }
+      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&sgam[t]); },
+                       [&](int t, int col) { return ld4s(&sdx[t * LT + col], LT); });
 #pragma unroll
       for (int r = 0; r < 4; ++r) ds[m][r] = gam_c * ds[m][r] + jv[m][r] - y[r];
     }
@@ -1121,55 +878,34 @@ __global__ __launch_bounds__(BNT) void bwd_scans_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------
 constexpr int GNT = 512;
 
-// Floats of the gradient kernel's area: the value-column tiles during the
-// loop over them (bf16 inputs: S, dS', V/X, dU in float, five transposed bf16
-// pairs and the dO rows; else seven float tiles), then the three C x C
-// matrices (bf16 inputs: one in float, two as bf16 pairs of rows BC + 8).
-template <int K, bool BF>
+// Floats of the gradient kernel's area: the value-column tiles (S, dS', V/X,
+// dO, U, dU, dX) during the loop over them, then the three C x C matrices.
+template <int K>
 constexpr int grad_area() {
-  constexpr int tiles = BF ? 2 * K * LT + 2 * BC * LT + (6 * 2 * 16 * (BC + 8) + BC * 24) / 2 : 2 * K * LT + 5 * BC * LT;
-  constexpr int tri = BF ? 3 * BC * (BC + 8) : 3 * BC * LC;
+  constexpr int tiles = 2 * K * LT + 5 * BC * LT, tri = 3 * BC * LC;
   return tri > tiles ? tri : tiles;
 }
 
 template <int K, int V, typename TIn>
 __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
-  constexpr int LK = K + 16 / sizeof(TIn), KT = K / 16, KH = KT / 2, LS = K + 8;
-  // bf16 inputs: K S, K dS' and Q S on bf16 MFMA (q, k exact; the state
-  // tiles as high + low parts); other input types on the fp32 MFMA
-  constexpr bool BF = std::is_same<TIn, u16>::value;
+  constexpr int LK = K + 16 / sizeof(TIn), KT = K / 16, KH = KT / 2;
   extern __shared__ __align__(16) float lds[];
   PBGDN_POISON_LDS(lds, (grad_lds<K, TIn>()));
   PBGDN_POISON_SYNC();
-  constexpr int LB = BC + 8, LO = 16 + 8, PAIR = 2 * 16 * LB;
-  // T and M: float rows of LC, or (bf16 inputs) bf16 high/low pairs of rows LB
-  constexpr int TSZ = BF ? BC * LB : BC * LC;
+  constexpr int TSZ = BC * LC;
   TIn *sq = reinterpret_cast<TIn *>(lds), *sk = sq + BC * LK;  // q, k rows as they are
   float *st = reinterpret_cast<float *>(sk + BC * LK), *sm = st + TSZ;
-  u16 *tp = reinterpret_cast<u16 *>(st), *mp = reinterpret_cast<u16 *>(sm);
   float *area = sm + TSZ;  // the value-column tiles, then three C x C matrices
   float *ss = area, *sds = ss + K * LT, *sx = sds + K * LT, *sdo = sx + BC * LT, *su = sdo + BC * LT;
   float *sdu = su + BC * LT, *sdx = sdu + BC * LT;
-  // bf16 inputs: the per-tile products take their operands from transposed
-  // bf16 high/low pairs [16][LB] (X^T, dU^T, U^T, (E U)^T, (-Gamma dX)^T,
-  // (beta X)^T) and dO rows as they are [64][LO]; sdu follows sx and these
-  // replace sdo, su, sdx
-  if constexpr (BF) sdu = sx + BC * LT;
-  u16 *xT = reinterpret_cast<u16 *>(sdu + BC * LT), *duT = xT + PAIR, *uT = duT + PAIR, *euT = uT + PAIR,
-      *gxT = euT + PAIR, *bxT = gxT + PAIR, *sdo16 = bxT + PAIR;
   float *b1 = area, *b2 = b1 + BC * LC, *b3 = b2 + BC * LC;
-  // bf16 inputs: dT (then W), dM o Mt and H + H^T as bf16 high/low pairs, rows of LB
-  u16 *b2p = reinterpret_cast<u16 *>(area), *b1p = b2p + 2 * BC * LB, *b3p = b1p + 2 * BC * LB;
-  float *vec = area + grad_area<K, BF>();
+  float *vec = area + grad_area<K>();
   float *sc = vec, *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
   float *sdgam = sbeta + BC, *sde = sdgam + BC;
   // per-wave sums of the dc and dbeta terms: over this wave's token rows
   // [wave][16] and over its two column tiles [wave][32]
   float *prc = sde + BC, *prb = prc + 16 * (GNT / 64), *pcc = prb + 16 * (GNT / 64), *pcb = pcc + 32 * (GNT / 64);
   float *sred = pcb + 32 * (GNT / 64);
-  // bf16 inputs: the tile's S^T and dS'^T as high and low bf16 parts, [16][LS]
-  u16 *shT = reinterpret_cast<u16 *>(sred + GNT / 64 + 8), *slT = shT + 16 * LS, *dhT = slT + 16 * LS,
-      *dlT = dhT + 16 * LS;
   const int h = blockIdx.y;
   BwdSeq seq;
   int i;
@@ -1185,11 +921,7 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
     rk.load(p.k, seq, t0, p.Hk, hk, K);
     rq.put(sq, LK);
     rk.put(sk, LK);
-    if constexpr (BF) {
-      load_t_pair(tp, LB, p.ws_T + rec(p, seq, h, i) * BC * BC);
-    } else {
-      load_t(st, p.ws_T + rec(p, seq, h, i) * BC * BC);
-    }
+    load_t(st, p.ws_T + rec(p, seq, h, i) * BC * BC);
     load_decays(p, seq, h, i, sc, sgam, se, sbeta);
     if (tid < BC) {
       sdgam[tid] = 0.f;
@@ -1200,21 +932,13 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
   // M = scale (Q K^T) o D, this wave's rows and column tiles 2 half, 2 half + 1
   for (int tc = 2 * half; tc < 2 * half + 2; ++tc) {
     float4_t qk;
-    if constexpr (BF) {
-      qk = rows_times_rows<K>(sq, sk, LK, tw, 16 * tc);
-    } else {
-      qk = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sq, (tw + r) * LK + kk); },
-                       [&](int kk, int j) { return ld4e(sk, (16 * tc + j) * LK + kk); });
-    }
+    qk = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sq, (tw + r) * LK + kk); },
+                     [&](int kk, int j) { return ld4e(sk, (16 * tc + j) * LK + kk); });
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = tw + 4 * g4 + r, s2 = 16 * tc + c;
       const float mv = t >= s2 ? p.scale * qk[r] * expf(sc[t] - sc[s2]) : 0.f;
-      if constexpr (BF) {
-        put_pair1(mp, BC * LB, t * LB + s2, mv);
-      } else {
-        sm[t * LC + s2] = mv;
-      }
+      sm[t * LC + s2] = mv;
     }
   }
 
@@ -1254,35 +978,16 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
       const int e = tid + BNT * m;
       *reinterpret_cast<float4_t *>(&ss[(e >> 2) * LT + 4 * (e & 3)]) = rs[m];
       *reinterpret_cast<float4_t *>(&sds[(e >> 2) * LT + 4 * (e & 3)]) = rd[m];
-      if constexpr (BF) {  // column c0 + j of the tile -> row c0 + j of the transposes
-        const int kk = e >> 2, c0 = 4 * (e & 3);
-        v2u32_t hi, lo;
-        split_bf16(rs[m], hi, lo);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          shT[(c0 + j) * LS + kk] = static_cast<u16>(hi[j >> 1] >> (16 * (j & 1)));
-          slT[(c0 + j) * LS + kk] = static_cast<u16>(lo[j >> 1] >> (16 * (j & 1)));
-        }
-        split_bf16(rd[m], hi, lo);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          dhT[(c0 + j) * LS + kk] = static_cast<u16>(hi[j >> 1] >> (16 * (j & 1)));
-          dlT[(c0 + j) * LS + kk] = static_cast<u16>(lo[j >> 1] >> (16 * (j & 1)));
-        }
-      }
     }
     if (tid < BC * PPR) {
       float x[EPP], y[EPP];
       decode16<TIn>(rv, x);
       decode16<TIn>(ro, y);
       const int row = tid / PPR, part = tid % PPR;
-      if constexpr (BF) *reinterpret_cast<uint4 *>(sdo16 + row * LO + part * EPP) = ro;
 #pragma unroll
       for (int j = 0; j < EPP; j += 4) {
         *reinterpret_cast<float4_t *>(&sx[row * LT + part * EPP + j]) = float4_t{x[j], x[j + 1], x[j + 2], x[j + 3]};
-        if constexpr (!BF) {
-          *reinterpret_cast<float4_t *>(&sdo[row * LT + part * EPP + j]) = float4_t{y[j], y[j + 1], y[j + 2], y[j + 3]};
-        }
+        *reinterpret_cast<float4_t *>(&sdo[row * LT + part * EPP + j]) = float4_t{y[j], y[j + 1], y[j + 2], y[j + 3]};
       }
     }
   };
@@ -1297,13 +1002,8 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
     __syncthreads();
     float4_t ks = zero4(), kd = zero4();
     if (chain) {
-      if constexpr (BF) {
-        ks = rows_times_state<K>(sk, LK, tw, shT, slT, LS);
-        kd = rows_times_state<K>(sk, LK, tw, dhT, dlT, LS);
-      } else {
-        ks = tile_mm4<K>(zero4(), in_rows(sk), state_cols(ss));
-        kd = tile_mm4<K>(zero4(), in_rows(sk), state_cols(sds));
-      }
+      ks = tile_mm4<K>(zero4(), in_rows(sk), state_cols(ss));
+      kd = tile_mm4<K>(zero4(), in_rows(sk), state_cols(sds));
       float4_t xv;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -1311,142 +1011,70 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
         xv[r] = sx[t * LT + c] - sgam[t] * ks[r];  // X = V - Gamma K S
         sx[t * LT + c] = xv[r];
       }
-      if constexpr (BF) {
-        put_t_pair(xT, LB, tw + 4 * g4, c, xv);
-        put_t_pair(bxT, LB, tw + 4 * g4, c, xv * ld4(&sbeta[tw + 4 * g4]));
-      }
     } else {
       float4_t qs;
-      if constexpr (BF) {
-        qs = rows_times_state<K>(sq, LK, tw, shT, slT, LS);
-      } else {
-        qs = tile_mm4<K>(zero4(), in_rows(sq), state_cols(ss));
-      }
+      qs = tile_mm4<K>(zero4(), in_rows(sq), state_cols(ss));
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = tw + 4 * g4 + r;
-        dgam_r[r] += p.scale * qs[r] * (BF ? ld_el(sdo16, t * LO + c) : sdo[t * LT + c]);
+        dgam_r[r] += p.scale * qs[r] * sdo[t * LT + c];
       }
     }
     __syncthreads();
     if (chain) {
       float4_t u, du;
-      if constexpr (BF) {  // U = T (beta X), dU0 part M^T dO (M^T, dO columns by transposing reads)
-        u = pair_times_pair<BC>(tp, tp + BC * LB, LB, tw, bxT, bxT + 16 * LB, LB);
-        du = zero4();
-#pragma unroll
-        for (int ts = 0; ts < BC; ts += 32) {
-          const bh8_t dof = tr_frag(sdo16, LO, ts, 0);
-          du = mfma_bf16(tr_frag(mp, LB, ts, tw), dof, du);
-          du = mfma_bf16(tr_frag(mp + BC * LB, LB, ts, tw), dof, du);
-        }
-      } else {
-        u = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4(&st[(tw + r) * LC + s2]) * ld4(&sbeta[s2]); },
-                         [&](int s2, int col) { return ld4s(&sx[s2 * LT + col], LT); });
-        du = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4s(&sm[s2 * LC + tw + r], LC); },
-                          [&](int s2, int col) { return ld4s(&sdo[s2 * LT + col], LT); });
-      }
+      u = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4(&st[(tw + r) * LC + s2]) * ld4(&sbeta[s2]); },
+                       [&](int s2, int col) { return ld4s(&sx[s2 * LT + col], LT); });
+      du = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4s(&sm[s2 * LC + tw + r], LC); },
+                        [&](int s2, int col) { return ld4s(&sdo[s2 * LT + col], LT); });
       float4_t eu;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = tw + 4 * g4 + r;
-        if constexpr (!BF) su[t * LT + c] = u[r];
+        su[t * LT + c] = u[r];
         eu[r] = se[t] * u[r];
         de_r[r] += kd[r] * u[r];
         du[r] += se[t] * kd[r];
         sdu[t * LT + c] = du[r];
       }
-      if constexpr (BF) {
-        put_t_pair(uT, LB, tw + 4 * g4, c, u);
-        put_t_pair(euT, LB, tw + 4 * g4, c, eu);
-        put_t_pair(duT, LB, tw + 4 * g4, c, du);
-      }
     }
     __syncthreads();
     if (chain) {
       float4_t dx;
-      if constexpr (BF) {  // dX = diag(beta) T^T dU
-        dx = tt_times_pair(tp, tp + BC * LB, LB, tw, duT, duT + 16 * LB, LB);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dx[r] *= sbeta[tw + 4 * g4 + r];
-      } else {
-        dx = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4s(&st[s2 * LC + tw + r], LC) * sbeta[tw + r]; },
-                          [&](int s2, int col) { return ld4s(&sdu[s2 * LT + col], LT); });
-      }
+      dx = tile_mm4<BC>(zero4(), [&](int r, int s2) { return ld4s(&st[s2 * LC + tw + r], LC) * sbeta[tw + r]; },
+                        [&](int s2, int col) { return ld4s(&sdu[s2 * LT + col], LT); });
       float4_t gx;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = tw + 4 * g4 + r;
-        if constexpr (!BF) sdx[t * LT + c] = dx[r];
+        sdx[t * LT + c] = dx[r];
         gx[r] = -sgam[t] * dx[r];
         if (t0 + t < seq.len) {
           store_el<TIn>(p.dv, ((seq.bos + t0 + t) * p.Hv + h) * V + v0 + c, dx[r]);
         }
         dgam_r[r] -= ks[r] * dx[r];
       }
-      if constexpr (BF) put_t_pair(gxT, LB, tw + 4 * g4, c, gx);
     }
     for (int e = tid; e < K * 16; e += GNT) dgc += ss[(e >> 4) * LT + (e & 15)] * sds[(e >> 4) * LT + (e & 15)];
     __syncthreads();
     // C x C products over these 16 columns (this wave's two column tiles):
-    // dTb += dU X^T, dM += dO U^T; then dQ += scale Gamma dO S^T (bf16
-    // inputs: the row scale after the loop), dK += E U dS'^T - Gamma dX S^T
-    // (this wave's half of the key tiles)
-    if constexpr (BF) {
-      // A operands of this wave's rows: dU, E U, -Gamma dX pairs, dO as it is
-      const bw_i16x4_t du_h = tr4(duT, LB, tw), du_l = tr4(duT + 16 * LB, LB, tw);
-      const bw_i16x4_t eu_h = tr4(euT, LB, tw), eu_l = tr4(euT + 16 * LB, LB, tw);
-      const bw_i16x4_t gx_h = tr4(gxT, LB, tw), gx_l = tr4(gxT + 16 * LB, LB, tw);
-      const bw_i16x4_t dof = *reinterpret_cast<const bw_i16x4_t *>(sdo16 + (tw + c) * LO + 4 * g4);
+    // dTb += dU X^T, dM += dO U^T; then dQ += scale Gamma dO S^T, dK += E U
+    // dS'^T - Gamma dX S^T (this wave's half of the key tiles)
 #pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        const int tc = 2 * half + m;
-        const bw_i16x4_t x_h = tr4(xT, LB, 16 * tc), x_l = tr4(xT + 16 * LB, LB, 16 * tc);
-        const bw_i16x4_t u_h = tr4(uT, LB, 16 * tc), u_l = tr4(uT + 16 * LB, LB, 16 * tc);
-        dtb[m] = mfma_bf16_k16(du_h, x_h, dtb[m]);
-        dtb[m] = mfma_bf16_k16(du_h, x_l, dtb[m]);
-        dtb[m] = mfma_bf16_k16(du_l, x_h, dtb[m]);
-        dm[m] = mfma_bf16_k16(dof, u_h, dm[m]);
-        dm[m] = mfma_bf16_k16(dof, u_l, dm[m]);
-      }
-#pragma unroll
-      for (int m = 0; m < KH; ++m) {
-        const int kt = half * KH + m;
-        const bw_i16x4_t s_h = tr4(shT, LS, 16 * kt), s_l = tr4(slT, LS, 16 * kt);
-        const bw_i16x4_t d_h = tr4(dhT, LS, 16 * kt), d_l = tr4(dlT, LS, 16 * kt);
-        dq[m] = mfma_bf16_k16(dof, s_h, dq[m]);
-        dq[m] = mfma_bf16_k16(dof, s_l, dq[m]);
-        dk[m] = mfma_bf16_k16(eu_h, d_h, dk[m]);
-        dk[m] = mfma_bf16_k16(eu_h, d_l, dk[m]);
-        dk[m] = mfma_bf16_k16(eu_l, d_h, dk[m]);
-        dk[m] = mfma_bf16_k16(gx_h, s_h, dk[m]);
-        dk[m] = mfma_bf16_k16(gx_h, s_l, dk[m]);
-        dk[m] = mfma_bf16_k16(gx_l, s_h, dk[m]);
-      }
-    } else {
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        const int tc = 2 * half + m;
-        dtb[m] = tile_mm4<16>(dtb[m], rows_of(sdu, LT), [&](int j, int col) { return ld4(&sx[(16 * tc + col) * LT + j]); });
-        dm[m] = tile_mm4<16>(dm[m], rows_of(sdo, LT), [&](int j, int col) { return ld4(&su[(16 * tc + col) * LT + j]); });
-      }
-#pragma unroll
-      for (int m = 0; m < KH; ++m) {
-        const int kt = half * KH + m;
-        auto s_t = [&](int j, int col) { return ld4(&ss[(16 * kt + col) * LT + j]); };
-        dq[m] = tile_mm4<16>(dq[m], [&](int r, int j) { return ld4(&sdo[(tw + r) * LT + j]) * sgam[tw + r] * p.scale; },
-                             s_t);
-        dk[m] = tile_mm4<16>(dk[m], [&](int r, int j) { return ld4(&su[(tw + r) * LT + j]) * se[tw + r]; },
-                             [&](int j, int col) { return ld4(&sds[(16 * kt + col) * LT + j]); });
-        dk[m] = tile_mm4<16>(dk[m], [&](int r, int j) { return ld4(&sdx[(tw + r) * LT + j]) * -sgam[tw + r]; }, s_t);
-      }
+    for (int m = 0; m < 2; ++m) {
+      const int tc = 2 * half + m;
+      dtb[m] = tile_mm4<16>(dtb[m], rows_of(sdu, LT), [&](int j, int col) { return ld4(&sx[(16 * tc + col) * LT + j]); });
+      dm[m] = tile_mm4<16>(dm[m], rows_of(sdo, LT), [&](int j, int col) { return ld4(&su[(16 * tc + col) * LT + j]); });
     }
-  }
-  if constexpr (BF) {  // dQ's row scale, scale Gamma
 #pragma unroll
     for (int m = 0; m < KH; ++m) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dq[m][r] *= sgam[tw + 4 * g4 + r] * p.scale;
+      const int kt = half * KH + m;
+      auto s_t = [&](int j, int col) { return ld4(&ss[(16 * kt + col) * LT + j]); };
+      dq[m] = tile_mm4<16>(dq[m], [&](int r, int j) { return ld4(&sdo[(tw + r) * LT + j]) * sgam[tw + r] * p.scale; },
+                           s_t);
+      dk[m] = tile_mm4<16>(dk[m], [&](int r, int j) { return ld4(&su[(tw + r) * LT + j]) * se[tw + r]; },
+                           [&](int j, int col) { return ld4(&sds[(16 * kt + col) * LT + j]); });
+      dk[m] = tile_mm4<16>(dk[m], [&](int r, int j) { return ld4(&sdx[(tw + r) * LT + j]) * -sgam[tw + r]; }, s_t);
     }
   }
   // per-token sums over the value columns (both halves add into sdgam)
@@ -1473,20 +1101,12 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
       const int t = tw + 4 * g4 + r, s2 = 16 * tc + c;
       const float d = t >= s2 ? p.scale * expf(sc[t] - sc[s2]) : 0.f;
       const float dmv = t >= s2 ? dm[m][r] : 0.f;
-      if constexpr (BF) {
-        put_pair1(b1p, BC * LB, t * LB + s2, dmv * d);
-      } else {
-        b1[t * LC + s2] = dmv * d;
-      }
-      const float dcv = dmv * (BF ? pair_val(mp, BC * LB, t * LB + s2) : sm[t * LC + s2]);
+      b1[t * LC + s2] = dmv * d;
+      const float dcv = dmv * sm[t * LC + s2];
       rc[r] += dcv;
       cc[m] -= dcv;
-      if constexpr (BF) {
-        put_pair1(b2p, BC * LB, t * LB + s2, dtb[m][r] * sbeta[s2]);
-      } else {
-        b2[t * LC + s2] = dtb[m][r] * sbeta[s2];
-      }
-      cb[m] += dtb[m][r] * (BF ? pair_val(tp, BC * LB, t * LB + s2) : st[t * LC + s2]);
+      b2[t * LC + s2] = dtb[m][r] * sbeta[s2];
+      cb[m] += dtb[m][r] * st[t * LC + s2];
     }
   }
   __syncthreads();
@@ -1495,32 +1115,16 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     const int tc = 2 * half + m;
-    if constexpr (BF) {  // T^T and dT's columns by transposing reads of the pairs
-      w4[m] = zero4();
-#pragma unroll
-      for (int ts = 0; ts < BC; ts += 32) {
-        const bh8_t th = tr_frag(tp, LB, ts, tw), tl = tr_frag(tp + BC * LB, LB, ts, tw);
-        const bh8_t dh = tr_frag(b2p, LB, ts, 16 * tc), dl = tr_frag(b2p + BC * LB, LB, ts, 16 * tc);
-        w4[m] = mfma_bf16(th, dh, w4[m]);
-        w4[m] = mfma_bf16(th, dl, w4[m]);
-        w4[m] = mfma_bf16(tl, dh, w4[m]);
-      }
-    } else {
-      w4[m] = tile_mm4<BC>(zero4(), [&](int r, int u2) { return ld4s(&st[u2 * LC + tw + r], LC); },
-                           [&](int u2, int col) { return ld4s(&b2[u2 * LC + 16 * tc + col], LC); });
-    }
+    w4[m] = tile_mm4<BC>(zero4(), [&](int r, int u2) { return ld4s(&st[u2 * LC + tw + r], LC); },
+                         [&](int u2, int col) { return ld4s(&b2[u2 * LC + 16 * tc + col], LC); });
   }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int e = (tw + 4 * g4 + r) * (BF ? LB : LC) + 16 * (2 * half + m) + c;
-      if constexpr (BF) {
-        put_pair1(b2p, BC * LB, e, w4[m][r]);
-      } else {
-        b2[e] = w4[m][r];
-      }
+      const int e = (tw + 4 * g4 + r) * LC + 16 * (2 * half + m) + c;
+      b2[e] = w4[m][r];
     }
   }
   __syncthreads();
@@ -1530,19 +1134,11 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
   for (int m = 0; m < 2; ++m) {
     const int tc = 2 * half + m;
     float4_t da;
-    if constexpr (BF) {  // W rows times T rows (both pairs)
-      da = pair_times_pair<BC>(b2p, b2p + BC * LB, LB, tw, tp + 16 * tc * LB, tp + BC * LB + 16 * tc * LB, LB);
-    } else {
-      da = tile_mm4<BC>(zero4(), [&](int r, int u2) { return ld4(&b2[(tw + r) * LC + u2]); },
-                        [&](int u2, int col) { return ld4(&st[(16 * tc + col) * LC + u2]); });
-    }
+    da = tile_mm4<BC>(zero4(), [&](int r, int u2) { return ld4(&b2[(tw + r) * LC + u2]); },
+                      [&](int u2, int col) { return ld4(&st[(16 * tc + col) * LC + u2]); });
     float4_t gk;
-    if constexpr (BF) {
-      gk = rows_times_rows<K>(sk, sk, LK, tw, 16 * tc);
-    } else {
-      gk = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sk, (tw + r) * LK + kk); },
-                       [&](int kk, int col) { return ld4e(sk, (16 * tc + col) * LK + kk); });
-    }
+    gk = tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4e(sk, (tw + r) * LK + kk); },
+                     [&](int kk, int col) { return ld4e(sk, (16 * tc + col) * LK + kk); });
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = tw + 4 * g4 + r, s2 = 16 * tc + c;
@@ -1554,19 +1150,10 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
         rb[r] += dav * gk[r] * d;
         rc[r] += dav * av;
         cc[m] -= dav * av;
-        if constexpr (BF) {
-          put_pair1(b3p, BC * LB, t * LB + s2, hv);
-          put_pair1(b3p, BC * LB, s2 * LB + t, hv);
-        } else {
-          b3[t * LC + s2] = hv;
-          b3[s2 * LC + t] = hv;
-        }
+        b3[t * LC + s2] = hv;
+        b3[s2 * LC + t] = hv;
       } else if (t == s2) {
-        if constexpr (BF) {
-          put_pair1(b3p, BC * LB, t * LB + s2, 0.f);
-        } else {
-          b3[t * LC + s2] = 0.f;
-        }
+        b3[t * LC + s2] = 0.f;
       }
     }
   }
@@ -1590,28 +1177,8 @@ __global__ __launch_bounds__(GNT) void bwd_grad_kernel(BwdParams p) {
   }
   __syncthreads();
   // dQ += (dM o Mt) K;  dK += (dM o Mt)^T Q + (H + H^T) K
-  if constexpr (BF) {  // K and Q columns by transposing reads (exact), the C x C pairs by rows or transposing reads
 #pragma unroll
-    for (int ts = 0; ts < BC; ts += 32) {
-      const int o = (tw + c) * LB + ts + 8 * g4;
-      const bh8_t a1h = *reinterpret_cast<const bh8_t *>(b1p + o), a1l = *reinterpret_cast<const bh8_t *>(b1p + BC * LB + o);
-      const bh8_t a3h = *reinterpret_cast<const bh8_t *>(b3p + o), a3l = *reinterpret_cast<const bh8_t *>(b3p + BC * LB + o);
-      const bh8_t t1h = tr_frag(b1p, LB, ts, tw), t1l = tr_frag(b1p + BC * LB, LB, ts, tw);
-#pragma unroll
-      for (int m = 0; m < KH; ++m) {
-        const int kt = half * KH + m;
-        const bh8_t kf = tr_frag(sk, LK, ts, 16 * kt), qf = tr_frag(sq, LK, ts, 16 * kt);
-        dq[m] = mfma_bf16(a1h, kf, dq[m]);
-        dq[m] = mfma_bf16(a1l, kf, dq[m]);
-        dk[m] = mfma_bf16(t1h, qf, dk[m]);
-        dk[m] = mfma_bf16(t1l, qf, dk[m]);
-        dk[m] = mfma_bf16(a3h, kf, dk[m]);
-        dk[m] = mfma_bf16(a3l, kf, dk[m]);
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < (BF ? 0 : KH); ++m) {
+  for (int m = 0; m < KH; ++m) {
     const int kt = half * KH + m;
     auto kcol = [&](int s2, int col) { return ld4es(sk, s2 * LK + 16 * kt + col, LK); };
     dq[m] = tile_mm4<BC>(dq[m], [&](int r, int s2) { return ld4(&b1[(tw + r) * LC + s2]); }, kcol);
@@ -1697,9 +1264,7 @@ constexpr size_t scan_lds() { return ScanLds<K, TIn>::BYTES; }
 template <int K, typename TIn>
 constexpr size_t grad_lds() {
   return sizeof(TIn) * 2 * BC * (K + 16 / sizeof(TIn)) +
-         sizeof(float) * (2 * (std::is_same<TIn, u16>::value ? BC * (BC + 8) : BC * LC) +
-                          grad_area<K, std::is_same<TIn, u16>::value>() + 6 * BC + 96 * (GNT / 64) + GNT / 64 + 8) +
-         (std::is_same<TIn, u16>::value ? sizeof(u16) * 4 * 16 * (K + 8) : 0);
+         sizeof(float) * (2 * BC * LC + grad_area<K>() + 6 * BC + 96 * (GNT / 64) + GNT / 64 + 8);
 }
 
 template <typename Kern>
@@ -1757,7 +1322,7 @@ int run_scans_bf16(const BwdParams &p, hipStream_t st) {
 
 template <int K, int V>
 int run_backward(const BwdParams &p, hipStream_t st) {
-  static_assert(grad_lds<K, float>() <= 160 * 1024 && grad_lds<K, u16>() <= 160 * 1024 && local_lds<K, V, float>() <= 160 * 1024, "LDS budget");
+  static_assert(grad_lds<K, float>() <= 160 * 1024 && local_lds<K, V, float>() <= 160 * 1024, "LDS budget");
   const dim3 per_chunk(p.cu_seqlens ? p.records : p.n, p.Hv, p.B), per_tile2((V / 16) * p.Hv * 2 * p.num_seqs);
   int rc = PBGDN_OK;
   if (p.records > 0) {
