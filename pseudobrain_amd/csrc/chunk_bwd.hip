@@ -70,6 +70,7 @@ struct BwdParams {
   int in_dtype, beta_dtype;
   int B, T, Hk, Hv, K, V, n;  // n: chunks of a batch row
   float scale;
+  bool narrow;  // dq, dk or dv not 8-byte aligned
   int cus, xcds;  // the device's compute units and XCDs (device.hpp)
 };
 
@@ -1281,8 +1282,9 @@ int launch(Kern kernel, dim3 grid, size_t lds, hipStream_t st, const BwdParams &
 // takes in turn: all of them (dq and dk are then summed in registers, with no
 // float32 copies per value head and no reduction pass), unless the call is so
 // small that one head per workgroup (one workgroup a CU) needs fewer rounds of
-// the CUs by more than a quarter: the reduction and the float32 copies cost
-// about an eighth (67 us beside 13 rounds of 30 us at 6,011 tokens of 32 heads).
+// the CUs by more than a quarter: the reduction and the float32 copies cost a
+// sixth to a fifth (at 6,011 tokens of 32 heads 414 + 67 us against 409, at
+// 4 x 2,048 542 + 92 against 514).
 int grad_heads(const BwdParams &p) {
   const long group = p.Hv / p.Hk, items = static_cast<long>(p.records) * p.Hk, cus = p.cus > 0 ? p.cus : 1;
   const long together = (items + cus - 1) / cus * group, apart = (items * group + cus - 1) / cus;
@@ -1313,7 +1315,10 @@ int launch_scans_bf16(const BwdParams &p, hipStream_t st) {
 }
 
 // The scans of bf16 inputs: 64 value columns a workgroup (four computing
-// waves) where that gives every CU a workgroup, else 32.
+// waves) where that gives every CU a workgroup, else 32. K = V = 128, 32 heads:
+// 4 x 2,048 tokens (512 workgroups of 64) 238 us against 351 with 32 columns,
+// packed 6,011 tokens of 7 sequences 239 against 302; 1 x 32,768 (128 of 64, 256
+// of 32) 1,716 against 1,380.
 template <int K>
 int run_scans_bf16(const BwdParams &p, hipStream_t st) {
   const long wide = 2L * p.num_seqs * p.Hv * (p.V / 64);
@@ -1461,6 +1466,7 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
   p.V = V;
   p.n = static_cast<int>(n);
   p.scale = scale;
+  p.narrow = ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) & 7) != 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (K == 64) return V == 64 ? run_backward<64, 64>(p, st) : run_backward<64, 128>(p, st);
   return V == 64 ? run_backward<128, 64>(p, st) : run_backward<128, 128>(p, st);

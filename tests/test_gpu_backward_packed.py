@@ -82,3 +82,23 @@ def test_many_heads_equal_few(dk, dv):
             for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta"), got, ref):
                 assert torch.equal(a[one, :, :2], b), f"{name} of row {n}, length {length}"
             assert torch.equal(got[5][one, :2], ref[5])
+
+
+@pytest.mark.parametrize("hk,hv", [(2, 2), (1, 2)])
+def test_outputs_of_any_alignment(monkeypatch, hk, hv):
+    """dq, dk and dv at addresses that are no multiple of 8 bytes: the same values."""
+    q, k, v, g, beta, h0 = (x.to(DEV) for x in generate(1, 100, hk, hv, 128, 128, torch.bfloat16, 0.05, seed=6))
+    gen = torch.Generator().manual_seed(6)
+    do = (torch.randn(1, 100, hv, 128, generator=gen) * 0.1).to(torch.bfloat16).to(DEV)
+    want = gd.chunk_bwd(q, k, v, g, beta, 0.1, h0, do)
+
+    def one_element_off(x, **kw):
+        return torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty_like", one_element_off)
+        got = gd.chunk_bwd(q, k, v, g, beta, 0.1, h0, do)
+    torch.cuda.synchronize()
+    assert got[0].data_ptr() % 8 == 2
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
