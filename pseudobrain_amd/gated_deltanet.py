@@ -30,10 +30,9 @@ for 256-wide keys with 16-bit inputs, and token by token through the
 recurrent kernel with float32 inputs.
 
 Gradients. gated_delta_rule's device paths are differentiable through the chunk
-operator's backward (pbgdn::gated_delta_chunk, for K, V <= 128; a packed
-call's backward runs sequence by sequence); a training call through
-"sequential" (T <= SEQUENTIAL_MAX) takes the
-same operator. The lower-level entry points (chunk_fwd, chunk_fwd_slots,
+operator's backward (pbgdn::gated_delta_chunk_f32, for K, V <= 128, batches
+and packed sequences alike); a training call through "sequential" (T <=
+SEQUENTIAL_MAX) takes the same operator. The lower-level entry points (chunk_fwd, chunk_fwd_slots,
 recurrent_fwd, the decode and slot ops, the layer kernels in
 pseudobrain_amd.layer) have no backward: with grad mode on and an input that
 requires grad they raise instead of returning tensors cut from the graph.
