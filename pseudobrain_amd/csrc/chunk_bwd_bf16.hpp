@@ -19,8 +19,11 @@
 //            dK2 = dX S^T, dQ0 = dO S^T (64 x K).
 //   C x C    the gradient through M, T and A, and the sums for dg and dbeta.
 //
-// Row sums that would need K S, K dS' or Q S again come from the K-wide
-// products: sum_v (K dS' o U)_t = sum_k (K o dK1)_t, likewise with dX and dQ0.
+// The decay sums sum_v (K dS' o U)_t and sum_v (K S o dX)_t are formed in the
+// chain, where all four are in float32: as sums over the keys of K o dK1 and K o
+// dK2, whose products take U and dX as bf16 pairs, they left dg with 1.2 to 1.9
+// times its error against 64 bits (and the kernel 1% slower). sum_v (Q S o dO)_t does come from the keys
+// (sum_k (Q o dQ0)_t): dO is exact in bf16 there.
 // LDS: 134 KiB at K = V = 128, so one workgroup a CU, eight waves.
 //
 // 3.55 (16-column tiles in turn, with the reduction) -> 1.71 ms at 1 x 32,768
@@ -124,7 +127,7 @@ struct GradLds {
   static constexpr int USED = 4 * TV > 2 * TV + V * K ? 4 * TV : 2 * TV + V * K,
                        AREA = USED > 8 * CC ? USED : 8 * CC;
   static_assert(2 * CC + BC * V <= AREA && 2 * TV + V * K <= AREA, "the area's uses");
-  static constexpr int FLOATS = 4 * BC + 4 * COLS * BC + 4 * BC + 16;
+  static constexpr int FLOATS = 4 * BC + 3 * COLS * BC + NW * BC + 4 * BC + 16;
   static constexpr size_t BYTES = sizeof(u16) * (2 * BC * K + BC * V + 2 * CC + AREA) + sizeof(float) * FLOATS;
 };
 
@@ -276,9 +279,10 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     u16 *sq = reinterpret_cast<u16 *>(lds + base), *sk = sq + BC * K, *sdo = sk + BC * K, *tp = sdo + BC * V,
         *area = tp + 2 * CC;
     float *sc = reinterpret_cast<float *>(area + L::AREA), *sgam = sc + BC, *se = sgam + BC, *sbeta = se + BC;
-    // partial sums: rows by wave pair (dc, dbeta, dgamma, de), columns by wave parity
-    float *prc = sbeta + BC, *prb = prc + COLS * BC, *pdg = prb + COLS * BC, *pde = pdg + COLS * BC;
-    float *pcc = pde + COLS * BC, *pcb = pcc + 2 * BC, *sred = pcb + 2 * BC;
+    // partial sums: rows by wave pair (dc, dbeta, dgamma's part of Q S) and by
+    // wave (the chain's decay sums), columns by wave parity
+    float *prc = sbeta + BC, *prb = prc + COLS * BC, *pdg = prb + COLS * BC, *pch = pdg + COLS * BC;
+    float *pcc = pch + NW * BC, *pcb = pcc + 2 * BC, *sred = pcb + 2 * BC;
     const int h = it.block * heads + hh, t0 = it.i * BC, left = it.seq.len - t0;  // the chunk's tokens: left, if under BC
     const long row0 = it.seq.bos + t0;
     // ---- this head's inputs into LDS
@@ -314,10 +318,8 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       split_bf16(df[m], dh[m], dl[m]);
     }
     keep_order();
-    dgc = wave_sum(dgc);
-    if (lane == 0) sred[wave] = dgc;
-    float4_t du[4];
-    v2u32_t xh[4], xl[4], bxh[4], bxl[4];
+    float4_t x[4], du[4], ekd[4];  // X; E K dS' + M^T dO, and E K dS' alone
+    v2u32_t bxh[4], bxl[4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
       float4_t ks = zero4(), kd = zero4();
@@ -330,12 +332,22 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         kd = mfma_bf16(a, frag_pair(dl[2 * kb], dl[2 * kb + 1]), kd);
       }
       const int o = 16 * rt + 4 * g4;
-      const float4_t x = bf16x4_float(L4.tr<V>(sv, 16 * rt, v0)) - ld4(&sgam[o]) * ks;
-      split_bf16(x, xh[rt], xl[rt]);
-      split_bf16(x * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
-      du[rt] = ld4(&se[o]) * kd;
+      x[rt] = bf16x4_float(L4.tr<V>(sv, 16 * rt, v0)) - ld4(&sgam[o]) * ks;
+      split_bf16(x[rt] * ld4(&sbeta[o]), bxh[rt], bxl[rt]);
+      du[rt] = ekd[rt] = ld4(&se[o]) * kd;
       keep_order();
     }
+    // The chain's decay sums, over this wave's columns: to d/dc of token t
+    // -(E K dS' o U + Gamma K S o dX), with V - X for Gamma K S (no registers for
+    // it); to that of the last one gamma_C S . dS' and all of E K dS' o U.
+    dgc *= sgam[BC - 1];
+    float4_t dch = zero4();  // element rt: token 16 rt + 4 g + (c & 3), over the columns of four lanes
+    auto add_rows = [&](float4_t y, int rt) {  // four sums over four lanes, one left in each
+      const bool odd = c & 1, upper = c & 2;
+      const float y01 = (odd ? y[1] : y[0]) + dpp_mov<0xb1>(odd ? y[0] : y[1]);
+      const float y23 = (odd ? y[3] : y[2]) + dpp_mov<0xb1>(odd ? y[2] : y[3]);
+      dch[rt] += (upper ? y23 : y01) + dpp_mov<0x4e>(upper ? y01 : y23);
+    };
     v2u32_t duh[4], dul[4];
     {
       bh8_t dof[2];
@@ -351,10 +363,10 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         split_bf16(du[rt], duh[rt], dul[rt]);
       }
     }
-    v2u32_t uh[4], ul[4], dxh[4], dxl[4];
+    v2u32_t xh[4], xl[4], dxh[4], dxl[4], uh[4], ul[4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
-      float4_t u = zero4(), dx = zero4();
+      float4_t dx = zero4(), u = zero4();
 #pragma unroll
       for (int kb = 0; kb <= rt >> 1; ++kb) {  // U = T (beta X), s <= t
         const bh8_t th = L4.rows<BC>(tp, 16 * rt, kb), tl = L4.rows<BC>(tp + CC, 16 * rt, kb);
@@ -372,10 +384,23 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
         dx = mfma_bf16(tl, bh, dx);
       }
       dx *= ld4(&sbeta[16 * rt + 4 * g4]);
+      const float4_t eu = ekd[rt] * u;
+      dgc += (eu[0] + eu[1]) + (eu[2] + eu[3]);
+      add_rows(eu + (bf16x4_float(L4.tr<V>(sv, 16 * rt, v0)) - x[rt]) * dx, rt);
       split_bf16(u, uh[rt], ul[rt]);
+      split_bf16(x[rt], xh[rt], xl[rt]);
       split_bf16(dx, dxh[rt], dxl[rt]);
       keep_order();
     }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {  // over the other lanes of the row: rotations by 8 and 4
+      dch[rt] += dpp_mov<0x128>(dch[rt]);
+      dch[rt] += dpp_mov<0x124>(dch[rt]);
+    }
+    pch[wave * BC + 16 * (c >> 2) + 4 * g4 + (c & 3)] =
+        c < 8 ? (c < 4 ? dch[0] : dch[1]) : (c < 12 ? dch[2] : dch[3]);
+    dgc = wave_sum(dgc);
+    if (lane == 0) sred[wave] = dgc;
     renew();
     // ---- contractions over the value columns
     u16 *a0 = area, *a1 = area + 2 * TV;
@@ -469,22 +494,12 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     renew();
-    // dK1's row scale, and its part of the decay sums over the keys
+    // dK1's row scale
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-      const int o = 32 * rp + 16 * a + 4 * g4;
-      const float4_t e4 = ld4(&se[o]);
-      float4_t de = zero4();
+      const float4_t e4 = ld4(&se[32 * rp + 16 * a + 4 * g4]);
 #pragma unroll
-      for (int m = 0; m < KTW; ++m) {
-        de += bf16x4_float(L4.tr<K>(sk, 32 * rp + 16 * a, 16 * (KTW * cp + m))) * dk1[m][a];
-        tk[m][a] += e4 * dk1[m][a];
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float y = group_sum(de[e], 16);
-        if (c == 0) pde[cp * BC + o + e] = y;
-      }
+      for (int m = 0; m < KTW; ++m) tk[m][a] += e4 * dk1[m][a];
     }
     __syncthreads();
     renew();
@@ -549,7 +564,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
       }
     }
     renew();
-    // ---- the other row scales and decay sums
+    // ---- the other row scales, and Q S's part of the decay sums over the keys
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
       const int o = 32 * rp + 16 * a + 4 * g4;
@@ -558,9 +573,7 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
 #pragma unroll
       for (int m = 0; m < KTW; ++m) {
         const int col = 16 * (KTW * cp + m);
-        const float4_t kx = bf16x4_float(L4.tr<K>(sk, 32 * rp + 16 * a, col));
-        const float4_t qx = bf16x4_float(L4.tr<K>(sq, 32 * rp + 16 * a, col));
-        dgam += p.scale * (qx * dq0[m][a]) - kx * dk2[m][a];
+        dgam += p.scale * (bf16x4_float(L4.tr<K>(sq, 32 * rp + 16 * a, col)) * dq0[m][a]);
         tq[m][a] += dq0[m][a] * (gam * p.scale);
         tk[m][a] -= gam * dk2[m][a];
       }
@@ -725,19 +738,20 @@ __global__ __launch_bounds__(4 * V) void bwd_grad_bf16_kernel(BwdParams p, int h
     }
     if (wave == 0) {  // dc -> dg = reverse cumulative sum within the chunk
       const int t = lane;
-      float dct = pcc[t] + pcc[BC + t], dbt = pcb[t] + pcb[BC + t], dgam = 0.f, de = 0.f, gc = 0.f;
+      float dct = pcc[t] + pcc[BC + t], dbt = pcb[t] + pcb[BC + t], dgam = 0.f, dch = 0.f, gc = 0.f;
 #pragma unroll
       for (int m = 0; m < COLS; ++m) {
         dct += prc[m * BC + t];
         dbt += prb[m * BC + t];
         dgam += pdg[m * BC + t];
-        de += pde[m * BC + t];
       }
 #pragma unroll
-      for (int w = 0; w < NW; ++w) gc += sred[w];
-      float dcv = dct + dgam * sgam[t] - de * se[t];
-      const float tail = wave_sum(de * se[t]);
-      if (t == BC - 1) dcv += tail + gc * sgam[BC - 1];
+      for (int w = 0; w < NW; ++w) {
+        dch += pch[w * BC + t];
+        gc += sred[w];
+      }
+      float dcv = dct + dgam * sgam[t] - dch;
+      if (t == BC - 1) dcv += gc;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
         const float y = __shfl_down(dcv, off, 64);
