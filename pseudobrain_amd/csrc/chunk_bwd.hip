@@ -1337,6 +1337,7 @@ int run_backward(const BwdParams &p, hipStream_t st) {
       default: rc = launch(bwd_local_kernel<K, V, half_t>, per_chunk, local_lds<K, V, half_t>(), st, p); break;
     }
   }
+  if (p.num_seqs == 0) return rc;  // no sequence: the local kernel has written the rows' zeros
   if (rc == PBGDN_OK) {  // both scans in one launch (with T = 0 only the reverse one writes: dh0 = dht)
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_scans_kernel<K, float>, per_tile2, scan_lds<K, float>(), st, p); break;

@@ -51,6 +51,20 @@ def test_packed_equals_each_sequence_alone(bounds, total, hk, hv, dk, dv, dtype)
         assert not a[:, :bounds[0]].any() and not a[:, bounds[-1]:].any()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("total", [70, 0])
+def test_no_sequence(dtype, total):
+    """cu_seqlens of one bound: every row gets zeros, and there is no dh0."""
+    q, k, v, g, beta, h0, do, dht, cu = make([0], total, 1, 2, 64, 64, dtype, seed=8)
+    leaves = [x.requires_grad_() for x in (q, k, v, g, beta)]
+    o, final = gd.gated_delta_rule(*leaves, 0.1, h0, "hip", cu)
+    grads = torch.autograd.grad([o, final], leaves, [do.to(o.dtype), dht])
+    torch.cuda.synchronize()
+    for x, grad in zip(leaves, grads):
+        assert grad.shape == x.shape and not grad.any()
+    assert packed(*(x.detach() for x in leaves), h0, do, dht, cu)[5].shape == (0, 2, 64, 64)
+
+
 def test_groups_of_sequences_equal_one_call(monkeypatch):
     bounds = [2, 90, 90, 300, 301, 420]
     args = make(bounds, 450, 1, 2, 64, 64, torch.bfloat16, seed=4)
