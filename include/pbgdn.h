@@ -61,7 +61,8 @@
 extern "C" {
 #endif
 
-#define PBGDN_ABI_VERSION 14
+/* Raised with every function that is added or changed. */
+#define PBGDN_ABI_VERSION 15
 
 /* element types */
 #define PBGDN_F32 0

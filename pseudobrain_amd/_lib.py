@@ -16,7 +16,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime before the library)
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libpbgdn.so")
 # The debug build of the same sources (build.py): LDS and outputs poisoned with NaN.
 DEBUG_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libpbgdn_debug.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 F32, BF16, F16 = 0, 1, 2
 OK, ERR_INVALID_ARGUMENT, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_SCRATCH = 0, 1, 2, 3, 4
@@ -74,19 +74,26 @@ class PbgdnError(RuntimeError):
         super().__init__(f"{where}: pbgdn status {status}: {status_string(status)}")
 
 
+def _declare(handle: ctypes.CDLL, name: str) -> None:
+    fn = getattr(handle, name)
+    fn.argtypes, fn.restype = SIGNATURES[name]
+
+
 def _load(path: str) -> ctypes.CDLL:
     if not os.path.exists(path):
         raise RuntimeError(
             f"pbgdn HIP library not found at {path}; build it with "
             "`python -m pseudobrain_amd.build` (there is no CPU fallback)")
     handle = ctypes.CDLL(path)
-    for name, (args, res) in SIGNATURES.items():
-        fn = getattr(handle, name)
-        fn.argtypes = args
-        fn.restype = res
-    version = handle.pbgdn_abi_version()
-    if version != ABI_VERSION:
-        raise RuntimeError(f"{os.path.basename(path)} ABI version {version}, expected {ABI_VERSION}; rebuild it")
+    try:  # the version before the other symbols: an older library lacks some of them
+        _declare(handle, "pbgdn_abi_version")
+        version = handle.pbgdn_abi_version()
+        if version != ABI_VERSION:
+            raise RuntimeError(f"{os.path.basename(path)} ABI version {version}, expected {ABI_VERSION}; rebuild it")
+        for name in SIGNATURES:
+            _declare(handle, name)
+    except AttributeError as e:
+        raise RuntimeError(f"{os.path.basename(path)} lacks a function of ABI {ABI_VERSION} ({e}); rebuild it") from e
     return handle
 
 

@@ -3,6 +3,8 @@ and rejects bad arguments with status codes before any launch (no GPU needed).""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -28,7 +30,7 @@ def test_library_exports_every_declared_symbol():
 
 
 def test_abi_version_and_status_strings():
-    assert _lib.lib().pbgdn_abi_version() == _lib.ABI_VERSION == 14
+    assert _lib.lib().pbgdn_abi_version() == _lib.ABI_VERSION == 15
     header = open(HEADER).read()
     assert re.search(r"#define PBGDN_ABI_VERSION (\d+)", header).group(1) == str(_lib.ABI_VERSION)
     assert _lib.status_string(0) == "ok"
@@ -36,6 +38,19 @@ def test_abi_version_and_status_strings():
         assert _lib.status_string(code)
     with pytest.raises(_lib.PbgdnError, match="status 2"):
         _lib.check(2, "x")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host C++ compiler")
+@pytest.mark.parametrize("version,message", [(_lib.ABI_VERSION - 1, "ABI version"), (_lib.ABI_VERSION, "lacks")])
+def test_a_stale_library_is_named_as_such(tmp_path, version, message):
+    """A library of another version, or one without a declared function, says to
+    rebuild it rather than which symbol ctypes missed."""
+    stub = tmp_path / "stub.cpp"
+    stub.write_text(f'extern "C" int pbgdn_abi_version(void) {{ return {version}; }}\n')
+    lib = tmp_path / "libstub.so"
+    subprocess.run(["g++", "-shared", "-fPIC", str(stub), "-o", str(lib)], check=True)
+    with pytest.raises(RuntimeError, match=f"{message}.*rebuild it"):
+        _lib._load(str(lib))
 
 
 FAKE = 0x1000  # never dereferenced: every call below fails validation first
