@@ -440,8 +440,10 @@ int pbgdn_prologue_varlen_fwd(const void *qkv, long qkv_stride,
  *   dbeta       [B, T, Hv] beta_dtype
  *   dh0         [B, Hv, K, V] float32, or NULL when not wanted
  *   workspace   device scratch of pbgdn_chunk_bwd_workspace_size(B, T, Hk,
- *               Hv, K, V) bytes, 16-byte aligned, no initialisation needed
- *               (per chunk: its start state, end adjoint, T, the dO terms)
+ *               Hv, K, V) bytes, or of the fewer that
+ *               pbgdn_chunk_bwd_workspace_size_dtype gives, 16-byte aligned, no
+ *               initialisation needed (per chunk: its start state, end
+ *               adjoint, T, the dO terms)
  *
  * Supported: K, V in {64, 128}; at most 65,535 chunks per sequence and
  * 32,767 batch rows.
@@ -454,9 +456,18 @@ int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int in_dtype,
                     size_t workspace_bytes, int B, int T, int Hk, int Hv,
                     int K, int V, float scale, void *stream);
 
-/* Workspace bytes pbgdn_chunk_bwd needs for these sizes. */
+/* Workspace bytes with which pbgdn_chunk_bwd runs these sizes in any dtype. */
 size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K,
                                       int V);
+/*
+ * What in_dtype needs of them on the current device: for B rows of T tokens
+ * (num_seqs -1), or for num_seqs sequences packed into T rows (B 1). bfloat16
+ * needs two thirds of float32's records at K = V = 128, and no float32 dq and
+ * dk per value head except in calls of few chunks. 0 for invalid arguments.
+ */
+size_t pbgdn_chunk_bwd_workspace_size_dtype(int in_dtype, int B, int T,
+                                            int num_seqs, int Hk, int Hv,
+                                            int K, int V);
 
 /*
  * The same for num_seqs independent sequences packed along T (q .. dout
@@ -465,7 +476,8 @@ size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K,
  * [0, T] whatever it holds), with its own h0, dht and dh0 row ([num_seqs, Hv,
  * K, V]). An empty sequence's dh0 is its dht. Rows of no sequence get zero
  * gradients. One call's launches for all sequences and no host read of
- * cu_seqlens. Workspace: pbgdn_chunk_bwd_packed_workspace_size bytes.
+ * cu_seqlens. Workspace: pbgdn_chunk_bwd_packed_workspace_size bytes, or
+ * pbgdn_chunk_bwd_workspace_size_dtype's.
  */
 int pbgdn_chunk_bwd_packed(const void *q, const void *k, const void *v,
                            int in_dtype, const float *g, const void *beta,

@@ -54,6 +54,7 @@ SIGNATURES = {
     "pbgdn_chunk_bwd": ([_vp, _vp, _vp, _i, _vp, _vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                          _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _i, _f, _vp], _i),
     "pbgdn_chunk_bwd_workspace_size": ([_i, _i, _i, _i, _i, _i], ctypes.c_size_t),
+    "pbgdn_chunk_bwd_workspace_size_dtype": ([_i, _i, _i, _i, _i, _i, _i, _i], ctypes.c_size_t),
     "pbgdn_chunk_bwd_packed": ([_vp, _vp, _vp, _i, _vp, _vp, _i, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp,
                                 _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _f, _vp], _i),
     "pbgdn_chunk_bwd_packed_workspace_size": ([_i, _i, _i, _i, _i, _i], ctypes.c_size_t),

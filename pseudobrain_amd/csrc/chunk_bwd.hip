@@ -61,8 +61,9 @@ struct BwdParams {
   void *dbeta;
   float *dh0;
   // ws_T: T, 64 x 64 a record in float32 (bf16 inputs: as a bf16 pair, the
-  // high halves' rows, then the low ones); ws_M (bf16 inputs, in ws_dU0's
-  // bytes): M^T, a pair like it
+  // high halves' rows, then the low ones). bf16 inputs: ws_M, M^T, a pair like
+  // it; others: ws_dU0 and ws_J. ws_dq, ws_dk: per value head, NULL where the
+  // gradient kernel writes dq and dk itself.
   float *ws_T, *ws_c, *ws_beta, *ws_dU0, *ws_M, *ws_J, *ws_S, *ws_dS, *ws_dq, *ws_dk;
   const int32_t *cu_seqlens;  // [num_seqs + 1] bounds of packed sequences (B = 1), or NULL: B rows of T tokens
   int num_seqs;               // sequences: B without cu_seqlens
@@ -1285,8 +1286,8 @@ int launch(Kern kernel, dim3 grid, size_t lds, hipStream_t st, const BwdParams &
 // the CUs by more than a quarter: the reduction and the float32 copies cost a
 // sixth to a fifth (at 6,011 tokens of 32 heads 414 + 67 us against 409, at
 // 4 x 2,048 542 + 92 against 514).
-int grad_heads(const BwdParams &p) {
-  const long group = p.Hv / p.Hk, items = static_cast<long>(p.records) * p.Hk, cus = p.cus > 0 ? p.cus : 1;
+int grad_heads(long records, int Hk, int Hv, int cus) {
+  const long group = Hv / Hk, items = records * Hk;
   const long together = (items + cus - 1) / cus * group, apart = (items * group + cus - 1) / cus;
   return 4 * together <= 5 * apart ? static_cast<int>(group) : 1;
 }
@@ -1326,7 +1327,7 @@ int run_scans_bf16(const BwdParams &p, hipStream_t st) {
 }
 
 template <int K, int V>
-int run_backward(const BwdParams &p, hipStream_t st) {
+int run_backward(const BwdParams &p, int heads, hipStream_t st) {
   static_assert(grad_lds<K, float>() <= 160 * 1024 && local_lds<K, V, float>() <= 160 * 1024, "LDS budget");
   const dim3 per_chunk(p.cu_seqlens ? p.records : p.n, p.Hv, p.B), per_tile2((V / 16) * p.Hv * 2 * p.num_seqs);
   int rc = PBGDN_OK;
@@ -1345,14 +1346,10 @@ int run_backward(const BwdParams &p, hipStream_t st) {
       default: rc = launch(bwd_scans_kernel<K, half_t>, per_tile2, scan_lds<K, half_t>(), st, p); break;
     }
   }
-  int heads = 1;  // value heads of a gradient workgroup
   if (rc == PBGDN_OK && p.records > 0) {
     switch (p.in_dtype) {
       case PBGDN_F32: rc = launch(bwd_grad_kernel<K, V, float>, per_chunk, grad_lds<K, float>(), st, p, GNT); break;
-      case PBGDN_BF16:
-        heads = grad_heads(p);
-        rc = launch_grad_bf16<K, V>(p, heads, st);
-        break;
+      case PBGDN_BF16: rc = launch_grad_bf16<K, V>(p, heads, st); break;
       default: rc = launch(bwd_grad_kernel<K, V, half_t>, per_chunk, grad_lds<K, half_t>(), st, p, GNT); break;
     }
   }
@@ -1365,9 +1362,10 @@ int run_backward(const BwdParams &p, hipStream_t st) {
   return rc;
 }
 
-// Workspace floats per (batch, value head, chunk), and the GQA scratch.
-long ws_record_floats(int K, int V) {
-  return static_cast<long>(BC) * BC + 2 * BC + static_cast<long>(BC) * V + 3L * K * V;
+// Workspace floats of a record (one chunk of one value head): T, c, beta, S, dS'
+// and, with bf16 inputs, M^T, else dU0 and J.
+long ws_record_floats(int in_dtype, int K, int V) {
+  return BC * BC + 2 * BC + 2L * K * V + (in_dtype == PBGDN_BF16 ? BC * BC : static_cast<long>(BC) * V + 1L * K * V);
 }
 
 }  // namespace
@@ -1376,9 +1374,17 @@ long ws_record_floats(int K, int V) {
 namespace pbgdn {
 namespace {
 
-size_t workspace_bytes_of(long records, long tokens, int Hk, int Hv, int K, int V) {
-  long floats = records * Hv * ws_record_floats(K, V);
-  if (Hk != Hv) floats += 2L * tokens * Hv * K;
+// Value heads a gradient workgroup takes in turn: one, or (bf16 inputs) what
+// grad_heads chooses. Without a device (cus 0) the one that needs more workspace.
+int heads_of(int in_dtype, long records, int Hk, int Hv, int cus) {
+  return in_dtype == PBGDN_BF16 && cus > 0 ? grad_heads(records, Hk, Hv, cus) : 1;
+}
+
+// The records, and dq and dk per value head in float32 where the gradient
+// kernel's items are not whole groups of value heads.
+size_t workspace_bytes_of(int in_dtype, long records, long tokens, int Hk, int Hv, int K, int V, int cus) {
+  long floats = records * Hv * ws_record_floats(in_dtype, K, V);
+  if (heads_of(in_dtype, records, Hk, Hv, cus) * Hk != Hv) floats += 2L * tokens * Hv * K;
   return static_cast<size_t>(floats) * sizeof(float) + 256;
 }
 
@@ -1406,10 +1412,15 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
   if (B == 0) return PBGDN_OK;
   if ((!cu_seqlens && n > 65535) || records > (1L << 22) || Hv > 65535 || B > 32767) return PBGDN_ERR_UNSUPPORTED;
   if (static_cast<long>(V / 16) * Hv * 2 * num_seqs > 0x7fffffffL) return PBGDN_ERR_UNSUPPORTED;  // the scans' 1-D grid
-  if (!workspace || workspace_bytes < workspace_bytes_of(records, static_cast<long>(B) * T, Hk, Hv, K, V) ||
-      reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
+  DeviceShape shape{};
+  const bool have_device = device_shape(shape);
+  if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 ||
+      workspace_bytes < workspace_bytes_of(in_dtype, records, static_cast<long>(B) * T, Hk, Hv, K, V, shape.cus)) {
     return PBGDN_ERR_INVALID_ARGUMENT;
   }
+  if (!have_device) return PBGDN_ERR_LAUNCH;
+  const int heads = heads_of(in_dtype, records, Hk, Hv, shape.cus);
+  const bool bf16 = in_dtype == PBGDN_BF16, per_head = heads * Hk != Hv;
   float *ws = static_cast<float *>(workspace);
   const long recs = records * Hv;
   {  // debug builds: the gradients and the workspace start as NaN
@@ -1425,8 +1436,6 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
     debug_poison(workspace, workspace_bytes, s);
   }
   BwdParams p{};
-  DeviceShape shape;
-  if (!device_shape(shape)) return PBGDN_ERR_LAUNCH;
   p.cus = shape.cus;
   p.xcds = shape.xcds;
   p.q = q;
@@ -1446,14 +1455,21 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
   p.ws_T = ws;
   p.ws_c = p.ws_T + recs * BC * BC;
   p.ws_beta = p.ws_c + recs * BC;
-  p.ws_dU0 = p.ws_beta + recs * BC;
-  p.ws_M = p.ws_dU0;
-  p.ws_J = p.ws_dU0 + recs * BC * V;
-  p.ws_S = p.ws_J + recs * K * V;
+  p.ws_S = p.ws_beta + recs * BC;
   p.ws_dS = p.ws_S + recs * K * V;
-  p.ws_dq = p.ws_dS + recs * K * V;
-  p.ws_dk = Hk != Hv ? p.ws_dq + static_cast<long>(B) * T * Hv * K : nullptr;
-  if (Hk == Hv) p.ws_dq = nullptr;
+  float *rest = p.ws_dS + recs * K * V;
+  if (bf16) {
+    p.ws_M = rest;
+    rest += recs * BC * BC;
+  } else {
+    p.ws_dU0 = rest;
+    p.ws_J = p.ws_dU0 + recs * BC * V;
+    rest = p.ws_J + recs * K * V;
+  }
+  if (per_head) {
+    p.ws_dq = rest;
+    p.ws_dk = p.ws_dq + static_cast<long>(B) * T * Hv * K;
+  }
   p.cu_seqlens = cu_seqlens;
   p.num_seqs = num_seqs;
   p.records = static_cast<int>(records);
@@ -1469,17 +1485,29 @@ int backward(const void *q, const void *k, const void *v, int in_dtype, const fl
   p.scale = scale;
   p.narrow = ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) & 7) != 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (K == 64) return V == 64 ? run_backward<64, 64>(p, st) : run_backward<64, 128>(p, st);
-  return V == 64 ? run_backward<128, 64>(p, st) : run_backward<128, 128>(p, st);
+  if (K == 64) return V == 64 ? run_backward<64, 64>(p, heads, st) : run_backward<64, 128>(p, heads, st);
+  return V == 64 ? run_backward<128, 64>(p, heads, st) : run_backward<128, 128>(p, heads, st);
 }
 }  // namespace
 }  // namespace pbgdn
 
-extern "C" size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K, int V) {
+extern "C" size_t pbgdn_chunk_bwd_workspace_size_dtype(int in_dtype, int B, int T, int num_seqs, int Hk, int Hv, int K,
+                                                       int V) {
   using namespace pbgdn;
-  if (B < 0 || T < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0) return 0;
-  return workspace_bytes_of(static_cast<long>(B) * ((static_cast<long>(T) + BC - 1) / BC), static_cast<long>(B) * T, Hk,
-                            Hv, K, V);
+  if (in_dtype < PBGDN_F32 || in_dtype > PBGDN_F16 || B < 0 || T < 0 || num_seqs < -1 || (num_seqs >= 0 && B != 1) ||
+      Hk <= 0 || Hv <= 0 || Hv % Hk != 0 || K <= 0 || V <= 0) {
+    return 0;
+  }
+  DeviceShape shape{};
+  device_shape(shape);
+  const long n = (static_cast<long>(T) + BC - 1) / BC;
+  const long records = num_seqs < 0 ? B * n : n == 0 ? 0 : packed_records(T, num_seqs);
+  return workspace_bytes_of(in_dtype, records, static_cast<long>(B) * T, Hk, Hv, K, V, shape.cus);
+}
+
+// For every dtype: float32's, the largest.
+extern "C" size_t pbgdn_chunk_bwd_workspace_size(int B, int T, int Hk, int Hv, int K, int V) {
+  return pbgdn_chunk_bwd_workspace_size_dtype(PBGDN_F32, B, T, -1, Hk, Hv, K, V);
 }
 
 extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int in_dtype, const float *g,
@@ -1492,9 +1520,7 @@ extern "C" int pbgdn_chunk_bwd(const void *q, const void *k, const void *v, int 
 }
 
 extern "C" size_t pbgdn_chunk_bwd_packed_workspace_size(int T, int num_seqs, int Hk, int Hv, int K, int V) {
-  using namespace pbgdn;
-  if (T < 0 || num_seqs < 0 || Hk <= 0 || Hv <= 0 || K <= 0 || V <= 0) return 0;
-  return workspace_bytes_of(T == 0 ? 0 : packed_records(T, num_seqs), T, Hk, Hv, K, V);
+  return num_seqs < 0 ? 0 : pbgdn_chunk_bwd_workspace_size_dtype(PBGDN_F32, 1, T, num_seqs, Hk, Hv, K, V);
 }
 
 extern "C" int pbgdn_chunk_bwd_packed(const void *q, const void *k, const void *v, int in_dtype, const float *g,

@@ -415,14 +415,13 @@ def _chunk_bwd(q, k, v, g, beta, scale: float, h0, cu_seqlens, do, dht):
     grads = (_lib.ptr(do), codes[do.dtype], _lib.ptr(dht), _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_), _lib.ptr(dg),
              _lib.ptr(dbeta), _lib.ptr(dh0))
     sizes = (length, hk, hv, dk, dv, float(scale), _lib.stream_handle(dev))
+    ws_bytes = lib.pbgdn_chunk_bwd_workspace_size_dtype(codes[q.dtype], batch, length,
+                                                        -1 if cu_seqlens is None else nseq, hk, hv, dk, dv)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     if cu_seqlens is None:
-        ws_bytes = lib.pbgdn_chunk_bwd_workspace_size(batch, length, hk, hv, dk, dv)
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         status = lib.pbgdn_chunk_bwd(*tensors, *grads, _lib.ptr(workspace), ws_bytes, batch, *sizes)
         _lib.check(status, "pbgdn_chunk_bwd")
     else:
-        ws_bytes = lib.pbgdn_chunk_bwd_packed_workspace_size(length, nseq, hk, hv, dk, dv)
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         status = lib.pbgdn_chunk_bwd_packed(*tensors, _lib.ptr(cu_seqlens), nseq, *grads, _lib.ptr(workspace), ws_bytes,
                                             *sizes)
         _lib.check(status, "pbgdn_chunk_bwd_packed")
@@ -507,8 +506,9 @@ def _(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
             q.new_empty(cu_seqlens.shape[0] - 1, v.shape[2], q.shape[3], v.shape[3], dtype=torch.float32))
 
 
-# Workspace up to which a packed backward runs as one call (about 118,000
-# tokens of 32 heads of 128 x 128; all sequences' records live at once there).
+# Workspace up to which a packed backward runs as one call: all sequences'
+# records live at once there (16 -> 32 heads of 128 x 128: 209,000 tokens of
+# bfloat16, 110,000 of the other dtypes).
 PACKED_BWD_WORKSPACE = 16 << 30
 
 
@@ -518,8 +518,8 @@ def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale
     sequences that stay within it (a longer sequence alone), so that the
     memory a call needs does not grow with the number of sequences."""
     total, nseq = q.shape[1], cu_seqlens.shape[0] - 1
-    size = lambda tokens, n: _lib.lib().pbgdn_chunk_bwd_packed_workspace_size(  # noqa: E731
-        tokens, n, q.shape[2], v.shape[2], q.shape[3], v.shape[3])
+    size = lambda tokens, n: _lib.lib().pbgdn_chunk_bwd_workspace_size_dtype(  # noqa: E731
+        _lib.DTYPE_CODES[q.dtype], 1, tokens, n, q.shape[2], v.shape[2], q.shape[3], v.shape[3])
     if nseq <= 1 or size(total, nseq) <= PACKED_BWD_WORKSPACE:
         return gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale)
     bounds = [min(max(int(x), 0), total) for x in cu_seqlens.tolist()]

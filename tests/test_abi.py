@@ -387,3 +387,23 @@ def test_chunk_layer_fuses_rejects_and_declines_without_a_device_call():
     assert q(_lib.F32, _lib.F32, _lib.F32, 4096, 8, 32, 128, 128) == 0    # float32 inputs: two passes
     assert q(_lib.BF16, _lib.F16, _lib.F32, 4096, 8, 32, 128, 128) == 0   # gate in another dtype
     assert q(_lib.BF16, _lib.BF16, _lib.F32, 4096, 8, 32, 64, 128) == 0   # K = 64
+
+
+def test_backward_workspace_by_dtype():
+    """bfloat16 records hold T, c, beta, S, dS' and M^T; the other dtypes' dU0 and
+    J in M^T's place. The dtype-less functions give the largest."""
+    lib = _lib.lib()
+    size = lib.pbgdn_chunk_bwd_workspace_size_dtype
+    for K, V in ((64, 64), (64, 128), (128, 64), (128, 128)):
+        common = 64 * 64 + 2 * 64 + 2 * K * V
+        assert size(_lib.BF16, 2, 130, -1, 3, 3, K, V) == 4 * 2 * 3 * 3 * (common + 64 * 64) + 256
+        for dtype in (_lib.F32, _lib.F16):
+            full = 4 * 2 * 3 * 3 * (common + 64 * V + K * V) + 256
+            assert size(dtype, 2, 130, -1, 3, 3, K, V) == full == lib.pbgdn_chunk_bwd_workspace_size(2, 130, 3, 3, K, V)
+        # GQA: dq and dk per value head; packed: tokens / 64 + sequences + 1 records
+        assert size(_lib.F32, 1, 130, 4, 1, 2, K, V) == 4 * (7 * 2 * (common + 64 * V + K * V) + 2 * 130 * 2 * K) + 256
+        assert size(_lib.F32, 1, 130, 4, 1, 2, K, V) == lib.pbgdn_chunk_bwd_packed_workspace_size(130, 4, 1, 2, K, V)
+        assert size(_lib.BF16, 1, 130, 4, 1, 2, K, V) < size(_lib.F32, 1, 130, 4, 1, 2, K, V)
+    for bad in ((3, 1, 64, -1, 1, 1, 64, 64), (1, 1, 64, -2, 1, 1, 64, 64), (1, 2, 64, 1, 1, 1, 64, 64),
+                (1, 1, -1, -1, 1, 1, 64, 64), (1, 1, 64, -1, 2, 3, 64, 64)):
+        assert size(*bad) == 0

@@ -6,10 +6,46 @@ import torch
 
 from oracle import gdn
 from pseudobrain_amd import gated_deltanet as gd
-from pseudobrain_amd.workloads import generate, to_numpy
+from pseudobrain_amd.workloads import cu_seqlens_of, generate, to_numpy
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+
+
+def make(batch, length, hk, hv, dk, dv, seed, dtype=torch.bfloat16, nseq=None):
+    q, k, v, g, beta, h0 = generate(batch, length, hk, hv, dk, dv, dtype, 0.05, seed=seed, nstates=nseq)
+    gen = torch.Generator().manual_seed(seed + 1)
+    do = (torch.randn(batch, length, hv, dv, generator=gen) * 0.1).to(dtype)
+    dht = torch.randn(nseq or batch, hv, dk, dv, generator=gen) * 0.1
+    return q, k, v, g, beta, h0, do, dht
+
+
+@pytest.mark.parametrize("batch,length,nseq,hk,hv,dk,dv,dtype", [
+    (8, 200, None, 16, 32, 128, 128, torch.bfloat16),
+    (1, 130, None, 2, 4, 128, 64, torch.bfloat16),     # per value head in the workspace
+    (1, 300, 3, 2, 2, 64, 128, torch.bfloat16),
+    (1, 300, 3, 1, 2, 64, 64, torch.float16),
+    (2, 65, None, 1, 2, 128, 128, torch.float32),
+])
+def test_the_workspace_is_not_overrun(monkeypatch, batch, length, nseq, hk, hv, dk, dv, dtype):
+    """A call with the bytes its dtype needs writes nothing behind them."""
+    q, k, v, g, beta, h0, do, dht = (x.to(DEV) for x in make(batch, length, hk, hv, dk, dv, 5, dtype, nseq))
+    cu = None if nseq is None else cu_seqlens_of([100, 0, 200]).to(DEV)
+    guards, empty = [], torch.empty
+
+    def guarded(*size, **kw):
+        if kw.get("dtype") != torch.uint8:
+            return empty(*size, **kw)
+        x = empty(size[0] + 4096, **kw)
+        x[size[0]:] = 0xA5
+        guards.append(x[size[0]:])
+        return x[:size[0]]
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", guarded)
+        gd._chunk_bwd(q, k, v, g, beta, 0.1, h0, cu, do, dht)
+    torch.cuda.synchronize()
+    assert len(guards) == 1 and bool((guards[0] == 0xA5).all())
 
 
 def test_decay_sums_are_in_float32():
