@@ -110,8 +110,8 @@ def test_autograd_through_the_operator():
 @pytest.mark.parametrize("dtype,dk,dv", [(torch.bfloat16, 128, 128), (torch.float32, 96, 64)])
 def test_autograd_through_packed_sequences(dtype, dk, dv):
     """A packed training call (cu_seqlens, one h0 per sequence, an empty
-    sequence among them) through gated_delta_rule(..., 'hip'): the backward
-    runs sequence by sequence and gives the oracle's gradients of each."""
+    sequence among them) through gated_delta_rule(..., 'hip') gives the oracle's
+    gradients of each sequence."""
     from pseudobrain_amd.workloads import cu_seqlens_of
     lengths = [70, 0, 130, 5, 64]
     n, total = len(lengths), sum(lengths)

@@ -5,8 +5,10 @@ import pytest
 import torch
 
 from oracle import gdn
+from pseudobrain_amd import _lib
 from pseudobrain_amd import gated_deltanet as gd
 from pseudobrain_amd.workloads import cu_seqlens_of, generate, to_numpy
+from tests.test_gpu_backward import check, oracle_grads
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -20,8 +22,88 @@ def make(batch, length, hk, hv, dk, dv, seed, dtype=torch.bfloat16, nseq=None):
     return q, k, v, g, beta, h0, do, dht
 
 
+def sums_in_registers(batch, length, nseq, hk, hv, dk, dv):
+    """The gradient kernel takes whole groups of value heads: the call's workspace
+    has no float32 dq and dk per value head."""
+    records = batch * -(-length // 64) if nseq is None else length // 64 + nseq + 1
+    floats = records * hv * (2 * 64 * 64 + 2 * 64 + 2 * dk * dv)
+    return _lib.lib().pbgdn_chunk_bwd_workspace_size_dtype(
+        _lib.BF16, batch, length, -1 if nseq is None else nseq, hk, hv, dk, dv) == 4 * floats + 256
+
+
+def one_element_off(x, **kw):
+    return torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("batch,length,hk,hv,dk,dv", [
+    (8, 200, 16, 32, 128, 128),  # two items a workgroup, the last chunk of 8 tokens
+    (8, 200, 8, 32, 128, 64),    # four value heads an item
+    (16, 193, 8, 32, 64, 128),   # a chunk of one token
+    (8, 200, 16, 32, 64, 64),
+])
+def test_value_heads_summed_in_registers(monkeypatch, batch, length, hk, hv, dk, dv, aligned):
+    """Key heads' gradients where one workgroup takes a key head's value heads in
+    turn and sums dq and dk over them: some key heads against the oracle, and
+    against a call of that key head alone, whose items are one value head each
+    (everything but that sum the same bits; dq and dk within their rounding)."""
+    with monkeypatch.context() as m:
+        if not aligned:
+            m.setattr(torch, "empty_like", one_element_off)
+        check_value_heads_summed_in_registers(batch, length, hk, hv, dk, dv)
+
+
+def check_value_heads_summed_in_registers(batch, length, hk, hv, dk, dv):
+    assert sums_in_registers(batch, length, None, hk, hv, dk, dv)
+    args = make(batch, length, hk, hv, dk, dv, seed=hk + dv)
+    q, k, v, g, beta, h0, do, dht = (x.to(DEV) for x in args)
+    scale, group = dk ** -0.5, hv // hk
+    got = gd.chunk_bwd(q, k, v, g, beta, scale, h0, do, dht)
+    torch.cuda.synchronize()
+    for n, kh in ((0, 0), (batch // 2, hk // 2), (batch - 1, hk - 1)):
+        print(f"[row {n}, key head {kh}]", flush=True)
+        one, keys, heads = slice(n, n + 1), slice(kh, kh + 1), slice(kh * group, (kh + 1) * group)
+        part = lambda x, hd: x[one, :, hd].contiguous()  # noqa: E731
+        sub = [part(q, keys), part(k, keys), part(v, heads), part(g, heads), part(beta, heads)]
+        mine = [part(x, hd) for x, hd in zip(got, (keys, keys, heads, heads, heads))] + [got[5][one, heads]]
+        alone = gd.chunk_bwd(*sub, scale, h0[one, heads], part(do, heads), dht[one, heads])
+        assert not sums_in_registers(1, length, None, 1, group, dk, dv)
+        for name, a, b in zip(("dv", "dg", "dbeta", "dh0"), mine[2:], alone[2:]):
+            assert torch.equal(a, b), f"{name} of row {n}, key head {kh}"
+        for name, a, b in zip(("dq", "dk"), mine, alone):  # two bf16 roundings of sums that differ in their last bits
+            diff = (a.double() - b.double()).abs()
+            assert (diff <= 2 ** -7 * b.double().abs() + 1e-6).all(), f"{name} of row {n}, key head {kh}"
+        ref = oracle_grads(*(x.cpu() for x in sub), scale, h0[one, heads].cpu(), part(do, heads).cpu(),
+                           dht[one, heads].cpu())
+        check(f"row {n} key head {kh}", mine, ref, dict(dq=q.dtype, dk=q.dtype, dv=q.dtype, dg=torch.float32,
+                                                        dbeta=torch.float32, dh0=torch.float32))
+
+
+def test_value_heads_summed_in_registers_packed():
+    """The same of packed sequences: each against a batched call of it alone."""
+    lengths = [200, 64, 0, 1, 321, 450, 65, 499]
+    nseq, total, hk, hv, dk, dv = len(lengths), sum(lengths), 16, 32, 128, 128
+    assert sums_in_registers(1, total, nseq, hk, hv, dk, dv)
+    q, k, v, g, beta, h0, do, dht = (x.to(DEV) for x in make(1, total, hk, hv, dk, dv, seed=3, nseq=nseq))
+    cu = cu_seqlens_of(lengths).to(DEV)
+    got = torch.ops.pbgdn.gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu, do, dht, 0.1)
+    torch.cuda.synchronize()
+    for n, (lo, hi) in enumerate(zip(cu.tolist(), cu.tolist()[1:])):
+        if lo == hi:
+            assert torch.equal(got[5][n], dht[n])
+            continue
+        sl = slice(lo, hi)
+        alone = gd.chunk_bwd(*(x[:, sl] for x in (q, k, v, g, beta)), 0.1, h0[n:n + 1], do[:, sl], dht[n:n + 1])
+        for name, a, b in zip(("dv", "dg", "dbeta"), got[2:], alone[2:]):
+            assert torch.equal(a[:, sl], b), f"{name} of sequence {n}"
+        assert torch.equal(got[5][n], alone[5][0]), f"dh0 of sequence {n}"
+        for name, a, b in zip(("dq", "dk"), got, alone):
+            diff = (a[:, sl].double() - b.double()).abs()
+            assert (diff <= 2 ** -7 * b.double().abs() + 1e-6).all(), f"{name} of sequence {n}"
+
+
 @pytest.mark.parametrize("batch,length,nseq,hk,hv,dk,dv,dtype", [
-    (8, 200, None, 16, 32, 128, 128, torch.bfloat16),
+    (8, 200, None, 16, 32, 128, 128, torch.bfloat16),  # dq and dk summed in registers
     (1, 130, None, 2, 4, 128, 64, torch.bfloat16),     # per value head in the workspace
     (1, 300, 3, 2, 2, 64, 128, torch.bfloat16),
     (1, 300, 3, 1, 2, 64, 64, torch.float16),

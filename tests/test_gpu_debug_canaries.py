@@ -20,7 +20,7 @@ import torch
 from pseudobrain_amd import _lib
 from pseudobrain_amd import gated_deltanet as gd
 from pseudobrain_amd.workloads import generate
-from tests import (test_gpu_backward, test_gpu_chunk, test_gpu_chunk_k256, test_gpu_chunk_layer, test_gpu_decode_layer,
+from tests import (test_gpu_backward, test_gpu_backward_bf16, test_gpu_backward_packed, test_gpu_chunk, test_gpu_chunk_k256, test_gpu_chunk_layer, test_gpu_decode_layer,
                    test_gpu_fla_schema, test_gpu_layer, test_gpu_prologue_varlen, test_gpu_recurrent,
                    test_gpu_state_pools, test_gpu_wide)
 
@@ -66,6 +66,17 @@ CASES = {
         1, 333, 1, 4, 128, 64, torch.bfloat16),
     "backward, float32, 16 chunks": lambda: test_gpu_backward.test_backward_matches_the_oracle(
         1, 1000, 2, 2, 128, 128, torch.float32),
+    "backward, bf16, key heads' sums in registers, 64-column scans": lambda: (
+        test_gpu_backward_bf16.check_value_heads_summed_in_registers(8, 200, 16, 32, 128, 128)),
+    "backward, bf16, several items a workgroup, Hk = Hv": lambda: test_gpu_backward_packed.test_many_heads_equal_few(
+        128, 64),
+    "backward, bf16, packed": test_gpu_backward_bf16.test_value_heads_summed_in_registers_packed,
+    "backward, bf16, packed, rows of no sequence": lambda: (
+        test_gpu_backward_packed.test_packed_equals_each_sequence_alone(
+            [3, 70, 198], 211, 2, 2, 64, 128, torch.bfloat16)),
+    "backward, float32, packed, rows of no sequence": lambda: (
+        test_gpu_backward_packed.test_packed_equals_each_sequence_alone(
+            [5, 40, 170], 171, 1, 2, 128, 128, torch.float32)),
     # fla's residuals (gc, A) of the reference's op
     "chunk residuals, GQA 2 -> 4": lambda: test_gpu_fla_schema.test_residuals_match_the_oracle(
         1, 130, 2, 4, 64, torch.bfloat16),
