@@ -39,6 +39,8 @@ requires grad they raise instead of returning tensors cut from the graph.
 """
 from __future__ import annotations
 
+import itertools
+
 import torch
 
 from . import _lib
@@ -377,9 +379,10 @@ def chunk_bwd(q, k, v, g, beta, scale: float, h0, do, dht=None):
     return _chunk_bwd(q, k, v, g, beta, scale, h0, None, do, dht)
 
 
-def _chunk_bwd(q, k, v, g, beta, scale: float, h0, cu_seqlens, do, dht):
+def _chunk_bwd(q, k, v, g, beta, scale: float, h0, cu_seqlens, do, dht, out=None):
     """chunk_bwd, or with cu_seqlens [N+1] the same for N packed sequences
-    (pbgdn_chunk_bwd_packed; h0, dht and dh0 [N,Hv,K,V])."""
+    (pbgdn_chunk_bwd_packed; h0, dht and dh0 [N,Hv,K,V]); out: contiguous
+    tensors for the six results."""
     batch, length, hk, hv, dk, dv = _shapes(q, k, v, g, beta)
     dev = _require_device(q, k, v, g, beta, h0, cu_seqlens, do, dht)
     if dk not in BACKWARD_HEAD_DIMS or dv not in BACKWARD_HEAD_DIMS:
@@ -403,11 +406,10 @@ def _chunk_bwd(q, k, v, g, beta, scale: float, h0, cu_seqlens, do, dht):
         if dht.shape != state_shape:
             raise ValueError(f"grad of the final state must be [N,Hv,K,V] = {state_shape}")
         dht = _aligned(dht.to(torch.float32).contiguous(), 16)
-    dq, dk_ = torch.empty_like(q), torch.empty_like(k)
-    dv_ = torch.empty_like(v)
-    dg = torch.empty(batch, length, hv, dtype=torch.float32, device=dev)
-    dbeta = torch.empty_like(beta)
-    dh0 = torch.empty(state_shape, dtype=torch.float32, device=dev)
+    dq, dk_, dv_, dg, dbeta, dh0 = out or (
+        torch.empty_like(q), torch.empty_like(k), torch.empty_like(v),
+        torch.empty(batch, length, hv, dtype=torch.float32, device=dev), torch.empty_like(beta),
+        torch.empty(state_shape, dtype=torch.float32, device=dev))
     lib = _lib.lib()
     codes = _lib.DTYPE_CODES
     tensors = (_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), codes[q.dtype], _lib.ptr(g), _lib.ptr(beta), codes[beta.dtype],
@@ -493,9 +495,9 @@ def _(q, k, v, g, beta, h0, grad_o, grad_final, scale):
                                 "-> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)")
 def gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
     """gated_delta_chunk_backward of packed sequences (cu_seqlens [N+1]; h0,
-    grad_final and dh0 [N,Hv,K,V]): one call for all of them, and cu_seqlens
-    is read on the device only."""
-    return _chunk_bwd(q, k, v, g, beta, scale, h0, cu_seqlens, grad_o, grad_final)
+    grad_final and dh0 [N,Hv,K,V]): one call for all of them, with cu_seqlens
+    read on the device only, up to PACKED_BWD_WORKSPACE."""
+    return _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale)
 
 
 @gated_delta_chunk_packed_backward.register_fake
@@ -512,30 +514,45 @@ def _(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
 PACKED_BWD_WORKSPACE = 16 << 30
 
 
+def _packed_groups(bounds, size, limit):
+    """[(a, b)]: consecutive groups of the packed sequences with these bounds whose
+    workspace size(rows, sequences) stays within the limit; a longer sequence alone."""
+    groups, first, nseq = [], 0, len(bounds) - 1
+    for n in range(1, nseq + 1):
+        if n == nseq or size(bounds[n + 1] - bounds[first], n + 1 - first) > limit:
+            groups.append((first, n))
+            first = n
+    return groups
+
+
 def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale):
     """The backward of a packed call: one launch set for all sequences; where
     their workspace would pass PACKED_BWD_WORKSPACE, groups of consecutive
     sequences that stay within it (a longer sequence alone), so that the
-    memory a call needs does not grow with the number of sequences."""
-    total, nseq = q.shape[1], cu_seqlens.shape[0] - 1
+    memory a call needs does not grow with the number of sequences. Rows of no
+    sequence belong to no group."""
+    total, hk, dk = q.shape[1:]
+    hv, dv = v.shape[2:]
+    nseq = cu_seqlens.shape[0] - 1
     size = lambda tokens, n: _lib.lib().pbgdn_chunk_bwd_workspace_size_dtype(  # noqa: E731
-        _lib.DTYPE_CODES[q.dtype], 1, tokens, n, q.shape[2], v.shape[2], q.shape[3], v.shape[3])
-    if nseq <= 1 or size(total, nseq) <= PACKED_BWD_WORKSPACE:
-        return gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale)
-    bounds = [min(max(int(x), 0), total) for x in cu_seqlens.tolist()]
-    groups, first = [], 0
-    for n in range(1, nseq + 1):
-        if n == nseq or size(max(bounds[n + 1] - bounds[first], 0), n + 1 - first) > PACKED_BWD_WORKSPACE:
-            groups.append((first, n))
-            first = n
-    parts = []
-    for a, b in groups:
-        lo, hi = (0 if a == 0 else bounds[a]), (total if b == nseq else max(bounds[a], bounds[b]))
-        sl = slice(lo, hi)
-        parts.append(gated_delta_chunk_packed_backward(
-            q[:, sl], k[:, sl], v[:, sl], g[:, sl], beta[:, sl], None if h0 is None else h0[a:b],
-            cu_seqlens[a:b + 1] - lo, grad_o[:, sl], None if grad_final is None else grad_final[a:b], scale))
-    return tuple(torch.cat([p[j] for p in parts], 1 if j < 5 else 0) for j in range(6))
+        _lib.DTYPE_CODES.get(q.dtype, _lib.F32), 1, tokens, n, hk, hv, dk, dv)
+    if size(total, nseq) <= PACKED_BWD_WORKSPACE:
+        return _chunk_bwd(q, k, v, g, beta, scale, h0, cu_seqlens, grad_o, grad_final)
+    bounds = list(itertools.accumulate((min(max(int(x), 0), total) for x in cu_seqlens.tolist()), max))
+    lo, hi = bounds[0], bounds[-1]
+    beta_dtype = beta.dtype if beta.dtype in (torch.float32, q.dtype) else torch.float32
+    out = [torch.empty(shape, dtype=dtype, device=q.device) for shape, dtype in (
+        (q.shape, q.dtype), (k.shape, q.dtype), (v.shape, q.dtype), (g.shape, torch.float32), (beta.shape, beta_dtype),
+        ((nseq, hv, dk, dv), torch.float32))]
+    for x in out[:5]:
+        x[:, :lo].zero_()
+        x[:, hi:].zero_()
+    for a, b in _packed_groups(bounds, size, PACKED_BWD_WORKSPACE):
+        rows = slice(bounds[a], bounds[b])
+        _chunk_bwd(q[:, rows], k[:, rows], v[:, rows], g[:, rows], beta[:, rows], scale, None if h0 is None else h0[a:b],
+                   cu_seqlens[a:b + 1] - bounds[a], grad_o[:, rows], None if grad_final is None else grad_final[a:b],
+                   out=[x[:, rows] for x in out[:5]] + [out[5][a:b]])
+    return tuple(out)
 
 
 def _chunk_setup(ctx, inputs, output):
@@ -552,8 +569,8 @@ def _chunk_grad(ctx, grad_o, grad_final):
     if grad_o is None:
         grad_o = torch.zeros(*q.shape[:2], v.shape[2], v.shape[3], dtype=q.dtype, device=q.device)
     if cu_seqlens is not None:
-        dq, dk, dv, dg, dbeta, dh0 = _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final,
-                                                      ctx.scale)
+        dq, dk, dv, dg, dbeta, dh0 = gated_delta_chunk_packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o,
+                                                                       grad_final, ctx.scale)
     else:
         dq, dk, dv, dg, dbeta, dh0 = gated_delta_chunk_backward(q, k, v, g, beta, h0, grad_o, grad_final,
                                                                 ctx.scale)

@@ -169,3 +169,14 @@ def test_layer_row_stride_accepts_token_slices_of_one_batch_row():
     assert _rows(z[:, 10:60, 16:48], "z") == 64  # a column slice as well
     with pytest.raises(ValueError, match="dense rows"):
         _rows(torch.empty(2, 100, 64)[:, 10:60], "z")
+
+
+def test_packed_backward_groups():
+    """Consecutive sequences, as many a group as the limit takes; one longer than
+    it alone; empty ones count as sequences."""
+    size = lambda rows, n: rows + 10 * n  # noqa: E731
+    assert gd._packed_groups([5, 95, 185, 275], size, 200) == [(0, 2), (2, 3)]
+    assert gd._packed_groups([0, 500, 510, 520, 900], size, 100) == [(0, 1), (1, 3), (3, 4)]
+    assert gd._packed_groups([7] * 8, size, 30) == [(0, 3), (3, 6), (6, 7)]
+    assert gd._packed_groups([3, 4], size, 0) == [(0, 1)]
+    assert gd._packed_groups([3], size, 0) == []

@@ -76,6 +76,31 @@ def test_groups_of_sequences_equal_one_call(monkeypatch):
         assert a.shape == b.shape and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("bounds", [[1000, 1090, 1090, 1300, 1301, 1420], [0, 200], [3900, 4000], [77], [0, 40, 90]])
+def test_groups_hold_no_rows_of_no_sequence(monkeypatch, bounds):
+    """Each group's workspace stays within the limit however long the buffer is
+    around the sequences, and the result is one call's."""
+    limit = 1 << 20  # (about 280 rows of these heads)
+    args = make(bounds, 4000, 1, 2, 64, 64, torch.bfloat16, seed=5)
+    q, k, v, g, beta, h0, do, dht, cu = args
+    want = packed(*args)
+    sizes, empty = [], torch.empty
+
+    def recorded(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            sizes.append(size[0])
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(gd, "PACKED_BWD_WORKSPACE", limit)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", recorded)
+        got = gd._packed_backward(q, k, v, g, beta, h0, cu, do, dht, 0.1)
+    torch.cuda.synchronize()
+    assert all(size <= limit for size in sizes) and (len(bounds) == 1 or sizes)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dk,dv", [(128, 128), (64, 64), (128, 64)])
 def test_many_heads_equal_few(dk, dv):
     """Scans of 64 value columns a workgroup (enough sequences and heads for
