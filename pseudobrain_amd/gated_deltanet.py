@@ -530,14 +530,19 @@ def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale
     their workspace would pass PACKED_BWD_WORKSPACE, groups of consecutive
     sequences that stay within it (a longer sequence alone), so that the
     memory a call needs does not grow with the number of sequences. Rows of no
-    sequence belong to no group."""
+    sequence belong to no group. Where even the one call's memory is not to be
+    had, each sequence alone: the call needs no more than its longest one."""
     total, hk, dk = q.shape[1:]
     hv, dv = v.shape[2:]
     nseq = cu_seqlens.shape[0] - 1
     size = lambda tokens, n: _lib.lib().pbgdn_chunk_bwd_workspace_size_dtype(  # noqa: E731
         _lib.DTYPE_CODES.get(q.dtype, _lib.F32), 1, tokens, n, hk, hv, dk, dv)
-    if size(total, nseq) <= PACKED_BWD_WORKSPACE:
-        return _chunk_bwd(q, k, v, g, beta, scale, h0, cu_seqlens, grad_o, grad_final)
+    limit = PACKED_BWD_WORKSPACE
+    if size(total, nseq) <= limit:
+        try:
+            return _chunk_bwd(q, k, v, g, beta, scale, h0, cu_seqlens, grad_o, grad_final)
+        except torch.OutOfMemoryError:
+            limit = 0
     bounds = list(itertools.accumulate((min(max(int(x), 0), total) for x in cu_seqlens.tolist()), max))
     lo, hi = bounds[0], bounds[-1]
     beta_dtype = beta.dtype if beta.dtype in (torch.float32, q.dtype) else torch.float32
@@ -547,7 +552,7 @@ def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale
     for x in out[:5]:
         x[:, :lo].zero_()
         x[:, hi:].zero_()
-    for a, b in _packed_groups(bounds, size, PACKED_BWD_WORKSPACE):
+    for a, b in _packed_groups(bounds, size, limit):
         rows = slice(bounds[a], bounds[b])
         _chunk_bwd(q[:, rows], k[:, rows], v[:, rows], g[:, rows], beta[:, rows], scale, None if h0 is None else h0[a:b],
                    cu_seqlens[a:b + 1] - bounds[a], grad_o[:, rows], None if grad_final is None else grad_final[a:b],

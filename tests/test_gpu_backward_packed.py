@@ -101,6 +101,30 @@ def test_groups_hold_no_rows_of_no_sequence(monkeypatch, bounds):
         assert a.shape == b.shape and torch.equal(a, b)
 
 
+def test_out_of_memory_leaves_each_sequence_alone(monkeypatch):
+    """A call whose workspace for all sequences cannot be had still runs if the
+    longest sequence's can."""
+    bounds = [0, 90, 90, 300, 301, 420]
+    args = make(bounds, 450, 1, 2, 64, 64, torch.bfloat16, seed=9)
+    q, k, v, g, beta, h0, do, dht, cu = args
+    want = packed(*args)
+    refused, empty = [], torch.empty
+
+    def small_only(*size, **kw):
+        if kw.get("dtype") == torch.uint8 and size[0] > 1 << 20:
+            refused.append(size[0])
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", small_only)
+        got = packed(*args)
+    torch.cuda.synchronize()
+    assert len(refused) == 1
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dk,dv", [(128, 128), (64, 64), (128, 64)])
 def test_many_heads_equal_few(dk, dv):
     """Scans of 64 value columns a workgroup (enough sequences and heads for
