@@ -35,3 +35,21 @@ def test_float32_o_rounds_to_the_16_bit_o(dtype, batch, lengths, hk, hv, dk, dv)
     assert o32.dtype == torch.float32 and o16.dtype == dtype
     assert torch.equal(o32.to(dtype), o16) and torch.equal(s32, s16)
     assert torch.equal(entry, o32) and torch.equal(final, s32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dk,dv,grad", [(128, 100, False), (64, 33, False), (256, 40, False), (96, 120, False),
+                                        (128, 100, True), (64, 33, True)])
+def test_padded_value_widths_cut_a_16_bit_o(dtype, dk, dv, grad):
+    """V no width of the kernels: o is the 16-bit o's columns, widened, contiguous."""
+    q, k, v, g, beta, h0 = (x.to(DEV) for x in generate(2, 130, 2, 4, dk, dv, dtype, 0.05, seed=dv))
+    with torch.set_grad_enabled(grad):
+        if grad:
+            q.requires_grad_()
+        o, final = gd.gated_delta_rule(q, k, v, g, beta, 0.1, h0, "hip")
+        kp, vp = gd._chunk_widths(dk, dv, grad)
+    with torch.no_grad():
+        o16, s16 = gd.chunk_fwd(gd._pad_last(q, kp), gd._pad_last(k, kp), gd._pad_last(v, vp), g, beta, 0.1,
+                                gd._pad_state(h0, kp, vp))
+    assert vp > dv and o.dtype == torch.float32 and o.is_contiguous() and o.requires_grad == grad
+    assert torch.equal(o, o16[..., :dv].float()) and torch.equal(final, s16[..., :dk, :dv])
