@@ -118,11 +118,6 @@ __device__ __forceinline__ float4_t ld4s(const float *p, int stride) {
 
 __device__ __forceinline__ float4_t zero4() { return float4_t{0.f, 0.f, 0.f, 0.f}; }
 
-template <typename T>
-constexpr int dtype_of_bwd() {
-  return sizeof(T) == 4 ? PBGDN_F32 : (std::is_same<T, u16>::value ? PBGDN_BF16 : PBGDN_F16);
-}
-
 // Sum over the 16 lanes that share lane >> 4 (the columns of one tile row).
 __device__ __forceinline__ float row16_sum(float x) {
 #pragma unroll
@@ -130,19 +125,14 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
-// Eight (four for float32) consecutive elements of TIn in a 16-byte piece, as float.
+// Eight half_t or four float elements in a 16-byte piece, as float. (TIn here and
+// in the next three is one of these two.)
 template <typename TIn>
 __device__ __forceinline__ void decode16(const uint4 &u, float *x) {
   const uint32_t w[4] = {u.x, u.y, u.z, u.w};
   if constexpr (sizeof(TIn) == 4) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = __uint_as_float(w[e]);
-  } else if constexpr (dtype_of_bwd<TIn>() == PBGDN_BF16) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x[2 * e] = __uint_as_float(w[e] << 16);
-      x[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
-    }
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -155,13 +145,7 @@ __device__ __forceinline__ void decode16(const uint4 &u, float *x) {
 // Element idx of an LDS array of TIn, as float.
 template <typename TIn>
 __device__ __forceinline__ float ld_el(const TIn *m, int idx) {
-  if constexpr (sizeof(TIn) == 4) {
-    return m[idx];
-  } else if constexpr (dtype_of_bwd<TIn>() == PBGDN_BF16) {
-    return __uint_as_float(static_cast<uint32_t>(m[idx]) << 16);
-  } else {
-    return static_cast<float>(m[idx]);
-  }
+  return static_cast<float>(m[idx]);
 }
 
 // Four consecutive elements of TIn (idx a multiple of 4; one 8- or 16-byte
@@ -172,15 +156,10 @@ __device__ __forceinline__ float4_t ld4e(const TIn *m, int idx) {
     return ld4(reinterpret_cast<const float *>(m) + idx);
   } else {
     const uint2 w = *reinterpret_cast<const uint2 *>(m + idx);
-    if constexpr (dtype_of_bwd<TIn>() == PBGDN_BF16) {
-      return float4_t{__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
-                      __uint_as_float(w.y & 0xffff0000u)};
-    } else {
-      return float4_t{static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.x & 0xffffu))),
-                      static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.x >> 16))),
-                      static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.y & 0xffffu))),
-                      static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.y >> 16)))};
-    }
+    return float4_t{static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.x & 0xffffu))),
+                    static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.x >> 16))),
+                    static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.y & 0xffffu))),
+                    static_cast<float>(__builtin_bit_cast(half_t, static_cast<u16>(w.y >> 16)))};
   }
 }
 
@@ -648,7 +627,7 @@ struct ScanStage {
 // ---------------------------------------------------------------------------
 // LDS of one scan workgroup: K rows, T, the state tile, the step's V or dU0
 // tile, the tile the next products read and the decay vectors, in float.
-template <int K, typename TIn>
+template <int K>
 struct ScanLds {
   static constexpr int LK = K + 4;
   static constexpr size_t K_BYTES = sizeof(float) * BC * LK;
@@ -661,16 +640,15 @@ struct ScanLds {
 };
 
 // K rows (row0 + r) times the state tile kept in LDS.
-template <int K, typename TIn>
+template <int K>
 __device__ __forceinline__ float4_t k_times_state(const void *sk, int row0, const void *sstate) {
-  using L = ScanLds<K, TIn>;
+  using L = ScanLds<K>;
   const float *kf = static_cast<const float *>(sk), *sf = static_cast<const float *>(sstate);
   return tile_mm4<K>(zero4(), [&](int r, int kk) { return ld4(&kf[(row0 + r) * L::LK + kk]); },
                      [&](int kk, int col) { return ld4s(&sf[kk * LT + col], LT); });
 }
 
 // Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the state tile, column c, into LDS.
-template <int K, typename TIn>
 __device__ __forceinline__ void put_state_rows(void *sstate, int kk0, int c, float4_t x) {
   float *sf = static_cast<float *>(sstate);
 #pragma unroll
@@ -678,15 +656,14 @@ __device__ __forceinline__ void put_state_rows(void *sstate, int kk0, int c, flo
 }
 
 // (diag(w) K)^T rows k0 + r, four tokens t .. t+3 of the K rows in LDS.
-template <int K, typename TIn>
+template <int K>
 __device__ __forceinline__ float4_t k_cols(const void *sk, int t, int col) {
-  using L = ScanLds<K, TIn>;
+  using L = ScanLds<K>;
   return ld4s(static_cast<const float *>(sk) + t * L::LK + col, L::LK);
 }
 
 // Key tile kt of the value columns v0 .. of a state record ([K][V]), from the
 // accumulator layout.
-template <int K, typename TIn>
 __device__ __forceinline__ void put_state_tile(float *ws, int V, int v0, int kt, float4_t x) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -696,7 +673,7 @@ __device__ __forceinline__ void put_state_tile(float *ws, int V, int v0, int kt,
 template <int K, typename TIn>
 __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
   const BwdSeq seq = seq_of(p, n);
-  using L = ScanLds<K, TIn>;
+  using L = ScanLds<K>;
   constexpr int PER = K / 64;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
   void *sk = base, *st = base + L::OFF_T, *ss = base + L::OFF_S;
@@ -720,14 +697,14 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
     float *ws = p.ws_S + rec(p, seq, h, i) * K * p.V;
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-      put_state_tile<K, TIn>(ws, p.V, v0, wave + 4 * m, s[m]);
-      put_state_rows<K, TIn>(ss, 16 * (wave + 4 * m) + 4 * g4, c, s[m]);
+      put_state_tile(ws, p.V, v0, wave + 4 * m, s[m]);
+      put_state_rows(ss, 16 * (wave + 4 * m) + 4 * g4, c, s[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sx);
     if (i + 1 < seq.n) stage.load(p, seq, h, hk, i + 1, v0);
     __syncthreads();
     // X = V - Gamma K S (rows 16w ..)
-    const float4_t ks = k_times_state<K, TIn>(sk, 16 * wave, ss);
+    const float4_t ks = k_times_state<K>(sk, 16 * wave, ss);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * wave + 4 * g4 + r;
@@ -748,7 +725,7 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
     for (int m = 0; m < PER; ++m) {
       const int k0 = 16 * (wave + 4 * m);
       float4_t y;
-      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&se[t]); },
+      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K>(sk, t, k0 + r) * ld4(&se[t]); },
                        [&](int t, int col) { return ld4s(&su[t * LT + col], LT); });
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[m][r] = gam_c * s[m][r] + y[r];
@@ -764,7 +741,7 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
 template <int K, typename TIn>
 __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int n, int h, int v0) {
   const BwdSeq seq = seq_of(p, n);
-  using L = ScanLds<K, TIn>;
+  using L = ScanLds<K>;
   constexpr int PER = K / 64;
   unsigned char *base = reinterpret_cast<unsigned char *>(lds);
   void *sk = base, *st = base + L::OFF_T, *sds = base + L::OFF_S;
@@ -788,8 +765,8 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     float *wds = p.ws_dS + rec(p, seq, h, i) * K * p.V;
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
-      put_state_tile<K, TIn>(wds, p.V, v0, wave + 4 * m, ds[m]);
-      put_state_rows<K, TIn>(sds, 16 * (wave + 4 * m) + 4 * g4, c, ds[m]);
+      put_state_tile(wds, p.V, v0, wave + 4 * m, ds[m]);
+      put_state_rows(sds, 16 * (wave + 4 * m) + 4 * g4, c, ds[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sdu);
     float jv[PER][4];
@@ -801,7 +778,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     if (i > 0) stage.load(p, seq, h, hk, i - 1, v0);
     __syncthreads();
     // dU = dU0 + E K dS'
-    const float4_t kd = k_times_state<K, TIn>(sk, 16 * wave, sds);
+    const float4_t kd = k_times_state<K>(sk, 16 * wave, sds);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * wave + 4 * g4 + r;
@@ -822,7 +799,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
     for (int m = 0; m < PER; ++m) {
       const int k0 = 16 * (wave + 4 * m);
       float4_t y;
-      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K, TIn>(sk, t, k0 + r) * ld4(&sgam[t]); },
+      y = tile_mm4<BC>(zero4(), [&](int r, int t) { return k_cols<K>(sk, t, k0 + r) * ld4(&sgam[t]); },
                        [&](int t, int col) { return ld4s(&sdx[t * LT + col], LT); });
 #pragma unroll
       for (int r = 0; r < 4; ++r) ds[m][r] = gam_c * ds[m][r] + jv[m][r] - y[r];
@@ -849,7 +826,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
 // one pair read the same K rows and T records every step, so when the pairs
 // fill the XCDs evenly all tiles of a pair are given indices on one XCD
 // (xcd_group) and those reads come from its L2 after the first.
-template <int K, typename TIn>
+template <int K>
 constexpr size_t scan_lds();
 template <int K, typename TIn>
 constexpr size_t grad_lds();
@@ -857,7 +834,7 @@ constexpr size_t grad_lds();
 template <int K, typename TIn>
 __global__ __launch_bounds__(BNT) void bwd_scans_kernel(BwdParams p) {
   extern __shared__ __align__(16) float lds[];
-  PBGDN_POISON_LDS(lds, (scan_lds<K, TIn>()));
+  PBGDN_POISON_LDS(lds, (scan_lds<K>()));
   PBGDN_POISON_SYNC();
   const int tiles = p.V / 16, pairs = 2 * p.num_seqs * p.Hv;
   const int l = blockIdx.x;
@@ -1261,8 +1238,8 @@ __global__ __launch_bounds__(BNT) void bwd_gqa_reduce_kernel(BwdParams p) {
 }
 
 // LDS bytes of each kernel.
-template <int K, typename TIn>
-constexpr size_t scan_lds() { return ScanLds<K, TIn>::BYTES; }
+template <int K>
+constexpr size_t scan_lds() { return ScanLds<K>::BYTES; }
 template <int K, typename TIn>
 constexpr size_t grad_lds() {
   return sizeof(TIn) * 2 * BC * (K + 16 / sizeof(TIn)) +
@@ -1341,9 +1318,9 @@ int run_backward(const BwdParams &p, int heads, hipStream_t st) {
   if (p.num_seqs == 0) return rc;  // no sequence: the local kernel has written the rows' zeros
   if (rc == PBGDN_OK) {  // both scans in one launch (with T = 0 only the reverse one writes: dh0 = dht)
     switch (p.in_dtype) {
-      case PBGDN_F32: rc = launch(bwd_scans_kernel<K, float>, per_tile2, scan_lds<K, float>(), st, p); break;
+      case PBGDN_F32: rc = launch(bwd_scans_kernel<K, float>, per_tile2, scan_lds<K>(), st, p); break;
       case PBGDN_BF16: rc = run_scans_bf16<K>(p, st); break;
-      default: rc = launch(bwd_scans_kernel<K, half_t>, per_tile2, scan_lds<K, half_t>(), st, p); break;
+      default: rc = launch(bwd_scans_kernel<K, half_t>, per_tile2, scan_lds<K>(), st, p); break;
     }
   }
   if (rc == PBGDN_OK && p.records > 0) {
