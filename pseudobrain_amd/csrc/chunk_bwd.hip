@@ -648,7 +648,9 @@ __device__ __forceinline__ float4_t k_times_state(const void *sk, int row0, cons
                      [&](int kk, int col) { return ld4s(&sf[kk * LT + col], LT); });
 }
 
-// Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the state tile, column c, into LDS.
+// Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the K-row state tile, column c, into
+// LDS. (Without the parameter the scans compile to another order of
+// instructions, 0.5% slower at 12,000 tokens in float32.)
 __device__ __forceinline__ void put_state_rows(void *sstate, int kk0, int c, float4_t x) {
   float *sf = static_cast<float *>(sstate);
 #pragma unroll
