@@ -651,6 +651,7 @@ __device__ __forceinline__ float4_t k_times_state(const void *sk, int row0, cons
 // Rows kk0 .. kk0+3 (4 g4 + 16 m ..) of the K-row state tile, column c, into
 // LDS. (Without the parameter the scans compile to another order of
 // instructions, 0.5% slower at 12,000 tokens in float32.)
+template <int K>
 __device__ __forceinline__ void put_state_rows(void *sstate, int kk0, int c, float4_t x) {
   float *sf = static_cast<float *>(sstate);
 #pragma unroll
@@ -700,7 +701,7 @@ __device__ __forceinline__ void state_pass(const BwdParams &p, float *lds, int n
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
       put_state_tile(ws, p.V, v0, wave + 4 * m, s[m]);
-      put_state_rows(ss, 16 * (wave + 4 * m) + 4 * g4, c, s[m]);
+      put_state_rows<K>(ss, 16 * (wave + 4 * m) + 4 * g4, c, s[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sx);
     if (i + 1 < seq.n) stage.load(p, seq, h, hk, i + 1, v0);
@@ -768,7 +769,7 @@ __device__ __forceinline__ void adjoint_pass(const BwdParams &p, float *lds, int
 #pragma unroll
     for (int m = 0; m < PER; ++m) {
       put_state_tile(wds, p.V, v0, wave + 4 * m, ds[m]);
-      put_state_rows(sds, 16 * (wave + 4 * m) + 4 * g4, c, ds[m]);
+      put_state_rows<K>(sds, 16 * (wave + 4 * m) + 4 * g4, c, ds[m]);
     }
     stage.store(sk, st, sc, sgam, se, sbeta, sdu);
     float jv[PER][4];
