@@ -135,7 +135,8 @@ def bench_backward(steps=3, warmup=1):
     achieved = flops / ksec / 1e12
     return {"workload": "prefill_qwen3next backward", "T": s.length, "ms_per_call": sec * 1e3,
             "kernel_ms": ksec * 1e3, "Mtok_s": s.length / sec / 1e6, "algorithmic_flops": flops,
-            "workspace_bytes": _lib.lib().pbgdn_chunk_bwd_workspace_size(1, s.length, s.hk, s.hv, s.dk, s.dv),
+            "workspace_bytes": _lib.lib().pbgdn_chunk_bwd_workspace_size_dtype(
+                _lib.BF16, 1, s.length, -1, s.hk, s.hv, s.dk, s.dv),
             "roofline": {"bound": "mfma", "achieved": achieved, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": achieved / MFMA_PEAK_TFLOPS, "peak_basis": "bf16 dense MFMA (bf16 inputs)",
                          "traffic": traffic, "algorithmic_bytes": nbytes,

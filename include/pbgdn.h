@@ -424,7 +424,9 @@ int pbgdn_prologue_varlen_fwd(const void *qkv, long qkv_stride,
  * state. It recomputes what it needs from the forward's inputs (no saved
  * intermediates): the state at every 64-token chunk start by a forward pass,
  * the state adjoint at every chunk end by a reverse pass, then each chunk's
- * gradients; all arithmetic float32.
+ * gradients. Sums and states are float32. float32 and fp16 inputs: every
+ * product in float32; bfloat16 inputs: on bf16 matrix products, a float32
+ * factor as a high/low pair of bf16 parts (about 2^-16 relative).
  *
  *   q, k, v, in_dtype, g, beta, beta_dtype, h0, B, T, Hk, Hv, K, V, scale:
  *               as pbgdn_chunk_fwd without cu_seqlens (h0 [B, Hv, K, V]

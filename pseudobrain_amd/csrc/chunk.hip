@@ -30,7 +30,12 @@ namespace {
 // tokens: 4 x 8,192 0.53 vs 0.72 ms, 8 x 4,096 0.39 vs 0.73 ms, 1024 x 32
 // 1.76 vs 2.68 ms); one or two sequences of that shape have 32 or 64 of them
 // and run faster on the narrow scan, which spreads each head over 8
-// workgroups (1 x 32,768: 0.78 vs 1.69 ms). PBGDN_SCAN=narrow|wide in the
+// workgroups (1 x 32,768: 0.78 vs 1.69 ms). A float32 o moves the line little
+// (whole calls, wide vs narrow: 4 x 2,048 160 vs 202 us, 16 x 2,048 430 vs 810,
+// 24 packed sequences of 19,001 tokens 296 vs 490) but for a few packed
+// sequences of uneven lengths, whose longest one is the call's length and has
+// the shorter step on the narrow scan (7 of 6,011 tokens 205 vs 160, 4 of 8,192
+// 220 vs 208): the lengths are on the device. PBGDN_SCAN=narrow|wide in the
 // environment forces a choice (for measurements).
 inline int scan_choice() {
   static const int choice = [] {

@@ -13,7 +13,7 @@
 //   dU = M^T dO + E K dS',  dX = Tb^T dU,
 //   dS = gamma_C dS' + scale (Gamma Q)^T dO - (Gamma K)^T dX,
 // and each chunk's gradients follow from its start state S, its end adjoint
-// dS' and its own inputs. Four launches on the caller's stream:
+// dS' and its own inputs. Three or four launches on the caller's stream:
 //
 //   bwd_local_kernel     per (chunk, value head): T = (I + A)^-1 by block
 //                        substitution, dU0 = M^T dO, J = scale (Gamma Q)^T dO
@@ -27,11 +27,12 @@
 // bf16 inputs have kernels of their own for the first three
 // (chunk_bwd_scan.hpp, chunk_bwd_bf16.hpp).
 //
-// Accumulation is float32. With bf16 inputs the products of inputs and states
-// run on bf16 MFMA, a float32 operand entering as a high/low pair of bf16
-// parts (A B_hi + A B_lo, or three products when both are paired: about
-// 2^-16 relative); the rest, and every product for fp16 / fp32 inputs, on the
-// 16x16x4 fp32 MFMA with four consecutive k per lane group.
+// Accumulation is float32. With bf16 inputs the products run on bf16 MFMA, a
+// float32 operand entering as a high/low pair of bf16 parts (A B_hi + A B_lo, or
+// three products when both are paired: about 2^-16 relative); sums of products
+// by element (the decay and beta gradients) take their operands in float32.
+// The 16x16 blocks of the inverse, and every product for fp16 / fp32 inputs, run
+// on the 16x16x4 fp32 MFMA with four consecutive k per lane group.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -246,8 +247,9 @@ __device__ __forceinline__ BwdSeq seq_of(const BwdParams &p, int s) {
 }
 
 // The sequence and chunk of block (x, z) of a per-chunk grid: chunk x of batch
-// row z, or packed the chunk of record x (false where it holds none): the last sequence whose first record is at most x, counted 64
-// sequences at a time across the wave (every wave gets the same answer).
+// row z, or packed the chunk of record x (false where it holds none): the last
+// sequence whose first record is at most x, counted 64 sequences at a time
+// across the wave (every wave gets the same answer).
 __device__ __forceinline__ bool chunk_of(const BwdParams &p, int x, int z, BwdSeq &q, int &i) {
   int s = z;
   if (p.cu_seqlens) {
@@ -1262,10 +1264,13 @@ int launch(Kern kernel, dim3 grid, size_t lds, hipStream_t st, const BwdParams &
 // Value heads of a key head that one workgroup of the bf16 gradient kernel
 // takes in turn: all of them (dq and dk are then summed in registers, with no
 // float32 copies per value head and no reduction pass), unless the call is so
-// small that one head per workgroup (one workgroup a CU) needs fewer rounds of
-// the CUs by more than a quarter: the reduction and the float32 copies cost a
-// sixth to a fifth (at 6,011 tokens of 32 heads 414 + 67 us against 409, at
-// 4 x 2,048 542 + 92 against 514).
+// small that this takes more than 5/4 of the rounds of the CUs (a head a round
+// each) that one head per workgroup takes. The whole backward, one head an item
+// against all, in us at K = V = 128: 16 -> 32 heads, rounds 4 : 4 (32 chunks)
+// 223 / 187, 8 : 7 398 / 356, 6 : 5 (33 chunks) 287 / 267, 4 : 3 (17 and 24
+// chunks) 166 / 170 and 176 / 170, 2 : 1 86 / 91; 8 -> 32, 12 : 10 529 / 488,
+// 12 : 9 488 / 474; 4 -> 32, 16 : 13 673 / 623. They meet at 4 : 3, where each
+// side wins somewhere; at K = V = 64 too (6 : 5 153 / 146, 4 : 3 103 / 104).
 int grad_heads(long records, int Hk, int Hv, int cus) {
   const long group = Hv / Hk, items = records * Hk;
   const long together = (items + cus - 1) / cus * group, apart = (items * group + cus - 1) / cus;

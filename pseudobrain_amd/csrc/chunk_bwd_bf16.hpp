@@ -21,15 +21,19 @@
 //
 // The decay sums sum_v (K dS' o U)_t and sum_v (K S o dX)_t are formed in the
 // chain, where all four are in float32: as sums over the keys of K o dK1 and K o
-// dK2, whose products take U and dX as bf16 pairs, they left dg with 1.2 to 1.9
-// times its error against 64 bits (and the kernel 1% slower). sum_v (Q S o dO)_t does come from the keys
+// dK2, whose products take U and dX as bf16 pairs, they left dg with 1.2 times
+// its error against 64 bits (geometric mean of 22 calls; up to 1.9), and the
+// kernel 1% slower. sum_v (Q S o dO)_t does come from the keys
 // (sum_k (Q o dQ0)_t): dO is exact in bf16 there.
 // LDS: 134 KiB at K = V = 128, so one workgroup a CU, eight waves.
 //
-// 3.55 (16-column tiles in turn, with the reduction) -> 1.71 ms at 1 x 32,768
-// tokens of 32 heads, 0.51 ms at 4 x 2,048. A head takes about 60,000 cycles:
-// chain 9,000, stages 20,000 (ten barriers), C x C products and sums 15,000, the
-// issue of the next head's loads 5,000 to 14,000; MFMA 12,000, LDS 20,000.
+// 3.55 (16-column tiles in turn, with the reduction) -> 1.57 ms at 1 x 32,768
+// tokens of 32 heads, 0.47 ms at 4 x 2,048 (kernel trace). A head takes about
+// 60,000 cycles (the medians of 32 heads): inputs into LDS 1,700, chain 9,200,
+// stages 19,200 (ten barriers), row scales 1,600, C x C matrices and sums 9,500,
+// last products and the issue of the next head's loads 9,500 (6,200 to 19,400),
+// dg and, after the last head, the output 6,000 (2,000 to 17,700). LDS is
+// active in 36% of the CU's busy cycles, a quarter of it bank conflicts.
 //
 // Contraction slots: the B operand of a 32-row step kb made of two
 // accumulator tiles holds, in lane (c, g), rows 32 kb + 4 g + j (j < 4) and
@@ -37,12 +41,13 @@
 // 8-byte pieces of a row, or two transposing reads).
 
 // LDS arrays are row-major without padding, W elements a row, the 16-byte units
-// of row r swizzled: unit u stands at u ^ unit_swz<W>(r). Both kinds of operand
-// read are then free of bank conflicts: 32 lanes of a transposing read take 32
-// bytes of 8 rows, 32 lanes of a row read 16 bytes of 16 rows, and either way
-// the 16 units differ modulo 256 bytes. (With rows padded by 16 bytes the
-// transposing reads conflicted two ways, with 32 the row reads: 46% of the
-// gradient kernel's LDS cycles.)
+// of row r swizzled: unit u stands at u ^ unit_swz<W>(r). 32 lanes of a
+// transposing read take 32 bytes of 8 rows, 32 lanes of a row read 16 bytes of
+// 16 rows, and either way the 16 units differ modulo 256 bytes. (With rows
+// padded by 16 bytes the transposing reads conflicted two ways, with 32 the row
+// reads.) Conflicts fell from 46% to 25% of the gradient kernel's LDS cycles and
+// from 42% to 32% of the scans' (4 x 2,048 tokens); what is left was not taken
+// apart (row reads that the compiler pairs, and the writes, are not covered).
 template <int W>
 __device__ __forceinline__ constexpr int unit_swz(int r) {
   static_assert(W == 128 || W == 64 || W == 32, "row widths");

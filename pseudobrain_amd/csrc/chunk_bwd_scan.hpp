@@ -20,13 +20,13 @@
 // 64, as a bf16 pair), Q and dO and forms the two products with dO itself:
 // they were records of the local kernel's (dU0 and J, 96 KiB in float32 a
 // chunk and head, written once and read once). At 1 x 32,768 tokens of 32 heads
-// 1.59 (four barriers a step, 16 columns a workgroup) -> 1.37 ms, the chain of a
-// step and its traffic 1.1 ms each by themselves; at 4 x 2,048 437 -> 235 us.
+// 1.59 (four barriers a step, 16 columns a workgroup) -> 1.34 ms, the chain of a
+// step and its traffic 1.1 ms each by themselves; at 4 x 2,048 437 -> 233 us.
 
 // ---------------------------------------------------------------------------
 // Per (chunk, value head): T = (I + A)^-1 and M^T as bf16 pairs, c, beta.
 // Wave w holds token rows 16 w .. of q as operands (no LDS), so four
-// workgroups share a CU. 0.70 (with dU0 and J) -> 0.26 ms at 1 x 32,768 tokens
+// workgroups share a CU. 0.70 (with dU0 and J) -> 0.25 ms at 1 x 32,768 tokens
 // of 32 heads, 0.6 GB written; the inverse's serial rows are what it waits for.
 // ---------------------------------------------------------------------------
 template <int K>

@@ -31,8 +31,9 @@
 // O is formed transposed (O^T = (Q S)^T diag(scale gamma) + U^T QKD^T: the
 // same registers with the MFMA operands swapped), so a lane holds 4
 // contiguous columns of a token row and stores them as one piece of 8 bytes
-// (16 for float32, whose o costs no more than a 16-bit one: the step is not
-// bound by its stores).
+// (16 for float32, whose calls take 8% to 12% longer than those of a 16-bit o,
+// less than widening it afterwards: 4 x 2,048 tokens of 32 heads 160 us against
+// 143 and, widened, 184).
 //
 // Staging. A chunk's K and Q rows (16-bit, 256 bytes at K = 128), its record
 // and its V rows (128 columns) are copied HBM -> LDS by direct-to-LDS buffer

@@ -30,9 +30,10 @@ for 256-wide keys with 16-bit inputs, and token by token through the
 recurrent kernel with float32 inputs.
 
 Gradients. gated_delta_rule's device paths are differentiable through the chunk
-operator's backward (pbgdn::gated_delta_chunk_f32, for K, V <= 128, batches
-and packed sequences alike); a training call through "sequential" (T <=
-SEQUENTIAL_MAX) takes the same operator. The lower-level entry points (chunk_fwd, chunk_fwd_slots,
+operator's backward (pbgdn::gated_delta_chunk_f32, or gated_delta_chunk where V
+is padded; K, V <= 128, batches and packed sequences alike); a training call
+through "sequential" (T <= SEQUENTIAL_MAX) takes the same operator. The
+lower-level entry points (chunk_fwd, chunk_fwd_slots,
 recurrent_fwd, the decode and slot ops, the layer kernels in
 pseudobrain_amd.layer) have no backward: with grad mode on and an input that
 requires grad they raise instead of returning tensors cut from the graph.
@@ -554,7 +555,7 @@ def _packed_backward(q, k, v, g, beta, h0, cu_seqlens, grad_o, grad_final, scale
         x[:, hi:].zero_()
     for a, b in _packed_groups(bounds, size, limit):
         rows = slice(bounds[a], bounds[b])
-        _chunk_bwd(q[:, rows], k[:, rows], v[:, rows], g[:, rows], beta[:, rows], scale, None if h0 is None else h0[a:b],
+        _chunk_bwd(*(x[:, rows] for x in (q, k, v, g, beta)), scale, None if h0 is None else h0[a:b],
                    cu_seqlens[a:b + 1] - bounds[a], grad_o[:, rows], None if grad_final is None else grad_final[a:b],
                    out=[x[:, rows] for x in out[:5]] + [out[5][a:b]])
     return tuple(out)

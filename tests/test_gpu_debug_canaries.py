@@ -20,9 +20,9 @@ import torch
 from pseudobrain_amd import _lib
 from pseudobrain_amd import gated_deltanet as gd
 from pseudobrain_amd.workloads import generate
-from tests import (test_gpu_backward, test_gpu_backward_bf16, test_gpu_backward_packed, test_gpu_chunk, test_gpu_chunk_k256, test_gpu_chunk_layer, test_gpu_decode_layer,
-                   test_gpu_fla_schema, test_gpu_layer, test_gpu_prologue_varlen, test_gpu_recurrent,
-                   test_gpu_state_pools, test_gpu_wide)
+from tests import (test_gpu_backward, test_gpu_backward_bf16, test_gpu_backward_packed, test_gpu_chunk,
+                   test_gpu_chunk_k256, test_gpu_chunk_layer, test_gpu_decode_layer, test_gpu_fla_schema, test_gpu_layer,
+                   test_gpu_prologue_varlen, test_gpu_recurrent, test_gpu_state_pools, test_gpu_wide)
 
 pytestmark = pytest.mark.gpu
 
