@@ -25,7 +25,7 @@
 // its error against 64 bits (geometric mean of 22 calls; up to 1.9), and the
 // kernel 1% slower. sum_v (Q S o dO)_t does come from the keys
 // (sum_k (Q o dQ0)_t): dO is exact in bf16 there.
-// LDS: 134 KiB at K = V = 128, so one workgroup a CU, eight waves.
+// LDS: 135 KiB at K = V = 128, so one workgroup a CU, eight waves.
 //
 // 3.55 (16-column tiles in turn, with the reduction) -> 1.57 ms at 1 x 32,768
 // tokens of 32 heads, 0.47 ms at 4 x 2,048 (kernel trace). A head takes about
